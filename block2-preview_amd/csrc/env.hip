@@ -1065,8 +1065,10 @@ extern "C" int b2g_contract_wfn_plan(b2g_ctx ctx, int symmetry,
     std::unique_ptr<b2g_gemmlist_s> g(new b2g_gemmlist_s());
     g->ctx = ctx;
     g->d_len = O.total();
-    tile_env_refresh();
+    std::vector<Seg> prods; // one product per output block, K = 0: none
     for (int i = 0; i < O.n(); i++) {
+        Seg sg{};
+        prods.push_back(sg);
         int il, ir;
         if (l_is_wfn) { // wfn = wfn x rot
             il = L.find_state(O.quanta[i]);
@@ -1082,8 +1084,6 @@ extern "C" int b2g_contract_wfn_plan(b2g_ctx ctx, int symmetry,
                     B2G_ERR_ARG, "contraction block shapes differ");
         if (K == 0 || M == 0 || N == 0)
             continue;
-        const uint32_t sb = (uint32_t)g->segs.size();
-        Seg sg{};
         sg.a_off = L.shift[il];
         sg.b_off = R.shift[ir];
         sg.lda = L.nket[il];
@@ -1091,10 +1091,18 @@ extern "C" int b2g_contract_wfn_plan(b2g_ctx ctx, int symmetry,
         sg.K = K;
         sg.flags = 0;
         sg.alpha = scale;
-        g->segs.push_back(sg);
-        add_tiles(g->tasks, O.shift[i], M, N, K, sb, sb + 1, 0);
+        prods.back() = sg;
         g->macs += (uint64_t)M * N * K;
         g->n_products++;
+    }
+    tile_env_refresh(g->macs, 0, ctx->num_cu);
+    for (int i = 0; i < O.n(); i++) {
+        if (prods[i].K == 0)
+            continue;
+        const uint32_t sb = (uint32_t)g->segs.size();
+        g->segs.push_back(prods[i]);
+        add_tiles(g->tasks, O.shift[i], O.nbra[i], O.nket[i], prods[i].K, sb,
+                  sb + 1, 0);
     }
     size_t bytes = g->segs.size() * sizeof(Seg);
     for (int c = 0; c < kTileConfigs; c++)

@@ -123,7 +123,7 @@ static bool launch_in_bounds(const Launch &L, uint64_t a_len, uint64_t b_len,
 }
 
 static int grad_plan_build(b2g_plan p, GradPlan **out) {
-    tile_env_refresh();
+    tile_env_refresh(p->macs, 0, p->ctx->num_cu);
     GradPlan *g = new GradPlan();
     const b2g_pair *pairs = p->pairs.data();
     const size_t n = p->pairs.size();
@@ -221,7 +221,7 @@ static int grad_plan_build(b2g_plan p, GradPlan **out) {
         for (Launch *L : {&ch.w, &ch.z, &ch.l0, &ch.l1, &ch.r0, &ch.r1})
             for (int c = 0; c < kTileConfigs; c++) {
                 sort_tasks(L->t[c], L->s);
-                g->flops += task_flops(L->t[c], L->s, c);
+                g->flops += task_flops(L->t[c], L->s);
             }
         const uint64_t llen = p->lbuf->n, rlen = p->rbuf->n;
         const uint64_t xl = p->x_len, yl = p->y_len;

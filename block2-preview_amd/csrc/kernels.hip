@@ -65,14 +65,18 @@ __device__ __forceinline__ float buf_load_s<float>(__amdgpu_buffer_rsrc_t r,
 // TM x TN, each wave owns (TM/2) x (TN/2) as (TM/32) x (TN/32) MFMA tiles.
 // K is staged through two LDS buffers in chunks of TK: while the MFMAs run on
 // one buffer, the next chunk's global loads are in flight in registers and
-// are then written to the other buffer, so one barrier per chunk suffices.
+// are then written to the other buffer, so one barrier per chunk suffices
+// (a second chunk in flight gained nothing on tiles of up to 64 x 64, whose
+// four workgroups per compute unit cover the latency: n=26 M=1000 product
+// 407 us against 397 us).
 // Element q of thread tid is e = tid + 256 q; since 256 is a multiple of TK,
 // TM and TN, one coordinate of e is the same for all q and the other
 // advances by a constant.  Tasks are strided over the grid (persistent
 // launch); blockIdx.y selects the right-hand side.
 //
-// The registers of one chunk and their store to LDS ([k][m] and [k][n]
-// layouts, one padding column), the per-segment alpha applied there.
+// The registers of one chunk, with the flags and alpha of its segment, and
+// their store to LDS ([k][m] and [k][n] layouts, one padding column), alpha
+// applied there.
 template <typename TA, typename TB, typename TC, int TM, int TN, int TK>
 struct TileRegs {
     static constexpr int NA = TM * TK / 256, NB = TN * TK / 256;
@@ -80,22 +84,23 @@ struct TileRegs {
                   "tile shape");
     TA ra[NA];
     TB rb[NB];
+    uint32_t flags;
+    double alpha;
     // registers -> LDS buffer ([k][m] and [k][n] layouts), alpha applied;
     // per layout, element q sits at a per-thread base plus a constant
-    __device__ __forceinline__ void store(TC *As, TC *Bs, const Seg &sg,
-                                          int tid) {
-        const bool ta = sg.flags & 1, tb = (sg.flags >> 1) & 1;
-        const TC alpha = (TC)sg.alpha;
+    __device__ __forceinline__ void store(TC *As, TC *Bs, int tid) const {
+        const bool ta = flags & 1, tb = (flags >> 1) & 1;
+        const TC al = (TC)alpha;
         if (!ta) { // m = tid / TK + q * 256 / TK, k = tid % TK
             TC *p = As + (tid % TK) * (TM + 1) + tid / TK;
 #pragma unroll
             for (int q = 0; q < NA; q++)
-                p[q * (256 / TK)] = (TC)ra[q] * alpha;
+                p[q * (256 / TK)] = (TC)ra[q] * al;
         } else { // m = tid % TM, k = tid / TM + q * 256 / TM
             TC *p = As + (tid / TM) * (TM + 1) + tid % TM;
 #pragma unroll
             for (int q = 0; q < NA; q++)
-                p[q * (256 / TM) * (TM + 1)] = (TC)ra[q] * alpha;
+                p[q * (256 / TM) * (TM + 1)] = (TC)ra[q] * al;
         }
         if (!tb) { // n = tid % TN, k = tid / TN + q * 256 / TN
             TC *p = Bs + (tid / TN) * (TN + 1) + tid % TN;
@@ -111,27 +116,42 @@ struct TileRegs {
     }
 };
 
-// Buffer loads at 32-bit byte offsets from the segment's blocks, with
-// segment-invariant offsets: at the first chunk of a segment every
-// element's byte offset at k0 = 0 is computed once (rows or columns outside
-// the block get an offset past the buffer's record count and read as zero);
-// each chunk then passes its k0 as the instruction's scalar offset, so a
-// full chunk costs no vector arithmetic before its loads.  Elements at
-// k >= K (the last, partial chunk of a segment) get the masked offset per
-// element.  Measured on the n=40 M=3000 middle site against 64-bit
-// addresses recomputed per chunk: FP64 H*psi 54.3 -> 48.0 ms per 4-RHS step,
-// its 128 x 128 phase-2 launch 17.5 -> 14.9 ms.
+// Walks the chunks of a task's segments and loads them.  Buffer loads at
+// 32-bit byte offsets from the segment's blocks, with segment-invariant
+// offsets: at the first chunk of a segment every element's byte offset at
+// k0 = 0 is computed once (rows or columns outside the block get an offset
+// past the buffer's record count and read as zero); each chunk then passes
+// its k0 as the instruction's scalar offset, so a full chunk costs no vector
+// arithmetic before its loads.  Elements at k >= K (the last, partial chunk
+// of a segment) get the masked offset per element.  Segments have K > 0 (the
+// plan drops empty ones); their descriptors are wave-uniform and read one
+// segment ahead.
 template <typename TA, typename TB, typename TC, int TM, int TN, int TK>
-struct TileLoaderS : TileRegs<TA, TB, TC, TM, TN, TK> {
-    using Base = TileRegs<TA, TB, TC, TM, TN, TK>;
-    static constexpr int NA = Base::NA, NB = Base::NB;
+struct TileLoader {
+    typedef TileRegs<TA, TB, TC, TM, TN, TK> Regs;
+    static constexpr int NA = Regs::NA, NB = Regs::NB;
     uint32_t va[NA], vb[NB]; // byte offsets at k0 = 0 (kMasked: outside)
     uint32_t sa, sb;         // bytes per unit of k0
     __amdgpu_buffer_rsrc_t rA, rB;
-    __device__ __forceinline__ void setup(const TA *__restrict__ A,
-                                          const TB *__restrict__ B,
-                                          const Seg &sg, const Task &task,
-                                          int tid) {
+    const TA *A;
+    const TB *B;
+    const Seg *segs;
+    Seg cur, nxt;
+    uint32_t s, end, k0;
+    __device__ __forceinline__ TileLoader(const TA *A_, const TB *B_,
+                                          const Seg *segs_, const Task &task)
+        : A(A_), B(B_), segs(segs_), s(task.seg_begin), end(task.seg_end),
+          k0(0) {
+        if (s < end) {
+            cur = segs[s];
+            nxt = cur;
+            if (s + 1 < end)
+                nxt = segs[s + 1];
+        }
+    }
+    __device__ __forceinline__ bool more() const { return s < end; }
+    __device__ __forceinline__ void setup(const Task &task, int tid) {
+        const Seg &sg = cur;
         const bool ta = sg.flags & 1, tb = (sg.flags >> 1) & 1;
         rA = buf_rsrc(A + sg.a_off);
         rB = buf_rsrc(B + sg.b_off);
@@ -180,40 +200,162 @@ struct TileLoaderS : TileRegs<TA, TB, TC, TM, TN, TK> {
         sa = __builtin_amdgcn_readfirstlane(sa);
         sb = __builtin_amdgcn_readfirstlane(sb);
     }
-    __device__ __forceinline__ void load(const TA *__restrict__ A,
-                                         const TB *__restrict__ B,
-                                         const Seg &sg, uint32_t k0,
-                                         const Task &task, int tid) {
+    // starts the loads of the current chunk into r and steps to the next
+    __device__ __forceinline__ void load(Regs &r, const Task &task, int tid) {
         if (k0 == 0)
-            setup(A, B, sg, task, tid);
+            setup(task, tid);
+        const Seg &sg = cur;
+        r.flags = sg.flags;
+        r.alpha = sg.alpha;
         const uint32_t soa = __builtin_amdgcn_readfirstlane(k0 * sa);
         const uint32_t sob = __builtin_amdgcn_readfirstlane(k0 * sb);
         if (k0 + TK <= sg.K) {
 #pragma unroll
             for (int q = 0; q < NA; q++)
-                this->ra[q] = buf_load_s<TA>(rA, va[q], soa);
+                r.ra[q] = buf_load_s<TA>(rA, va[q], soa);
 #pragma unroll
             for (int q = 0; q < NB; q++)
-                this->rb[q] = buf_load_s<TB>(rB, vb[q], sob);
-            return;
-        }
-        // partial chunk: the k of element q, per storage order
-        const bool ta = sg.flags & 1, tb = (sg.flags >> 1) & 1;
+                r.rb[q] = buf_load_s<TB>(rB, vb[q], sob);
+        } else {
+            // partial chunk: the k of element q, per storage order
+            const bool ta = sg.flags & 1, tb = (sg.flags >> 1) & 1;
 #pragma unroll
-        for (int q = 0; q < NA; q++) {
-            const uint32_t k =
-                k0 + (ta ? tid / TM + q * (256 / TM) : tid % TK);
-            this->ra[q] = buf_load_s<TA>(rA, k < sg.K ? va[q] : kMasked, soa);
-        }
+            for (int q = 0; q < NA; q++) {
+                const uint32_t k =
+                    k0 + (ta ? tid / TM + q * (256 / TM) : tid % TK);
+                r.ra[q] = buf_load_s<TA>(rA, k < sg.K ? va[q] : kMasked, soa);
+            }
 #pragma unroll
-        for (int q = 0; q < NB; q++) {
-            const uint32_t k =
-                k0 + (tb ? tid % TK : tid / TN + q * (256 / TN));
-            this->rb[q] = buf_load_s<TB>(rB, k < sg.K ? vb[q] : kMasked, sob);
+            for (int q = 0; q < NB; q++) {
+                const uint32_t k =
+                    k0 + (tb ? tid % TK : tid / TN + q * (256 / TN));
+                r.rb[q] = buf_load_s<TB>(rB, k < sg.K ? vb[q] : kMasked, sob);
+            }
+        }
+        k0 += TK;
+        if (k0 >= sg.K) {
+            k0 = 0;
+            s++;
+            cur = nxt;
+            if (s + 1 < end)
+                nxt = segs[s + 1];
         }
     }
 };
 
+// One task: the K loop, then the epilogue.  smem: 2 * TK * (TM + TN + 2)
+// elements.
+template <typename TA, typename TB, typename TD, typename TC, int TM, int TN,
+          int TK>
+__device__ __forceinline__ void seg_gemm_task(
+    const TA *__restrict__ A, const TB *__restrict__ B, TD *__restrict__ D,
+    TD *__restrict__ P, const Task &task, const Seg *__restrict__ segs,
+    double scale, int beta0, TC *smem) {
+    constexpr int WM = TM / 2, WN = TN / 2;
+    constexpr int FM = WM / 16, FN = WN / 16;
+    constexpr int ASZ = TK * (TM + 1), BSZ = TK * (TN + 1);
+    typedef typename Mfma<TC>::acc_t acc_t;
+    typedef TileLoader<TA, TB, TC, TM, TN, TK> Loader;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int lr = lane & 15, lk = lane >> 4;
+    acc_t acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+            acc[i][j] = acc_t{0, 0, 0, 0};
+    // MFMAs on one LDS buffer, fragment reads one k-step ahead
+    auto mac = [&](const TC *As) {
+        const TC *Bs = As + ASZ;
+        TC a[2][FM], b[2][FN];
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+            a[0][i] = As[lk * (TM + 1) + wm * WM + i * 16 + lr];
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+            b[0][j] = Bs[lk * (TN + 1) + wn * WN + j * 16 + lr];
+#pragma unroll
+        for (int ks = 0; ks < TK / 4; ks++) {
+            const int cb = ks & 1, nb = cb ^ 1;
+            if (ks + 1 < TK / 4) {
+                const int kr = (ks + 1) * 4 + lk;
+#pragma unroll
+                for (int i = 0; i < FM; i++)
+                    a[nb][i] = As[kr * (TM + 1) + wm * WM + i * 16 + lr];
+#pragma unroll
+                for (int j = 0; j < FN; j++)
+                    b[nb][j] = Bs[kr * (TN + 1) + wn * WN + j * 16 + lr];
+            }
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++)
+                    acc[i][j] = Mfma<TC>::op(a[cb][i], b[cb][j], acc[i][j]);
+        }
+    };
+    Loader ld(A, B, segs, task);
+    if (ld.more()) {
+        TC *use = smem, *fill = smem + ASZ + BSZ;
+        typename Loader::Regs r;
+        ld.load(r, task, tid);
+        r.store(use, use + ASZ, tid);
+        __syncthreads();
+        while (true) {
+            const bool more = ld.more();
+            if (more)
+                ld.load(r, task, tid);
+            mac(use);
+            if (!more)
+                break;
+            // `fill` was released by the barrier that ended the previous
+            // chunk
+            r.store(fill, fill + ASZ, tid);
+            TC *t = use;
+            use = fill, fill = t;
+            __syncthreads();
+        }
+        __syncthreads(); // all waves done with LDS before the next task
+    }
+    mfma_settle<acc_t, FM * FN>(&acc[0][0]);
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const uint32_t row =
+                    task.row0 + wm * WM + i * 16 + Mfma<TC>::row(lk, r);
+                const uint32_t col = task.col0 + wn * WN + j * 16 + lr;
+                if (row < task.M && col < task.N) {
+                    const uint64_t idx =
+                        task.d_off + (uint64_t)row * task.ldd + col;
+                    const double v = scale * (double)acc[i][j][r];
+                    if (task.beta & 2)
+                        P[idx] = (TD)v; // partial tile, reduced later
+                    else if ((task.beta | beta0) & 1)
+                        D[idx] = (TD)((double)D[idx] + v);
+                    else
+                        D[idx] = (TD)v;
+                }
+            }
+}
+
+// Tasks of one launch: first index, end and stride of this workgroup
+struct TaskRange {
+    int t0, tend, tstep;
+    __device__ __forceinline__ TaskRange(int ntasks, const XcdSplit &xs)
+        : t0(blockIdx.x), tend(ntasks), tstep(gridDim.x) {
+        if (xs.off[8] != 0) {
+            const int x = blockIdx.x & 7;
+            t0 = (int)xs.off[x] + (int)(blockIdx.x >> 3);
+            tend = (int)xs.off[x + 1];
+            tstep = gridDim.x >> 3;
+        }
+    }
+};
+
+// tiles with a side of 128: one launch per shape
 template <typename TA, typename TB, typename TD, typename TC, int TM, int TN,
           int TK, int PHASE>
 __global__ __launch_bounds__(256) void seg_gemm_kernel(
@@ -221,146 +363,76 @@ __global__ __launch_bounds__(256) void seg_gemm_kernel(
     TD *__restrict__ P, const Task *__restrict__ tasks, int ntasks,
     const Seg *__restrict__ segs, uint64_t a_rs, uint64_t b_rs, uint64_t d_rs,
     uint64_t p_rs, double scale, int beta0, XcdSplit xs) {
-    constexpr int WM = TM / 2, WN = TN / 2;
-    constexpr int FM = WM / 16, FN = WN / 16;
-    constexpr int ASZ = TK * (TM + 1), BSZ = TK * (TN + 1);
-    typedef typename Mfma<TC>::acc_t acc_t;
-    __shared__ TC smem[2 * (ASZ + BSZ)];
+    __shared__ TC smem[2 * TK * (TM + TN + 2)];
+    const int rhs = blockIdx.y;
+    const TaskRange tr(ntasks, xs);
+    for (int t = tr.t0; t < tr.tend; t += tr.tstep) {
+        const Task task = tasks[t];
+        seg_gemm_task<TA, TB, TD, TC, TM, TN, TK>(
+            A + rhs * a_rs, B + rhs * b_rs, D + rhs * d_rs, P + rhs * p_rs,
+            task, segs, scale, beta0, smem);
+    }
+}
+
+// Tiles of 32 and 64 in one launch, the shape taken from each task
+// (task_cfg): one launch per phase keeps four workgroups (33 KB of LDS each)
+// on every compute unit until the phase's last tasks, where a launch per
+// shape drained the chip at the end of each.  Four rather than nine shapes
+// cover a block of up to 64 x 64, so nothing is rounded up past 32.  Bound
+// by the FP64 matrix cores and what keeps them waiting: at the n=26 M=1000
+// middle site they are busy 63 % of the time a compute unit has work, and
+// its blocks of 1..300 rows leave a quarter of the MFMA work in padding.
+// Product at that site, one right-hand side: 1279 -> 391 us (FP64), three at
+// n=16 M=500: 1930 -> 412 us, FP32, two: 1588 -> 401 us, n=8 M=50: 127 -> 47
+// us (with the split along K of tile_env_refresh); one launch per shape for
+// the same tiles: 444, 498 and 460 us for the first three.
+template <typename TA, typename TB, typename TD, typename TC, int PHASE>
+__global__ __launch_bounds__(256, 4) void seg_gemm_small_kernel(
+    const TA *__restrict__ A, const TB *__restrict__ B, TD *__restrict__ D,
+    TD *__restrict__ P, const Task *__restrict__ tasks, int ntasks,
+    const Seg *__restrict__ segs, uint64_t a_rs, uint64_t b_rs, uint64_t d_rs,
+    uint64_t p_rs, double scale, int beta0, XcdSplit xs) {
+    __shared__ TC smem[2 * 32 * (32 + 32 + 2)]; // >= 2 * 16 * (64 + 64 + 2)
     const int rhs = blockIdx.y;
     A += rhs * a_rs;
     B += rhs * b_rs;
     D += rhs * d_rs;
     P += rhs * p_rs;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lr = lane & 15, lk = lane >> 4;
-    TileLoaderS<TA, TB, TC, TM, TN, TK> ld;
-    int t0 = blockIdx.x, tend = ntasks, tstep = gridDim.x;
-    if (xs.off[8] != 0) {
-        const int x = blockIdx.x & 7;
-        t0 = (int)xs.off[x] + (int)(blockIdx.x >> 3);
-        tend = (int)xs.off[x + 1];
-        tstep = gridDim.x >> 3;
-    }
-    for (int t = t0; t < tend; t += tstep) {
+    const TaskRange tr(ntasks, xs);
+    for (int t = tr.t0; t < tr.tend; t += tr.tstep) {
         const Task task = tasks[t];
-        acc_t acc[FM][FN];
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-            for (int j = 0; j < FN; j++)
-                acc[i][j] = acc_t{0, 0, 0, 0};
-        // segments have K > 0 (the plan drops empty ones); descriptors are
-        // wave-uniform and read one segment ahead
-        uint32_t s = task.seg_begin, k0 = 0;
-        if (s < task.seg_end) {
-            Seg cur = segs[s];
-            Seg nxt = cur;
-            if (s + 1 < task.seg_end)
-                nxt = segs[s + 1];
-            int buf = 0;
-            ld.load(A, B, cur, k0, task, tid);
-            ld.store(smem, smem + ASZ, cur, tid);
-            __syncthreads();
-            while (true) {
-                // advance the loader to the next chunk and start its loads
-                k0 += TK;
-                if (k0 >= cur.K) {
-                    k0 = 0;
-                    s++;
-                    cur = nxt;
-                    if (s + 1 < task.seg_end)
-                        nxt = segs[s + 1];
-                }
-                const bool more = s < task.seg_end;
-                if (more)
-                    ld.load(A, B, cur, k0, task, tid);
-                const TC *As = smem + buf * (ASZ + BSZ);
-                const TC *Bs = As + ASZ;
-                // MFMAs on this buffer, fragment reads one k-step ahead
-                TC a[2][FM], b[2][FN];
-#pragma unroll
-                for (int i = 0; i < FM; i++)
-                    a[0][i] = As[lk * (TM + 1) + wm * WM + i * 16 + lr];
-#pragma unroll
-                for (int j = 0; j < FN; j++)
-                    b[0][j] = Bs[lk * (TN + 1) + wn * WN + j * 16 + lr];
-#pragma unroll
-                for (int ks = 0; ks < TK / 4; ks++) {
-                    const int cb = ks & 1, nb = cb ^ 1;
-                    if (ks + 1 < TK / 4) {
-                        const int kr = (ks + 1) * 4 + lk;
-#pragma unroll
-                        for (int i = 0; i < FM; i++)
-                            a[nb][i] = As[kr * (TM + 1) + wm * WM + i * 16 + lr];
-#pragma unroll
-                        for (int j = 0; j < FN; j++)
-                            b[nb][j] = Bs[kr * (TN + 1) + wn * WN + j * 16 + lr];
-                    }
-#pragma unroll
-                    for (int i = 0; i < FM; i++)
-#pragma unroll
-                        for (int j = 0; j < FN; j++)
-                            acc[i][j] = Mfma<TC>::op(a[cb][i], b[cb][j],
-                                                     acc[i][j]);
-                }
-                if (!more)
-                    break;
-                // the other buffer was released by the barrier that ended
-                // the previous chunk
-                buf ^= 1;
-                TC *Ns = smem + buf * (ASZ + BSZ);
-                ld.store(Ns, Ns + ASZ, cur, tid);
-                __syncthreads();
-            }
-            __syncthreads(); // all waves done with LDS before the next task
+#define B2G_TASK(TM_, TN_, TK_)                                                \
+    seg_gemm_task<TA, TB, TD, TC, TM_, TN_, TK_>(A, B, D, P, task, segs,       \
+                                                 scale, beta0, smem)
+        switch (__builtin_amdgcn_readfirstlane(task_cfg(task))) {
+        case 0: B2G_TASK(32, 32, 32); break;
+        case 1: B2G_TASK(32, 64, 16); break;
+        case 3: B2G_TASK(64, 32, 16); break;
+        default: B2G_TASK(64, 64, 16); break;
         }
-        mfma_settle<acc_t, FM * FN>(&acc[0][0]);
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-            for (int j = 0; j < FN; j++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const uint32_t row =
-                        task.row0 + wm * WM + i * 16 + Mfma<TC>::row(lk, r);
-                    const uint32_t col = task.col0 + wn * WN + j * 16 + lr;
-                    if (row < task.M && col < task.N) {
-                        const uint64_t idx =
-                            task.d_off + (uint64_t)row * task.ldd + col;
-                        const double v = scale * (double)acc[i][j][r];
-                        if (task.beta & 2)
-                            P[idx] = (TD)v; // partial tile, reduced later
-                        else if ((task.beta | beta0) & 1)
-                            D[idx] = (TD)((double)D[idx] + v);
-                        else
-                            D[idx] = (TD)v;
-                    }
-                }
+#undef B2G_TASK
     }
 }
 
-// One workgroup reduces a 1024-element slice of one tile (tiles hold at most
-// 128 x 128 = 16 slices): thread i takes elements 4i..4i+3 of the slice,
+// One workgroup reduces a 1024-element slice of one tile (`slices` of them,
+// those of the launch's largest tile): thread i takes elements 4i..4i+3 of the slice,
 // reading each part's four values as two 16-byte loads (partial slots are
 // 1024-element aligned and tile widths multiples of 32, so the four share a
 // row).  Parts are summed in increasing order: the result does not depend on
 // the launch shape.
-constexpr int kRedSlices = 16;
-
 template <typename TD>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(
     TD *__restrict__ D, const TD *__restrict__ P,
-    const RedTask *__restrict__ tasks, int ntasks, uint64_t d_rs,
+    const RedTask *__restrict__ tasks, int ntasks, int slices, uint64_t d_rs,
     uint64_t p_rs, int beta0) {
     const int rhs = blockIdx.y;
     D += rhs * d_rs;
     P += rhs * p_rs;
-    const int64_t nwork = (int64_t)ntasks * kRedSlices;
+    const int64_t nwork = (int64_t)ntasks * slices;
     for (int64_t w = blockIdx.x; w < nwork; w += gridDim.x) {
-        const RedTask rt = tasks[w / kRedSlices];
+        const RedTask rt = tasks[w / slices];
         const uint32_t tsz = rt.tm * rt.tn;
-        const uint32_t e = (uint32_t)(w % kRedSlices) * 1024 + 4 * threadIdx.x;
+        const uint32_t e = (uint32_t)(w % slices) * 1024 + 4 * threadIdx.x;
         if (e >= tsz)
             continue;
         const uint32_t r = e / rt.tn, c = e % rt.tn;
@@ -389,29 +461,25 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(
 
 template <typename TD>
 hipError_t launch_splitk_reduce(TD *D, const TD *P, const RedTask *tasks,
-                                int ntasks, uint64_t d_rs, uint64_t p_rs,
-                                int beta0, int n_rhs, int grid,
+                                int ntasks, int slices, uint64_t d_rs,
+                                uint64_t p_rs, int beta0, int n_rhs, int grid,
                                 hipStream_t st) {
     if (ntasks <= 0)
         return hipSuccess;
-    const int64_t nwork = (int64_t)ntasks * kRedSlices;
+    const int64_t nwork = (int64_t)ntasks * slices;
     const int64_t cap = (int64_t)grid * 4;
     dim3 g((unsigned)(nwork < cap ? nwork : cap), (unsigned)n_rhs);
     hipLaunchKernelGGL(splitk_reduce_kernel<TD>, g, dim3(256), 0, st, D, P,
-                       tasks, ntasks, d_rs, p_rs, beta0);
+                       tasks, ntasks, slices, d_rs, p_rs, beta0);
     return hipGetLastError();
 }
 template hipError_t launch_splitk_reduce<double>(double *, const double *,
-                                                 const RedTask *, int,
+                                                 const RedTask *, int, int,
                                                  uint64_t, uint64_t, int, int,
                                                  int, hipStream_t);
-template hipError_t launch_splitk_reduce<float>(float *, const float *,
-                                                const RedTask *, int, uint64_t,
-                                                uint64_t, int, int, int,
-                                                hipStream_t);
 
-// tile configurations (index = Task bucket id): cfg = 3 * i + j with
-// TM = 32 << i and TN = 32 << j; K chunk 16 (32 for the 32x32 tile)
+// tile configurations: cfg = 3 * i + j with TM = 32 << i and TN = 32 << j;
+// K chunk 16 (32 for the 32x32 tile)
 int tile_m(int cfg) { return 32 << (cfg / 3); }
 int tile_n(int cfg) { return 32 << (cfg % 3); }
 
@@ -436,15 +504,16 @@ hipError_t launch_seg_gemm(int cfg, const TA *A, const TB *B, TD *D, TD *P,
                        dim3(256), 0, st, A, B, D, P, tasks, ntasks, segs,      \
                        a_rs, b_rs, d_rs, p_rs, scale, beta0, xs)
     switch (cfg) {
-    case 0: B2G_LAUNCH(32, 32, 32); break;
-    case 1: B2G_LAUNCH(32, 64, 16); break;
     case 2: B2G_LAUNCH(32, 128, 16); break;
-    case 3: B2G_LAUNCH(64, 32, 16); break;
-    case 4: B2G_LAUNCH(64, 64, 16); break;
     case 5: B2G_LAUNCH(64, 128, 16); break;
     case 6: B2G_LAUNCH(128, 32, 16); break;
     case 7: B2G_LAUNCH(128, 64, 16); break;
-    default: B2G_LAUNCH(128, 128, 16); break;
+    case 8: B2G_LAUNCH(128, 128, 16); break;
+    default:
+        hipLaunchKernelGGL((seg_gemm_small_kernel<TA, TB, TD, TC, PHASE>), g,
+                           dim3(256), 0, st, A, B, D, P, tasks, ntasks, segs,
+                           a_rs, b_rs, d_rs, p_rs, scale, beta0, xs);
+        break;
     }
 #undef B2G_LAUNCH
     return hipGetLastError();

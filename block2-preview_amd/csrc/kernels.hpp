@@ -71,9 +71,13 @@ struct Task {
     uint32_t row0, col0;
     uint32_t seg_begin, seg_end;
     // bit 0: accumulate into D; bit 1: partial tile (split K) written to the
-    // partial buffer P with d_off / ldd addressing the tile's dense slot
+    // partial buffer P with d_off / ldd addressing the tile's dense slot;
+    // bits 4..7: tile configuration (launch.hpp)
     uint32_t beta;
 };
+__host__ __device__ inline int task_cfg(const Task &t) {
+    return (int)((t.beta >> 4) & 15u);
+}
 
 // Per-XCD task ranges of one launch: when off[8] != 0, workgroup b (dealt
 // to XCD b % 8 by the dispatcher) walks tasks [off[b % 8], off[b % 8 + 1])

@@ -11,6 +11,10 @@ namespace b2g {
 int tile_m(int cfg);
 int tile_n(int cfg);
 constexpr int kTileConfigs = 9;
+// launch of the FP64 / FP32 tiles of up to 64 x 64, shapes mixed
+constexpr int kSmallCfg = 4;
+// tile area in units of 32 x 32
+inline int tile_area(int cfg) { return (1 << (cfg / 3)) << (cfg % 3); }
 
 // persistent grid size of a grouped-GEMM launch (a multiple of 8 when the
 // launch has per-XCD task ranges)
@@ -27,8 +31,8 @@ hipError_t launch_seg_gemm(int cfg, const TA *A, const TB *B, TD *D, TD *P,
                            int grid, hipStream_t st, XcdSplit xs = XcdSplit{});
 template <typename TD>
 hipError_t launch_splitk_reduce(TD *D, const TD *P, const RedTask *tasks,
-                                int ntasks, uint64_t d_rs, uint64_t p_rs,
-                                int beta0, int n_rhs, int grid,
+                                int ntasks, int slices, uint64_t d_rs,
+                                uint64_t p_rs, int beta0, int n_rhs, int grid,
                                 hipStream_t st);
 
 // split-BF16 three-term variant on packed operand planes (gemm_bf16x3.hip):

@@ -132,7 +132,6 @@ static int pk_pack_ops(b2g_plan p, PkPlan *k) {
 
 static int pk_build_into(b2g_plan p, PkPlan *k) {
     SetupTimer tm("packed plan");
-    tile_env_refresh();
     const bool group_b = pk_group_b();
     Packer L, R, X;
     L.src_len = p->lbuf->n;
@@ -247,7 +246,7 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
         // one W^T block per phase-1 segment, tiled with the split-BF16
         // rates (segment K from the plan's own segments)
         jobs.emplace_back([&]() {
-            tile_env_refresh();
+            tile_env_refresh(~0ull, ~0ull, p->ctx->num_cu);
             for (size_t si = 0; si < ch.s1.size(); si++)
                 for (const Tile &t :
                      tile_cover(m1[si], n1[si], ch.s1[si].K, 1))
@@ -258,7 +257,7 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
         // output blocks re-tiled likewise, with split-K partial slots and
         // reductions of their own
         jobs.emplace_back([&]() {
-            tile_env_refresh();
+            tile_env_refresh(~0ull, ~0ull, p->ctx->num_cu);
             for (const BlockJob &j : ch.jobs2)
                 add_split_tiles(ch.s2, j, 1, h.t2, h.red, h.p_len);
         });
@@ -388,11 +387,12 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
             pc.x2[c] = h.x2[c];
             pc.n1[c] = h.t1[c].size();
             pc.n2[c] = h.t2[c].size();
-            pc.f1[c] = task_flops(h.t1[c], h.s1, c);
-            pc.f2[c] = task_flops(h.t2[c], h.s2, c);
+            pc.f1[c] = task_flops(h.t1[c], h.s1);
+            pc.f2[c] = task_flops(h.t2[c], h.s2);
         }
         pc.d_red = (RedTask *)put(h.red.data(), h.red.size() * sizeof(RedTask));
         pc.n_red = (int)h.red.size();
+        pc.slices = red_slices(h.red);
         pc.d_s1 = (Seg *)put(h.s1.data(), h.s1.size() * sizeof(Seg));
         pc.d_s2 = (Seg *)put(h.s2.data(), h.s2.size() * sizeof(Seg));
         k->chunks.push_back(pc);

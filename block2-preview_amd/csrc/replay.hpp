@@ -26,6 +26,7 @@ struct Chunk {
     std::vector<Seg> s1, s2;
     std::vector<RedTask> red; // split-K reductions of phase 2
     std::vector<BlockJob> jobs2; // phase-2 blocks (re-tiled by the packed plan)
+    int slices = 1; // of the largest tile in red
     uint64_t w_len = 0;       // W elements per right-hand side
     uint64_t p_len = 0;       // partial-tile elements per right-hand side
     // device copies (inside plan->dev)
@@ -44,7 +45,7 @@ struct b2g_plan_s {
     b2g_ctx ctx = nullptr;
     b2g_buf lbuf = nullptr, rbuf = nullptr;
     size_t x_len = 0, y_len = 0;
-    uint64_t macs = 0;
+    uint64_t macs = 0, macs2 = 0; // multiply-adds: both phases, phase 2
     std::vector<b2g::Chunk> chunks;
     uint64_t w_max = 0;
     void *dev = nullptr; // one allocation for all task / segment arrays
@@ -52,6 +53,8 @@ struct b2g_plan_s {
     void *w = nullptr; // W scratch
     size_t w_bytes = 0;
     uint64_t p_max = 0;   // partial elements per RHS (max over chunks)
+    uint64_t p_ref = 0;   // the same for the plain split (2048 deep, tiles to
+                          // 128): what the allocation-free entry admits by
     void *pbuf = nullptr; // split-K partial tiles (FP64)
     size_t p_bytes = 0;
     unsigned flags = 0;
@@ -83,9 +86,13 @@ namespace b2g {
 struct Tile {
     uint32_t row0, col0, tm, tn;
 };
-// reads the tiling settings of the environment (B2G_TILE, B2G_KSPLIT) for
-// the plans this host thread builds next; every plan builder calls it first
-void tile_env_refresh();
+// Tiling settings for the plan this host thread builds next; every plan
+// builder calls it first.  macs: multiply-adds of the plan's products (both
+// phases), macs2 those of the phase that is split along K (0: none), on
+// num_cu compute units.  B2G_TILE, B2G_TILE_CAP and B2G_KSPLIT override.
+void tile_env_refresh(uint64_t macs, uint64_t macs2, int num_cu);
+// 1024-element slices of the largest tile of a reduction list
+int red_slices(const std::vector<RedTask> &red);
 // tiling of an M x N output block for tasks of depth K (measured tile
 // rates, or B2G_TILE); the reference stays valid until the next call
 const std::vector<Tile> &tile_cover(uint32_t M, uint32_t N, uint64_t K,
@@ -93,6 +100,9 @@ const std::vector<Tile> &tile_cover(uint32_t M, uint32_t N, uint64_t K,
 Task make_task(uint64_t d_off, uint32_t ldd, uint32_t M, uint32_t N,
                const Tile &t, uint32_t sb, uint32_t se, uint32_t beta);
 int cfg_of(const Tile &t);
+// launch (task bucket) of a tile of the FP64 / FP32 (table 0) or split-BF16
+// (1) kernels
+int launch_of(const Tile &t, int table);
 // one task per tile of the block, all over segments [sb, se)
 void add_tiles(std::vector<Task> *tasks, uint64_t d_off, uint32_t M,
                uint32_t N, uint64_t K, uint32_t sb, uint32_t se,
@@ -103,8 +113,7 @@ void add_tiles(std::vector<Task> *tasks, uint64_t d_off, uint32_t M,
 void add_split_tiles(const std::vector<Seg> &s2, const BlockJob &j, int table,
                      std::vector<Task> *t2, std::vector<RedTask> &red,
                      uint64_t &p_len);
-double task_flops(const std::vector<Task> &tasks, const std::vector<Seg> &segs,
-                  int cfg);
+double task_flops(const std::vector<Task> &tasks, const std::vector<Seg> &segs);
 void sort_tasks(std::vector<Task> &tasks, const std::vector<Seg> &segs);
 // order one launch's tasks: grouped onto the 8 XCDs (the returned per-XCD
 // ranges) by segment list, or (by_b) by the B operand of their first
@@ -130,7 +139,7 @@ struct PkChunk {
     Task *d_t1[kTileConfigs] = {}, *d_t2[kTileConfigs] = {};
     Seg *d_s1 = nullptr, *d_s2 = nullptr;
     RedTask *d_red = nullptr;
-    int n_red = 0;
+    int n_red = 0, slices = 1;
     size_t n1[kTileConfigs] = {}, n2[kTileConfigs] = {};
     double f1[kTileConfigs] = {}, f2[kTileConfigs] = {};
     XcdSplit x1[kTileConfigs] = {}, x2[kTileConfigs] = {};

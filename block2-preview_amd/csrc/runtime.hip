@@ -33,10 +33,16 @@ void set_error(const std::string &msg) { g_err = msg; }
 // a host-side stand-in, never the device memory: kernels get the device
 // address taken by hipGetSymbolAddress at context creation
 // (g_scratch_ptr[device]).
+// A product is taken when its W windows and the partials of the plain split
+// (b2g_plan_s::p_ref) fill at most 64 MiB; the array also holds the
+// partials of the finer split small plans run with (at most
+// kPartialLimit elements per right-hand side).
 constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;
+constexpr uint64_t kPartialLimit = (uint64_t)12 << 20;
+constexpr size_t kScratchBytes = kNoAllocScratchBytes + kPartialLimit * 8;
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) double
-    scratch[kNoAllocScratchBytes / sizeof(double)];
+    scratch[kScratchBytes / sizeof(double)];
 static std::mutex g_scratch_mu;
 static void *g_scratch_ptr[kMaxDevices];
 
@@ -334,9 +340,9 @@ static double g_rates[2][kTileConfigs] = {
 static int size_index(uint32_t t) { return t == 32 ? 0 : t == 64 ? 1 : 2; }
 
 // candidate row (or column) covers of a dimension of length d
-static std::vector<std::vector<uint32_t>> covers(uint32_t d) {
-    std::vector<uint32_t> base(d / 128, 128u);
-    const uint32_t r = d % 128;
+static std::vector<std::vector<uint32_t>> covers(uint32_t d, uint32_t cap) {
+    std::vector<uint32_t> base(d / cap, cap);
+    const uint32_t r = d % cap;
     std::vector<std::vector<uint32_t>> out;
     if (r == 0) {
         out.push_back(base);
@@ -348,7 +354,7 @@ static std::vector<std::vector<uint32_t>> covers(uint32_t d) {
         uint32_t cov = 0;
         for (uint32_t t : tail)
             cov += t;
-        if (cov < r)
+        if (cov < r || tail[0] > cap)
             continue;
         std::vector<uint32_t> v = base;
         v.insert(v.end(), tail.begin(), tail.end());
@@ -373,10 +379,28 @@ static thread_local TileMemo t_memo;
 struct TileEnv {
     uint32_t fm = 0, fn = 0; // forced tile shape (0: measured rates)
     uint64_t ksplit = 2048;  // split-K depth threshold of phase 2
+    uint32_t cap = 128;      // largest tile side
 };
-static thread_local TileEnv t_env;
+// of the plan being built, and the settings it would have without regard to
+// its size
+static thread_local TileEnv t_env, t_plain;
 
-void tile_env_refresh() {
+// Plans below this many multiply-adds take tiles of up to 64 x 64: they have
+// too few 128-wide tiles to fill the chip.  FP64 product, one right-hand
+// side, tiles to 64 against to 128 at the better split of either:
+// 1.3e10 multiply-adds (n=30 M=1500) 817 / 925 us, 4.1e10 (n=36 M=2000)
+// 2236 / 2255 us and with four right-hand sides 8.98 / 8.48 ms, 1.1e11 (n=40
+// M=2500) 5736 / 5642 us.
+constexpr uint64_t kSmallPlanMacs = 25000000000ull;
+// Phase 2 is cut along K into about this many tasks of a full tile per
+// compute unit (between 64 deep, where a partial tile's write and read cost
+// as much as its products, and 2048): one task is a serial chain over its
+// segments, and a small site has a few hundred output tiles.  At n=26 M=1000
+// (tiles to 64) depths 256 / 512 / 1024 / 2048 take 410 / 397 / 428 / 460 us,
+// at n=8 M=50 depths 64 / 256 / 1024 take 48 / 59 / 107 us.
+constexpr uint64_t kSplitTasksPerCu = 6;
+
+void tile_env_refresh(uint64_t macs, uint64_t macs2, int num_cu) {
     TileEnv v;
     if (const char *e = getenv("B2G_TILE")) {
         // "T" (square) or "TMxTN", sizes from {32, 64, 128}
@@ -388,10 +412,29 @@ void tile_env_refresh() {
         if (nr >= 1 && okv(a) && okv(b))
             v.fm = a, v.fn = b;
     }
-    if (const char *e = getenv("B2G_KSPLIT"))
-        if (atoll(e) > 0)
-            v.ksplit = (uint64_t)atoll(e);
+    const char *ks = getenv("B2G_KSPLIT");
+    if (ks != nullptr && atoll(ks) > 0)
+        v.ksplit = (uint64_t)atoll(ks);
+    else
+        ks = nullptr;
+    t_plain = v;
+    if (macs < kSmallPlanMacs)
+        v.cap = 64;
+    if (const char *e = getenv("B2G_TILE_CAP"))
+        if (atoi(e) == 64 || atoi(e) == 128)
+            v.cap = (uint32_t)atoi(e);
+    if (ks == nullptr)
+        v.ksplit = std::min<uint64_t>(
+            2048, std::max<uint64_t>(64, macs2 / (kSplitTasksPerCu * num_cu *
+                                                  v.cap * v.cap)));
     t_env = v;
+}
+
+int red_slices(const std::vector<RedTask> &red) {
+    uint32_t a = 1024;
+    for (const RedTask &r : red)
+        a = std::max(a, r.tm * r.tn);
+    return (int)(a / 1024);
 }
 
 const std::vector<Tile> &tile_cover(uint32_t M, uint32_t N, uint64_t K,
@@ -407,7 +450,8 @@ const std::vector<Tile> &tile_cover(uint32_t M, uint32_t N, uint64_t K,
     const bool memo = M < (1u << 24) && N < (1u << 24);
     const uint64_t key = ((uint64_t)M << 36) | ((uint64_t)N << 12) |
                          ((uint64_t)(table == 1) << 11) |
-                         ((uint64_t)(fm >> 5) << 8) | ((uint64_t)(fn >> 5) << 4);
+                         ((uint64_t)(fm >> 5) << 8) | ((uint64_t)(fn >> 5) << 4) |
+                         (uint64_t)(t_env.cap >> 7);
     if (memo) {
         auto it = t_memo.map.find(key);
         if (it != t_memo.map.end())
@@ -418,8 +462,8 @@ const std::vector<Tile> &tile_cover(uint32_t M, uint32_t N, uint64_t K,
         cols.assign((N + fn - 1) / fn, fn);
     } else {
         double best = 1e300;
-        for (const auto &rc : covers(M))
-            for (const auto &cc : covers(N)) {
+        for (const auto &rc : covers(M, t_env.cap))
+            for (const auto &cc : covers(N, t_env.cap)) {
                 double c = 0;
                 for (uint32_t a : rc)
                     for (uint32_t b : cc)
@@ -456,7 +500,7 @@ Task make_task(uint64_t d_off, uint32_t ldd, uint32_t M, uint32_t N,
     k.col0 = t.col0;
     k.seg_begin = sb;
     k.seg_end = se;
-    k.beta = beta;
+    k.beta = beta | (uint32_t)cfg_of(t) << 4;
     return k;
 }
 
@@ -464,12 +508,23 @@ int cfg_of(const Tile &t) {
     return 3 * size_index(t.tm) + size_index(t.tn);
 }
 
+// The launch a tile belongs to: the FP64 / FP32 kernels (table 0) run every
+// shape up to 64 x 64 in one launch, that of 64 x 64, unless one shape is
+// forced; the split-BF16 kernels run one launch per shape.
+int launch_of(const Tile &t, int table) {
+    const int c = cfg_of(t);
+    if (table == 1 || t_env.fm != 0 || t.tm > 64 || t.tn > 64)
+        return c;
+    return kSmallCfg;
+}
+
 // one task per tile (phase 1 and unsplit phase-2 blocks)
 void add_tiles(std::vector<Task> *tasks, uint64_t d_off, uint32_t M,
                       uint32_t N, uint64_t K, uint32_t sb, uint32_t se,
                       uint32_t beta) {
     for (const Tile &t : tile_cover(M, N, K, 0))
-        tasks[cfg_of(t)].push_back(make_task(d_off, N, M, N, t, sb, se, beta));
+        tasks[launch_of(t, 0)].push_back(
+            make_task(d_off, N, M, N, t, sb, se, beta));
 }
 
 // Phase-2 tiles of an output block whose segments [sb, se) are deep: the
@@ -477,33 +532,53 @@ void add_tiles(std::vector<Task> *tasks, uint64_t d_off, uint32_t M,
 // ksplit(); each (tile, group) becomes a partial task writing a dense
 // TM x TN slot of the partial buffer, and a reduction task sums the slots in
 // group order (deterministic) into the output.
-void add_split_tiles(const std::vector<Seg> &s2, const BlockJob &j, int table,
-                     std::vector<Task> *t2, std::vector<RedTask> &red,
-                     uint64_t &p_len) {
-    std::vector<std::pair<uint32_t, uint32_t>> groups;
-    // maximum depth of one phase-2 task before its segment list is split
-    const uint64_t kmax = t_env.ksplit;
+typedef std::vector<std::pair<uint32_t, uint32_t>> SegGroups;
+static SegGroups split_groups(const std::vector<Seg> &s2, const BlockJob &j,
+                              int table, uint64_t kmax) {
+    SegGroups groups;
     // depth as the kernels walk it: every segment takes whole k-steps
     // (16 deep for the FP64 / FP32 kernels, 32 for the split-BF16 ones), so
     // that a long list of shallow segments is split like a deep one
     const uint64_t step = table == 1 ? 32 : 16;
-    uint64_t K = 0, acc = 0;
+    uint64_t acc = 0;
     uint32_t g0 = j.sb;
     for (uint32_t k = j.sb; k < j.se; k++) {
-        const uint64_t kk = (s2[k].K + step - 1) / step * step;
-        K += kk;
-        acc += kk;
+        acc += (s2[k].K + step - 1) / step * step;
         if (acc >= kmax && k + 1 < j.se) {
             groups.emplace_back(g0, k + 1);
             g0 = k + 1, acc = 0;
         }
     }
     groups.emplace_back(g0, j.se);
+    return groups;
+}
+
+// partial elements of the jobs under the settings `v`
+static uint64_t partial_len(const std::vector<Seg> &s2,
+                            const std::vector<BlockJob> &jobs,
+                            const TileEnv &v) {
+    const TileEnv kept = t_env;
+    t_env = v;
+    uint64_t len = 0;
+    for (const BlockJob &j : jobs) {
+        const size_t n = split_groups(s2, j, 0, v.ksplit).size();
+        if (n > 1)
+            for (const Tile &t : tile_cover(j.M, j.N, 1, 0))
+                len += n * t.tm * t.tn;
+    }
+    t_env = kept;
+    return len;
+}
+
+void add_split_tiles(const std::vector<Seg> &s2, const BlockJob &j, int table,
+                     std::vector<Task> *t2, std::vector<RedTask> &red,
+                     uint64_t &p_len) {
+    const SegGroups groups = split_groups(s2, j, table, t_env.ksplit);
     const std::vector<Tile> &tiles =
-        tile_cover(j.M, j.N, K / groups.size(), table);
+        tile_cover(j.M, j.N, 1, table);
     if (groups.size() == 1) {
         for (const Tile &t : tiles)
-            t2[cfg_of(t)].push_back(
+            t2[launch_of(t, table)].push_back(
                 make_task(j.d_off, j.ldd, j.M, j.N, t, j.sb, j.se, j.beta));
         return;
     }
@@ -515,9 +590,9 @@ void add_split_tiles(const std::vector<Seg> &s2, const BlockJob &j, int table,
             // p0 + g*tsz + (row - row0)*tn + (col - col0)  (mod 2^64)
             const uint64_t doff = p0 + g * tsz - (uint64_t)t.row0 * t.tn -
                                   (uint64_t)t.col0;
-            t2[cfg_of(t)].push_back(make_task(doff, t.tn, j.M, j.N, t,
-                                              groups[g].first,
-                                              groups[g].second, 2u));
+            t2[launch_of(t, table)].push_back(
+                make_task(doff, t.tn, j.M, j.N, t, groups[g].first,
+                          groups[g].second, 2u));
         }
         RedTask rt;
         rt.d_off = j.d_off;
@@ -540,12 +615,13 @@ void add_split_tiles(const std::vector<Seg> &s2, const BlockJob &j, int table,
 // multiply-adds x 2 of the tasks restricted to their tiles (the edge tiles'
 // masked rows and columns do not count)
 double task_flops(const std::vector<Task> &tasks,
-                         const std::vector<Seg> &segs, int cfg) {
+                  const std::vector<Seg> &segs) {
     double f = 0;
-    const uint32_t tm = 32u << (cfg / 3), tn = 32u << (cfg % 3);
     const std::vector<uint64_t> d = task_depths(tasks, segs);
     for (size_t i = 0; i < tasks.size(); i++) {
         const Task &t = tasks[i];
+        const uint32_t tm = (uint32_t)tile_m(task_cfg(t));
+        const uint32_t tn = (uint32_t)tile_n(task_cfg(t));
         const uint32_t m = std::min(tm, t.M - t.row0);
         const uint32_t n = std::min(tn, t.N - t.col0);
         f += 2.0 * m * n * (double)(d[i] - 1);
@@ -578,9 +654,11 @@ void sort_keyed(std::vector<std::pair<uint64_t, size_t>> &v) {
     }
 }
 
-// deepest first, creation order among equal depths
+// costliest first (depth times tile area), creation order among equal costs
 void sort_tasks(std::vector<Task> &tasks, const std::vector<Seg> &segs) {
-    const std::vector<uint64_t> d = task_depths(tasks, segs);
+    std::vector<uint64_t> d = task_depths(tasks, segs);
+    for (size_t i = 0; i < tasks.size(); i++)
+        d[i] *= (uint64_t)tile_area(task_cfg(tasks[i]));
     const uint64_t dmax =
         d.empty() ? 0 : *std::max_element(d.begin(), d.end());
     std::vector<std::pair<uint64_t, size_t>> order(tasks.size());
@@ -870,7 +948,15 @@ static int upload_chunks(b2g_plan p) {
 static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
                         const b2g_block *yb, size_t n_yb) {
     SetupTimer tm("plan");
-    tile_env_refresh();
+    uint64_t macs1 = 0, macs2 = 0;
+    for (size_t i = 0; i < n_pairs; i++) {
+        const b2g_pair &q = pairs[i];
+        macs1 += (uint64_t)q.c_m * q.c_n * q.v_n;
+        macs2 += (uint64_t)q.v_m * q.c_m * q.v_n;
+    }
+    p->macs = macs1 + macs2;
+    p->macs2 = macs2;
+    tile_env_refresh(p->macs, macs2, p->ctx->num_cu);
     const size_t llen = p->lbuf->n, rlen = p->rbuf->n;
     FlatMap<uint64_t, size_t, U64Hash> yidx(n_yb);
     std::vector<std::pair<uint64_t, size_t>> ysorted; // (offset, block)
@@ -881,7 +967,6 @@ static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
         ysorted.emplace_back(yb[i].off, i);
     }
     std::sort(ysorted.begin(), ysorted.end());
-    p->macs = 0;
     std::vector<size_t> whole, windows; // pair indices by kind
     // output block of each whole-block pair (by pair index)
     std::vector<uint32_t> yof(n_pairs, 0);
@@ -935,8 +1020,6 @@ static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
                         B2G_ERR_ARG, msg("V window outside its block"));
             windows.push_back(i);
         }
-        p->macs += (uint64_t)q.c_m * q.c_n * q.v_n +
-                   (uint64_t)q.v_m * q.c_m * q.v_n;
     }
     const uint64_t cap = w_cap_elems();
     // Chunks of the pairs in `idx` whose W scratch fits the cap.  Whole-block
@@ -1025,7 +1108,6 @@ static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
                 const BlockJob job{off, ldd, m, n, sb,
                                    (uint32_t)ch.s2.size(), beta};
                 ch.jobs2.push_back(job);
-                add_split_tiles(ch.s2, job, 0, ch.t2, ch.red, ch.p_len);
             };
             // phase 2: this chunk's pairs grouped by output block or window,
             // record order within a group
@@ -1073,16 +1155,35 @@ static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
                     g0 = g1;
                 }
             }
+            // phase-2 tiles; a plan that the allocation-free entry may run
+            // keeps its partials below the room that entry has for them
+            const bool small = ch.w_len * 4 <= kNoAllocScratchBytes;
+            if (small)
+                p->p_ref = std::max(p->p_ref,
+                                    partial_len(ch.s2, ch.jobs2, t_plain));
+            else
+                p->p_ref = ~(uint64_t)0 >> 8; // W alone is past its limit
+            while (small && (t_env.ksplit < t_plain.ksplit ||
+                             t_env.cap < t_plain.cap) &&
+                   partial_len(ch.s2, ch.jobs2, t_env) > kPartialLimit) {
+                if (t_env.ksplit < t_plain.ksplit)
+                    t_env.ksplit = std::min(2 * t_env.ksplit, t_plain.ksplit);
+                else
+                    t_env.cap = t_plain.cap;
+            }
+            for (const BlockJob &job : ch.jobs2)
+                add_split_tiles(ch.s2, job, 0, ch.t2, ch.red, ch.p_len);
             tm.mark("chunk tasks");
             for (int c = 0; c < kTileConfigs; c++) {
                 ch.x1[c] = xcd_order(ch.t1[c], ch.s1, xcd_enabled());
                 ch.x2[c] = xcd_order(ch.t2[c], ch.s2, xcd_enabled());
-                ch.f1[c] = task_flops(ch.t1[c], ch.s1, c);
-                ch.f2[c] = task_flops(ch.t2[c], ch.s2, c);
+                ch.f1[c] = task_flops(ch.t1[c], ch.s1);
+                ch.f2[c] = task_flops(ch.t2[c], ch.s2);
                 p->kflops[B2G_K_PHASE1 + c] += ch.f1[c];
                 p->kflops[B2G_K_PHASE2 + c] += ch.f2[c];
             }
             tm.mark("chunk order and flops");
+            ch.slices = red_slices(ch.red);
             p->w_max = std::max(p->w_max, ch.w_len);
             p->p_max = std::max(p->p_max, ch.p_len);
             p->chunks.push_back(std::move(ch));
@@ -1475,8 +1576,8 @@ static int hpsi_run(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
                 B2G_HIP(timed(B2G_K_SPLITK_REDUCE, ctx->stream,
                               [&](hipStream_t st) {
                     return launch_splitk_reduce<double>(
-                        y, P, kc.d_red, kc.n_red, p->y_len, pstride, beta0,
-                        n_rhs, grid, st);
+                        y, P, kc.d_red, kc.n_red, kc.slices, p->y_len,
+                        pstride, beta0, n_rhs, grid, st);
                 }));
             continue;
         }
@@ -1510,9 +1611,9 @@ static int hpsi_run(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
         const int nr = (int)ch.red.size();
         if (nr > 0)
             B2G_HIP(timed(B2G_K_SPLITK_REDUCE, ctx->stream, [&](hipStream_t st) {
-                return launch_splitk_reduce<double>(y, P, ch.d_red, nr,
-                                                    p->y_len, p->p_max, beta0,
-                                                    n_rhs, grid, st);
+                return launch_splitk_reduce<double>(
+                    y, P, ch.d_red, nr, ch.slices, p->y_len, p->p_max, beta0,
+                    n_rhs, grid, st);
             }));
     }
     return B2G_OK;
@@ -1554,12 +1655,16 @@ extern "C" int b2g_hpsi_noalloc(b2g_ctx ctx, b2g_plan p, const double *x,
     B2G_REQUIRE(p->ctx == ctx, B2G_ERR_ARG, "plan belongs to another context");
     const size_t es = precision == B2G_PREC_F64 ? 8 : 4;
     // W windows first, the split-K partials 256-byte aligned after them
-    const uint64_t w_bytes =
-        (std::max<uint64_t>(p->w_max, 1) * n_rhs * es + 255) & ~(uint64_t)255;
-    const uint64_t p_bytes = std::max<uint64_t>(p->p_max, 1) * n_rhs * 8;
-    if (w_bytes + p_bytes > kNoAllocScratchBytes) {
+    auto need = [p, es](int n, uint64_t partials, uint64_t &w_bytes) {
+        w_bytes = (std::max<uint64_t>(p->w_max, 1) * n * es + 255) &
+                  ~(uint64_t)255;
+        return w_bytes + std::max<uint64_t>(partials, 1) * n * 8;
+    };
+    uint64_t w_bytes = 0;
+    const uint64_t bytes = need(n_rhs, p->p_ref, w_bytes);
+    if (bytes > kNoAllocScratchBytes) {
         set_error("b2g_hpsi_noalloc: the product needs " +
-                  std::to_string(w_bytes + p_bytes) +
+                  std::to_string(bytes) +
                   " bytes of scratch; the allocation-free entry holds " +
                   std::to_string(kNoAllocScratchBytes));
         return B2G_ERR_ARG;
@@ -1567,12 +1672,26 @@ extern "C" int b2g_hpsi_noalloc(b2g_ctx ctx, b2g_plan p, const double *x,
     char *base = (char *)scratch_ptr(ctx->device);
     B2G_REQUIRE(base != nullptr, B2G_ERR_STATE,
                 "no scratch address for this device");
+    // right-hand sides run as many at a time as the array holds (their
+    // results do not depend on each other)
+    int step = n_rhs;
+    while (step > 1 && need(step, p->p_max, w_bytes) > kScratchBytes)
+        step = (step + 1) / 2;
+    B2G_REQUIRE(need(step, p->p_max, w_bytes) <= kScratchBytes, B2G_ERR_ARG,
+                "b2g_hpsi_noalloc: split-K partials exceed the scratch");
     B2G_HIP(hipSetDevice(ctx->device));
     // nothing in the scratch needs to start at zero: phase 1 writes every
     // W element phase 2 reads, and each split-K partial is written before
     // the reduction reads it
-    return hpsi_run(ctx, p, x, y, n_rhs, scale, accumulate, precision, base,
-                    (double *)(base + w_bytes));
+    for (int r = 0; r < n_rhs; r += step) {
+        const int rc = hpsi_run(ctx, p, x + (size_t)r * p->x_len,
+                                y + (size_t)r * p->y_len,
+                                std::min(step, n_rhs - r), scale, accumulate,
+                                precision, base, (double *)(base + w_bytes));
+        if (rc != B2G_OK)
+            return rc;
+    }
+    return B2G_OK;
 }
 
 // ----------------------------------------------------------------- diagonal

@@ -792,6 +792,10 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
     // quotients
     {
         TaskSet ts;
+        uint64_t macs = 0;
+        for (size_t i = 0; i < nm; i++)
+            macs += (uint64_t)n[i] * n[i] * n[i];
+        tile_env_refresh(macs, 0, ctx->num_cu);
         for (size_t i = 0; i < nm; i++) {
             if (n[i] == 0)
                 continue;
@@ -1100,7 +1104,14 @@ static int split_impl(b2g_ctx ctx, int symmetry, const b2g_sparse_info *wfn,
     *out = nullptr;
     B2G_HIP(hipSetDevice(ctx->device));
     SetupTimer tm("split");
-    tile_env_refresh();
+    {
+        uint64_t macs = 0; // of the density matrix (the split's are fewer)
+        for (int i = 0; i < wfn->n; i++) {
+            const uint64_t m = wfn->n_states_bra[i], n = wfn->n_states_ket[i];
+            macs += m * n * (trace_right ? m : n) * n_roots;
+        }
+        tile_env_refresh(macs, 0, ctx->num_cu);
+    }
     const Symm sy = symmetry == B2G_SZ ? Symm::SZ : Symm::SU2;
     const int nw = wfn->n;
     const uint64_t wdq = wfn->delta_quantum;

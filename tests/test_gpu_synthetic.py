@@ -87,6 +87,21 @@ def test_split_k(gpu_ctx, problem, ksplit):
         assert rel(y[r], ys[r]) < 2e-6, r
 
 
+@pytest.mark.parametrize("cap", ["64", "128"])
+@pytest.mark.parametrize("ksplit", ["16", "64", "2048"])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_tile_cap(gpu_ctx, problem, cap, ksplit, precision):
+    # tiles of 32 and 64 mixed in one launch, and up to 128 with one launch
+    # per larger shape, each with shallow and deep partial tasks (1e-12: sums
+    # of 1e4 FP64 products; FP32 as below)
+    pb, xs, ys = problem
+    print("cap", cap, "ksplit", ksplit, precision, flush=True)
+    y = run(gpu_ctx, pb, xs, {"B2G_TILE_CAP": cap, "B2G_KSPLIT": ksplit},
+            precision=precision)
+    for r in range(4):
+        assert rel(y[r], ys[r]) < (1e-12 if precision == "f64" else 2e-6), r
+
+
 @pytest.mark.parametrize("tile", TILES)
 def test_bf16x3_tile_configurations(gpu_ctx, problem, tile):
     # split-BF16 three-term kernels, every tile shape; 1e-4 relative

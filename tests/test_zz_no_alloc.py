@@ -44,7 +44,8 @@ def _products(ctx, pb, nrhs, precision, accumulate, seed):
 
 
 @pytest.mark.parametrize("nrhs,precision,accumulate",
-                         [(1, "f64", 0), (4, "f64", 1), (2, "f32", 0)])
+                         [(1, "f64", 0), (4, "f64", 1), (2, "f32", 0),
+                          (7, "f64", 1)])  # 7: run in two batches
 def test_noalloc_matches_hpsi_on_two_calls(gpu_ctx, nrhs, precision,
                                            accumulate):
     # first a larger problem, then a smaller one: the second call must not
