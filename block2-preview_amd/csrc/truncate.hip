@@ -15,9 +15,11 @@
 //   * density matrix blocks D[b] = sum over wavefunction blocks a of
 //     psi_a psi_a^T (trace_right) or psi_a^T psi_a, as output-stationary
 //     grouped-GEMM tasks (the H*psi engine, FP64 MFMA);
-//   * a batched symmetric eigensolver: block Jacobi over 16-column blocks.
+//   * a batched symmetric eigensolver: one QR step (A <- Q^T A Q, V <- Q,
+//     blocked Householder), then block Jacobi over 16-column blocks.
 //     Each round pairs the column blocks of every matrix (round-robin); the
-//     32 x 32 subproblem of a pair is diagonalised by cyclic Jacobi in LDS,
+//     32 x 32 subproblem of a pair is swept by cyclic Jacobi in LDS (the
+//     entries between its two blocks; those within a block once per sweep),
 //     giving an orthogonal Q, and the whole matrix is updated as
 //     A <- J^T A J, V <- V J with J the block-diagonal of the round's Qs:
 //     every 32 x 32 region (pair P rows, pair R columns) becomes
@@ -25,7 +27,7 @@
 //     and columns, which no rotation touches (a zero off-diagonal entry is
 //     never rotated), so positions >= n stay out of the spectrum.  A global
 //     sweep is max(nb) - 1 rounds (smaller matrices cycle through their own
-//     rounds); the solve ends after a sweep with no rotation anywhere.
+//     rounds); the solve ends when no entry passes the rotation test.
 //     Off-diagonal entries below 64 eps ||A_b||_F are left (the rounding
 //     level of a region update), so eigenvalues carry an absolute error of
 //     that order, like xsyev's;
@@ -157,27 +159,32 @@ __global__ void jacobi_floor_kernel(JacBlock *__restrict__ blocks, int nblocks,
     blocks[b].floor_abs = 64.0 * 2.220446049250313e-16 * sqrt(s);
 }
 
-// One kJS x kJS pair subproblem per workgroup: cyclic Jacobi in LDS,
-// sweeps until one applies no rotation (at most max_sweeps); writes the
-// accumulated rotation Q and whether it differs from I, and counts rotating
-// pairs.  The kJB rotations of a round act on disjoint row / column pairs,
-// so thread (k, l) applies rotation k to the rows and rotation l to the
-// columns of the 2 x 2 block where they meet, reading its four entries
-// before writing them; the diagonal block of each rotating pair gets its
-// exact rotated values.  Two barriers per round: after the angles and
-// after the block updates.
+// One kJS x kJS pair subproblem per workgroup: a cyclic Jacobi sweep in LDS;
+// writes the accumulated rotation Q and whether it differs from I, and
+// counts rotating pairs.  `cross`: only the kJB x kJB entries between the two
+// column blocks are swept (16 rounds of 16 disjoint rotations instead of the
+// 31 of the whole subproblem); the entries within a block are swept once per
+// outer sweep, in its first round.
+//
+// The kJB rotations of a round act on disjoint row / column pairs, so thread
+// (k, l) applies rotation k to the rows and rotation l to the columns of the
+// 2 x 2 block where they meet.  S is read from one buffer and written to the
+// other, and every wave holds all 16 rotations in its lanes (thread (k, l)
+// computes rotation l and fetches rotation k from lane k), so a round takes
+// one barrier and no exchange of angles through LDS.  Bound by the latency
+// of one round: two reciprocal square roots, two LDS accesses, a barrier.
+// n=40 M=3000 truncation (600 states in the largest block): 27.5 us per
+// launch with separate angle and block phases over 31 rounds, 13.3 us
+// now.
 __global__ __launch_bounds__(256) void jacobi_pair_kernel(
     const JacBlock *__restrict__ blocks, const JacTask *__restrict__ tasks,
     const double *__restrict__ A, double *__restrict__ Q,
-    int *__restrict__ qflag, int round, double tol, int max_sweeps,
+    int *__restrict__ qflag, int round, double tol, int cross, int max_sweeps,
     unsigned *__restrict__ nrot) {
     static_assert(kJB * kJB == 256, "one thread per 2 x 2 block of a round");
-    __shared__ double S[kJS * kJLD];
+    __shared__ double S[2][kJS * kJLD];
     __shared__ double U[kJS * kJLD];
-    __shared__ double rc[kJB], rs[kJB], rpp[kJB], rqq[kJB];
-    __shared__ int rp[kJB], rq[kJB], rot[kJB];
-    __shared__ int any_rot, need;
-    __shared__ unsigned rmask[2]; // rotating pairs of a round, by parity
+    __shared__ int need;
     const JacTask tk = tasks[blockIdx.x];
     const JacBlock bl = blocks[tk.blk];
     const uint32_t N = bl.nb * kJB;
@@ -192,103 +199,89 @@ __global__ __launch_bounds__(256) void jacobi_pair_kernel(
     rr_pair((int)bl.nb, round % (int)(bl.nb - 1), (int)tk.x, bi, bj);
     for (int e = tid; e < kJS * kJS; e += 256) {
         const int l = e / kJS, c = e % kJS;
-        S[l * kJLD + c] = A[bl.a_off + (uint64_t)pair_index(bi, bj, l) * N +
-                            pair_index(bi, bj, c)];
+        S[0][l * kJLD + c] = A[bl.a_off + (uint64_t)pair_index(bi, bj, l) * N +
+                               pair_index(bi, bj, c)];
         U[l * kJLD + c] = l == c ? 1.0 : 0.0;
     }
-    int rotated = 0;
+    const int k = tid >> 4, l = tid & 15;
+    const int nrounds = cross ? kJB : kJS - 1;
+    int rotated = 0, cur = 0;
     for (int sw = 0; sw < max_sweeps; sw++) {
         if (tid == 0)
-            any_rot = 0, need = 0;
+            need = 0;
         __syncthreads();
-        // skip the sweep when no off-diagonal entry passes the test
+        // skip the sweep when no swept entry passes the test
         for (int e = tid; e < kJS * kJS; e += 256) {
             const int i = e / kJS, j = e % kJS;
-            if (i < j && wants(S[i * kJLD + j], S[i * kJLD + i],
-                               S[j * kJLD + j]))
+            if (i < j && (!cross || (i < kJB && j >= kJB)) &&
+                wants(S[cur][i * kJLD + j], S[cur][i * kJLD + i],
+                      S[cur][j * kJLD + j]))
                 need = 1;
         }
         __syncthreads();
         if (!need)
             break;
-        for (int r = 0; r < kJS - 1; r++) {
-            int f = 0;
-            if (tid < kJB) {
-                int p, q;
-                rr_pair(kJS, r, tid, p, q);
-                const double apq = S[p * kJLD + q], app = S[p * kJLD + p],
-                             aqq = S[q * kJLD + q];
-                double c = 1.0, s = 0.0;
-                if (wants(apq, app, aqq)) {
-                    // symmetric Schur rotation zeroing a_pq
-                    const double th = (aqq - app) / (2.0 * apq);
-                    double t;
-                    if (fabs(th) > 1e150)
-                        t = 0.5 / th;
-                    else
-                        t = (th >= 0.0 ? 1.0 : -1.0) /
-                            (fabs(th) + sqrt(th * th + 1.0));
-                    c = rsqrt(t * t + 1.0);
-                    s = t * c;
-                    rpp[tid] = app - t * apq;
-                    rqq[tid] = aqq + t * apq;
-                    f = 1;
-                    any_rot = 1;
-                }
-                rc[tid] = c;
-                rs[tid] = s;
-                rp[tid] = p;
-                rq[tid] = q;
-                rot[tid] = f;
+        int any = 0;
+        for (int r = 0; r < nrounds; r++) {
+            int pk, qk, pl, ql;
+            if (cross) {
+                pk = k, qk = kJB + ((k + r) & (kJB - 1));
+                pl = l, ql = kJB + ((l + r) & (kJB - 1));
+            } else {
+                rr_pair(kJS, r, k, pk, qk);
+                rr_pair(kJS, r, l, pl, ql);
             }
-            // the angle threads are lanes 0..kJB-1 of wave 0: its ballot is the
-            // round's rotation mask.  Slot r & 1 is rewritten two rounds
-            // later, after a barrier every wave must reach once it has read
-            // the slot.
-            const unsigned long long bm = __ballot(f);
-            if (tid == 0)
-                rmask[r & 1] = (unsigned)bm;
-            __syncthreads();
-            // a round without rotations leaves S and U as they are
-            if (rmask[r & 1] == 0u)
+            const double *Sc = S[cur];
+            const double apq = Sc[pl * kJLD + ql], app = Sc[pl * kJLD + pl],
+                         aqq = Sc[ql * kJLD + ql];
+            const bool rl = wants(apq, app, aqq);
+            // lanes 0..15 of a wave hold the 16 rotations of the round
+            const unsigned m = (unsigned)(__ballot(rl) & 0xFFFFu);
+            // a round without rotations leaves S and U as they are (every
+            // wave sees the same values)
+            if (m == 0u)
                 continue;
-            // the 2 x 2 block of pair k's rows and pair l's columns, for
-            // thread (k, l): rows rotated by pair k, then columns by pair l
-            // (a pair that does not rotate has c = 1, s = 0), and the
-            // columns of U by pair l.  The blocks partition S and U.
-            {
-                const int k = tid >> 4, l = tid & 15;
-                const unsigned m = rmask[r & 1];
-                const bool rk = (m >> k) & 1u, rl = (m >> l) & 1u;
-                if (rk || rl) {
-                    const int pk = rp[k], qk = rq[k], pl = rp[l], ql = rq[l];
-                    const double ck = rc[k], sk = rs[k], cl = rc[l], sl = rs[l];
-                    const double a = S[pk * kJLD + pl], b = S[pk * kJLD + ql],
-                                 c = S[qk * kJLD + pl], d = S[qk * kJLD + ql];
-                    const double xa = ck * a - sk * c, xb = ck * b - sk * d;
-                    const double xc = sk * a + ck * c, xd = sk * b + ck * d;
-                    double na = cl * xa - sl * xb, nb = sl * xa + cl * xb;
-                    double nc = cl * xc - sl * xd, nd = sl * xc + cl * xd;
-                    if (k == l) // exact rotated 2 x 2 block of the pair
-                        na = rpp[k], nb = 0.0, nc = 0.0, nd = rqq[k];
-                    S[pk * kJLD + pl] = na;
-                    S[pk * kJLD + ql] = nb;
-                    S[qk * kJLD + pl] = nc;
-                    S[qk * kJLD + ql] = nd;
-                    if (rl) {
-                        const double u0 = U[pk * kJLD + pl], u1 = U[pk * kJLD + ql],
-                                     u2 = U[qk * kJLD + pl], u3 = U[qk * kJLD + ql];
-                        U[pk * kJLD + pl] = cl * u0 - sl * u1;
-                        U[pk * kJLD + ql] = sl * u0 + cl * u1;
-                        U[qk * kJLD + pl] = cl * u2 - sl * u3;
-                        U[qk * kJLD + ql] = sl * u2 + cl * u3;
-                    }
-                }
+            any = 1;
+            const double a = Sc[pk * kJLD + pl], b = Sc[pk * kJLD + ql],
+                         c = Sc[qk * kJLD + pl], d = Sc[qk * kJLD + ql];
+            double u[4];
+            if (rl) {
+                u[0] = U[pk * kJLD + pl], u[1] = U[pk * kJLD + ql];
+                u[2] = U[qk * kJLD + pl], u[3] = U[qk * kJLD + ql];
             }
+            double cl = 1.0, sl = 0.0, tl = 0.0;
+            if (rl) {
+                // symmetric Schur rotation zeroing a_pq: with h = (a_qq -
+                // a_pp, 2 a_pq), cos 2 phi = |h_0| / |h|, sin 2 phi = h_1 / |h|
+                const double h0 = aqq - app, h1 = 2.0 * apq;
+                const double rh = rsqrt(fma(h0, h0, h1 * h1));
+                const double c2 = fma(0.5 * fabs(h0), rh, 0.5);
+                const double rc = rsqrt(c2);
+                cl = c2 * rc;
+                sl = 0.5 * (h0 < 0.0 ? -h1 : h1) * rh * rc;
+                tl = sl * rc;
+            }
+            const double ck = __shfl(cl, k), sk = __shfl(sl, k);
+            const double xa = ck * a - sk * c, xb = ck * b - sk * d;
+            const double xc = sk * a + ck * c, xd = sk * b + ck * d;
+            double na = cl * xa - sl * xb, nb = sl * xa + cl * xb;
+            double nc = cl * xc - sl * xd, nd = sl * xc + cl * xd;
+            if (k == l && rl) // exact rotated 2 x 2 block of the pair
+                na = app - tl * apq, nb = 0.0, nc = 0.0, nd = aqq + tl * apq;
+            double *Sn = S[cur ^ 1];
+            Sn[pk * kJLD + pl] = na;
+            Sn[pk * kJLD + ql] = nb;
+            Sn[qk * kJLD + pl] = nc;
+            Sn[qk * kJLD + ql] = nd;
+            if (rl) {
+                U[pk * kJLD + pl] = cl * u[0] - sl * u[1];
+                U[pk * kJLD + ql] = sl * u[0] + cl * u[1];
+                U[qk * kJLD + pl] = cl * u[2] - sl * u[3];
+                U[qk * kJLD + ql] = sl * u[2] + cl * u[3];
+            }
+            cur ^= 1;
             __syncthreads();
         }
-        const int any = any_rot;
-        __syncthreads(); // every thread has read any_rot before its reset
         if (!any)
             break;
         rotated = 1;
@@ -301,6 +294,28 @@ __global__ __launch_bounds__(256) void jacobi_pair_kernel(
         if (rotated)
             atomicAdd(nrot, 1u);
     }
+}
+
+// *flag = 1 when any matrix has an entry above the diagonal that passes the
+// rotation test (the sweep it stands for would be 2 (max nb - 1) launches)
+__global__ __launch_bounds__(256) void jacobi_check_kernel(
+    const JacBlock *__restrict__ blocks, const double *__restrict__ A,
+    double tol, unsigned *__restrict__ flag) {
+    const JacBlock bl = blocks[blockIdx.y];
+    const uint32_t N = bl.nb * kJB;
+    const double *a = A + bl.a_off;
+    const double tol2 = tol * tol;
+    bool any = false;
+    for (uint32_t i = blockIdx.x; i < bl.n; i += gridDim.x) {
+        const double d = a[(uint64_t)i * N + i];
+        for (uint32_t j = i + 1 + threadIdx.x; j < bl.n; j += 256) {
+            const double v = a[(uint64_t)i * N + j];
+            any = any || (fabs(v) > bl.floor_abs &&
+                          v * v > tol2 * fabs(d * a[(uint64_t)j * N + j]));
+        }
+    }
+    if (any)
+        *flag = 1u;
 }
 
 typedef double jv4d __attribute__((ext_vector_type(4)));
@@ -336,7 +351,8 @@ __device__ __forceinline__ void mm_pos(int r, int &row, int &col) {
     col = 16 * (w & 1) + (lane & 15);
 }
 
-// Region update A_PR <- Q_P^T A_PR Q_R (kind 1) and V slice update
+// Region update A_PR <- Q_P^T A_PR Q_R with its mirror image A_RP (kind 1,
+// pairs P <= R) and V slice update
 // V[rows, P] <- V[rows, P] Q_P (kind 2) of one round.  Two LDS buffers:
 // the operand and one Q; the product A_PR Q_R goes back into the operand
 // buffer and the final result from registers to memory.
@@ -418,6 +434,23 @@ __global__ __launch_bounds__(256) void jacobi_update_kernel(
             A[bl.a_off + (uint64_t)pair_index(pi, pj, row) * N +
               pair_index(ri, rj, col)] = acc[r4];
         }
+        if (tk.x == tk.y)
+            return;
+        // the mirrored region, rows of it along consecutive lanes
+        __syncthreads();
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+            int row, col;
+            mm_pos(r4, row, col);
+            X[row * kJLD + col] = acc[r4];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < EPT; i++) {
+            const int e = tid + 256 * i, l = e / kJS, c = e % kJS;
+            A[bl.a_off + (uint64_t)pair_index(ri, rj, l) * N +
+              pair_index(pi, pj, c)] = X[c * kJLD + l];
+        }
     } else {
         if (!qflag[bl.f_off + tk.x])
             return;
@@ -447,6 +480,339 @@ __global__ __launch_bounds__(256) void jacobi_update_kernel(
             mm_pos(r4, row, col);
             V[bl.a_off + (uint64_t)(row0 + row) * N + pair_index(pi, pj, col)] =
                 acc[r4];
+        }
+    }
+}
+
+// ------------------------------------------------------ QR preconditioning
+// Before the Jacobi iteration every matrix is replaced by A1 = R Q = Q^T A Q
+// of its QR factorisation A = Q R, and V starts at Q: one step of the QR
+// algorithm, which gathers a graded spectrum (a density matrix's weights
+// decay over many decades) along the diagonal.  Jacobi then needs 5 to 7
+// sweeps where it needed 20 to 26 (random eigenvectors, weights over 8 to 14
+// decades, n = 128 and 300); a flat spectrum (2 decades) gains 11 -> 9.  The
+// similarity is orthogonal, so nothing is assumed about A.  Blocked
+// Householder, panels of kJB columns: H_c = I - w_c w_c^T (w scaled to
+// |w|^2 = 2), H_1 .. H_16 = I - W T W^T with T^-1 = I + the strictly upper
+// part of W^T W.  W of column c sits in column c of H (rows >= c).
+constexpr int kQrWaves = 8;      // of a panel's workgroup
+constexpr int kMaxQrBlocks = 72; // orders above 1152 are iterated as they are
+
+// value of lane C of each row of 16 lanes
+template <int C> __device__ __forceinline__ double row_bcast(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x150 + C,
+                                               0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(
+        0, (int)(uint32_t)(u >> 32), 0x150 + C, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (uint64_t)(uint32_t)hi << 32 |
+                                          (uint64_t)(uint32_t)lo);
+}
+
+// Column C of the panel: reflector, its application to the columns after it,
+// and its products with the reflectors before it.  Thread (wave, g, k) holds
+// column k of rows c0 + 32 i + 4 wave + g; one reduction of x_C . x_k over
+// the rows >= C (all k at once) gives norm and projections.
+template <int R, int C>
+__device__ __forceinline__ void qr_column(double (&x)[R],
+                                          double (&red)[2][kQrWaves][16],
+                                          double (&piv)[2][16],
+                                          double (&G)[16][17], double &diag) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int k = lane & 15, g = lane >> 4;
+    const int lr = 4 * wave + g; // local row of i = 0
+    double s = 0.0, v[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        v[i] = row_bcast<C>(x[i]);
+        if (i == 0 && lr < C)
+            v[0] = 0.0;
+        s = fma(v[i], x[i], s);
+    }
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    if (g == 0)
+        red[C & 1][wave][k] = s;
+    if (lr == C)
+        piv[C & 1][k] = x[0];
+    // one barrier per column: the slots written now were last read two
+    // columns ago, before the barrier of the column between
+    __syncthreads();
+    double gk = 0.0;
+#pragma unroll
+    for (int w = 0; w < kQrWaves; w++)
+        gk += red[C & 1][w][k];
+    const double pk = piv[C & 1][k];
+    const double gc = row_bcast<C>(gk), pc = row_bcast<C>(pk);
+    double beta = pc, v0 = pc, sc = 0.0, ws = 0.0;
+    if (gc > 1e-307) { // else the column is zero: H = I
+        const double nrm = sqrt(gc);
+        beta = pc >= 0.0 ? -nrm : nrm;
+        v0 = pc - beta;
+        sc = 1.0 / (nrm * fabs(v0));
+        ws = sqrt(sc);
+    }
+    const double dot = gk - beta * pk; // v . x_k (w_k for k < C)
+    if (k < C && lane < 16 && wave == 0)
+        G[k][C] = ws * dot;
+    const double f = k > C ? sc * dot : 0.0;
+    if (k == C)
+        diag = beta;
+    if (lr == C)
+        v[0] = v0;
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        if (k > C)
+            x[i] = fma(-f, v[i], x[i]);
+        else if (k == C && !(i == 0 && lr < C))
+            x[i] = v[i] * ws;
+    }
+}
+
+template <int R, int C>
+__device__ __forceinline__ void qr_columns(double (&x)[R],
+                                           double (&red)[2][kQrWaves][16],
+                                           double (&piv)[2][16],
+                                           double (&G)[16][17], double &diag) {
+    if constexpr (C < 16) {
+        qr_column<R, C>(x, red, piv, G, diag);
+        qr_columns<R, C + 1>(x, red, piv, G, diag);
+    }
+}
+
+// Panel p of every matrix, one workgroup each, up to 32 R rows below the
+// panel's first: the panel in registers, one barrier per column.  A receives
+// R's columns (zeros below the diagonal), H the reflectors, T the panel's T.
+template <int R>
+__global__ __launch_bounds__(64 * kQrWaves) void qr_panel_kernel(
+    const JacBlock *__restrict__ blocks, double *__restrict__ A,
+    double *__restrict__ H, double *__restrict__ T, int p) {
+    __shared__ double red[2][kQrWaves][16], piv[2][16], G[16][17];
+    const JacBlock bl = blocks[blockIdx.x];
+    if (p >= (int)bl.nb || bl.nb > kMaxQrBlocks)
+        return;
+    const int N = (int)bl.nb * kJB, c0 = p * kJB;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int k = lane & 15, lr = 4 * wave + (lane >> 4);
+    double *Ab = A + bl.a_off + (uint64_t)c0 * N + c0 + k;
+    double *Hb = H + bl.a_off + (uint64_t)c0 * N + c0 + k;
+    double x[R], diag = 0.0;
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const int r = lr + 32 * i;
+        x[i] = c0 + r < N ? Ab[(uint64_t)r * N] : 0.0;
+    }
+    if (threadIdx.x < 16 * 17)
+        (&G[0][0])[threadIdx.x] = 0.0;
+    __syncthreads();
+    qr_columns<R, 0>(x, red, piv, G, diag);
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const int r = lr + 32 * i;
+        if (c0 + r < N) {
+            Ab[(uint64_t)r * N] = r < k ? x[i] : r == k ? diag : 0.0;
+            Hb[(uint64_t)r * N] = r < k ? 0.0 : x[i];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 16) { // column of (I + striu G)^-1
+        const int c = threadIdx.x;
+        double t[16];
+#pragma unroll
+        for (int i = 15; i >= 0; i--) {
+            double s = i == c ? 1.0 : 0.0;
+#pragma unroll
+            for (int j = i + 1; j < 16; j++)
+                s -= G[i][j] * t[j];
+            t[i] = s;
+            T[bl.q_off + (uint64_t)p * 256 + i * 16 + c] = s;
+        }
+    }
+}
+
+typedef double qv4d __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ qv4d qr_mfma(double a, double b, qv4d c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// 32 columns right of panel p: X <- X - W T^T (W^T X) on FP64 MFMA.  Lane l
+// feeds A[l % 16][l / 16] and B[l / 16][l % 16]; accumulator element q is
+// D[4 q + l / 16][l % 16].
+__global__ __launch_bounds__(512) void qr_update_kernel(
+    const JacBlock *__restrict__ blocks, double *__restrict__ A,
+    const double *__restrict__ H, const double *__restrict__ T, int p) {
+    __shared__ double part[8][16][33], Y[16][33], Tm[16][17];
+    const JacBlock bl = blocks[blockIdx.y];
+    const int N = (int)bl.nb * kJB, c0 = p * kJB;
+    const int c1 = c0 + kJB + 32 * (int)blockIdx.x;
+    if (c1 >= N || bl.nb > kMaxQrBlocks)
+        return;
+    const bool two = c1 + 16 < N;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    double *Ab = A + bl.a_off;
+    const double *Hb = H + bl.a_off + c0;
+    if (tid < 256)
+        Tm[tid >> 4][tid & 15] = T[bl.q_off + (uint64_t)p * 256 + tid];
+    qv4d acc[2] = {qv4d{0, 0, 0, 0}, qv4d{0, 0, 0, 0}};
+#pragma unroll 4
+    for (int r = c0 + 4 * wave; r < N; r += 32) {
+        const uint64_t row = (uint64_t)(r + lk) * N;
+        const double a = Hb[row + lr];
+        const double b0 = Ab[row + c1 + lr];
+        const double b1 = two ? Ab[row + c1 + 16 + lr] : 0.0;
+        acc[0] = qr_mfma(a, b0, acc[0]);
+        acc[1] = qr_mfma(a, b1, acc[1]);
+    }
+    mfma_settle<qv4d, 2>(&acc[0]);
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            part[wave][4 * q + lk][16 * h + lr] = acc[h][q];
+    __syncthreads();
+    const int m = tid >> 5, n = tid & 31;
+    {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < 8; w++)
+            s += part[w][m][n];
+        __syncthreads();
+        part[0][m][n] = s;
+    }
+    __syncthreads();
+    {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+            s = fma(Tm[k][m], part[0][k][n], s);
+        Y[m][n] = s;
+    }
+    __syncthreads();
+    for (int rt = p + wave; rt < (int)bl.nb; rt += 8) {
+        acc[0] = acc[1] = qv4d{0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const double a = Hb[(uint64_t)(16 * rt + lr) * N + 4 * s + lk];
+            acc[0] = qr_mfma(a, Y[4 * s + lk][lr], acc[0]);
+            acc[1] = qr_mfma(a, Y[4 * s + lk][16 + lr], acc[1]);
+        }
+        mfma_settle<qv4d, 2>(&acc[0]);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            double *d = Ab + (uint64_t)(16 * rt + 4 * q + lk) * N + c1 + lr;
+            d[0] -= acc[0][q];
+            if (two)
+                d[16] -= acc[1][q];
+        }
+    }
+}
+
+// Rows i0 .. i0 + 15 of R (z = 0) or I (z = 1) times all reflectors of the
+// matrix, panel after panel: S <- S - (S W) T W^T, with S^T in registers (an
+// accumulator tile of S^T is the B operand of its own product).  Wave w
+// holds the column tiles w, w + 4, ...; one launch per range (lo, hi] of nb,
+// so that small matrices run with few registers.  Out: A1 (= R Q, symmetric, written
+// transposed) and V = Q; matrices too large for it are copied, V = I.
+template <int NT>
+__global__ __launch_bounds__(256) void qr_apply_kernel(
+    const JacBlock *__restrict__ blocks, const double *__restrict__ A,
+    const double *__restrict__ H, const double *__restrict__ T,
+    double *__restrict__ A1, double *__restrict__ V, int lo, int hi) {
+    __shared__ double part[4][16][17], Y[16][17], Tm[16][17];
+    const JacBlock bl = blocks[blockIdx.y];
+    const int nb = (int)bl.nb, N = nb * kJB, i0 = 16 * (int)blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const bool ident = blockIdx.z == 1;
+    if (i0 >= N || nb <= lo || nb > hi)
+        return;
+    if (nb > kMaxQrBlocks) {
+        for (int e = tid; e < 16 * N; e += 256) {
+            const uint64_t o = bl.a_off + (uint64_t)i0 * N + e;
+            if (ident)
+                V[o] = e % N == i0 + e / N ? 1.0 : 0.0;
+            else
+                A1[o] = A[o];
+        }
+        return;
+    }
+    qv4d z[NT];
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+        const int t = wave + 4 * i;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int c = 16 * t + 4 * q + lk;
+            z[i][q] = t >= nb ? 0.0
+                      : ident ? (c == i0 + lr ? 1.0 : 0.0)
+                              : A[bl.a_off + (uint64_t)(i0 + lr) * N + c];
+        }
+    }
+    for (int p = 0; p < nb; p++) {
+        const double *Hb = H + bl.a_off + p * kJB;
+        Tm[tid >> 4][tid & 15] = T[bl.q_off + (uint64_t)p * 256 + tid];
+        // the panel's reflectors as A operands of both products, loaded
+        // together (tiles above the panel hold none)
+        double h1[NT][4], h2[NT][4];
+#pragma unroll
+        for (int i = 0; i < NT; i++) {
+            const int t = wave + 4 * i;
+            const bool in = t >= p && t < nb;
+            const uint64_t r1 = (uint64_t)(16 * (in ? t : p) + lk) * N + lr;
+            const uint64_t r2 = (uint64_t)(16 * (in ? t : p) + lr) * N + lk;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const double a = Hb[r1 + (uint64_t)(4 * q) * N];
+                const double b = Hb[r2 + 4 * q];
+                h1[i][q] = in ? a : 0.0;
+                h2[i][q] = in ? -b : 0.0;
+            }
+        }
+        qv4d acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < NT; i++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                acc = qr_mfma(h1[i][q], z[i][q], acc);
+        mfma_settle<qv4d, 1>(&acc);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            part[wave][4 * q + lk][lr] = acc[q];
+        __syncthreads();
+        const int m = tid >> 4, n = tid & 15;
+        const double y = (part[0][m][n] + part[1][m][n]) +
+                         (part[2][m][n] + part[3][m][n]);
+        __syncthreads();
+        part[0][m][n] = y;
+        __syncthreads();
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+            s = fma(Tm[k][m], part[0][k][n], s);
+        Y[m][n] = s;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NT; i++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                z[i] = qr_mfma(h2[i][q], Y[4 * q + lk][lr], z[i]);
+        mfma_settle<qv4d, NT>(&z[0]);
+        // the next panel's Tm is written after the barriers above, its Y
+        // after three more
+    }
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+        const int t = wave + 4 * i;
+        if (t >= nb)
+            continue;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int c = 16 * t + 4 * q + lk;
+            if (ident)
+                V[bl.a_off + (uint64_t)(i0 + lr) * N + c] = z[i][q];
+            else
+                A1[bl.a_off + (uint64_t)c * N + i0 + lr] = z[i][q];
         }
     }
 }
@@ -633,6 +999,7 @@ struct Syev {
     uint64_t a_len = 0, q_len = 0, f_len = 0, w_len = 0;
     uint32_t max_nb = 2;
     double *A = nullptr, *V = nullptr, *Q = nullptr, *w = nullptr;
+    double *H = nullptr, *A1 = nullptr; // reflectors, preconditioned matrices
     int *qflag = nullptr;
     unsigned *nrot = nullptr, *h_nrot = nullptr; // device counter, pinned copy
     JacBlock *d_blk = nullptr;
@@ -642,6 +1009,7 @@ struct Syev {
     int sweeps = 0;
     ~Syev() {
         for (void *p : {(void *)A, (void *)V, (void *)Q, (void *)w,
+                        (void *)H, (void *)A1,
                         (void *)qflag, (void *)nrot, (void *)d_blk,
                         (void *)d_pair, (void *)d_upd, (void *)d_src_off,
                         (void *)d_w_off})
@@ -651,6 +1019,54 @@ struct Syev {
             hipHostFree(h_nrot);
     }
 };
+
+// A <- Q^T A Q, V <- Q of every matrix's QR factorisation (Q also holds the
+// panels' T, 256 elements per panel of the 512 per panel it has).
+static int qr_precondition(b2g_ctx ctx, Syev &s) {
+    hipStream_t st = ctx->stream;
+    const unsigned nm = (unsigned)s.blk.size();
+    int nb = 0;
+    for (const JacBlock &b : s.blk)
+        if (b.nb <= (uint32_t)kMaxQrBlocks)
+            nb = std::max(nb, (int)b.nb);
+    if (nb == 0) // nothing to precondition
+        return B2G_OK;
+    B2G_HIP(hipMalloc(&s.H, s.a_len * sizeof(double)));
+    B2G_HIP(hipMalloc(&s.A1, s.a_len * sizeof(double)));
+    for (int p = 0; p < nb; p++) {
+        const int rows = (nb - p) * kJB;
+#define B2G_PANEL(R_)                                                          \
+    hipLaunchKernelGGL(qr_panel_kernel<R_>, dim3(nm), dim3(64 * kQrWaves), 0,  \
+                       st, s.d_blk, s.A, s.H, s.Q, p)
+        if (rows <= 256)
+            B2G_PANEL(8);
+        else if (rows <= 640)
+            B2G_PANEL(20);
+        else
+            B2G_PANEL(36);
+#undef B2G_PANEL
+        if (p + 1 < nb)
+            hipLaunchKernelGGL(qr_update_kernel,
+                               dim3((unsigned)((rows - kJB + 31) / 32), nm),
+                               dim3(512), 0, st, s.d_blk, s.A, s.H, s.Q, p);
+        B2G_HIP(hipGetLastError());
+    }
+    const int top = (int)s.max_nb;
+#define B2G_APPLY(NT_, LO_, HI_)                                               \
+    if (top > (LO_))                                                           \
+    hipLaunchKernelGGL(qr_apply_kernel<NT_>,                                   \
+                       dim3((unsigned)std::min<int>(top, HI_), nm, 2),         \
+                       dim3(256), 0, st, s.d_blk, s.A, s.H, s.Q, s.A1, s.V,    \
+                       LO_, HI_)
+    B2G_APPLY(18, 40, 1 << 30);
+    B2G_APPLY(10, 24, 40);
+    B2G_APPLY(6, 8, 24);
+    B2G_APPLY(2, 0, 8);
+#undef B2G_APPLY
+    B2G_HIP(hipGetLastError());
+    std::swap(s.A, s.A1);
+    return B2G_OK;
+}
 
 // Eigen-decomposition of the compact symmetric matrices src + src_off[i]
 // (order n[i]): eigenvalues (ascending) into w_sorted (host, compact),
@@ -700,7 +1116,7 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
         for (uint32_t k = 0; k < h; k++)
             pairs.push_back(JacTask{(uint32_t)i, 0, k, 0});
         for (uint32_t a = 0; a < h; a++)
-            for (uint32_t b = 0; b < h; b++)
+            for (uint32_t b = a; b < h; b++)
                 upd.push_back(JacTask{(uint32_t)i, 1, a, b});
         for (uint32_t a = 0; a < h; a++)
             for (uint32_t rb = 0; rb < h; rb++) // slices of kJS rows
@@ -753,6 +1169,11 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
         B2G_HIP(hipGetLastError());
         B2G_HIP(hipStreamSynchronize(st));
     }
+    {
+        const int r = qr_precondition(ctx, s);
+        if (r != B2G_OK)
+            return r;
+    }
     const int max_sweeps = 60;
     const double tol = 2.220446049250313e-16;
     // cyclic sweeps per pair subproblem and round (B2G_JACOBI_INNER): the
@@ -764,25 +1185,36 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
             inner = atoi(e);
     int sweep = 0;
     for (; sweep < max_sweeps; sweep++) {
+        // anything left to rotate?
+        B2G_HIP(hipMemsetAsync(s.nrot, 0, sizeof(unsigned), st));
+        hipLaunchKernelGGL(jacobi_check_kernel, dim3(64, (unsigned)nm),
+                           dim3(256), 0, st, s.d_blk, s.A, tol, s.nrot);
+        B2G_HIP(hipGetLastError());
+        B2G_HIP(hipMemcpyAsync(s.h_nrot, s.nrot, sizeof(unsigned),
+                               hipMemcpyDeviceToHost, st));
+        B2G_HIP(hipStreamSynchronize(st));
+        if (*s.h_nrot == 0)
+            break;
+        const bool trace = getenv("B2G_JACOBI_TRACE") != nullptr;
         B2G_HIP(hipMemsetAsync(s.nrot, 0, sizeof(unsigned), st));
         for (uint32_t r = 0; r + 1 < s.max_nb; r++) {
             hipLaunchKernelGGL(jacobi_pair_kernel, dim3((unsigned)s.n_pair),
                                dim3(256), 0, st, s.d_blk, s.d_pair, s.A, s.Q,
-                               s.qflag, (int)r, tol, inner, s.nrot);
+                               s.qflag, (int)r, tol, r > 0 ? 1 : 0, inner,
+                               s.nrot);
             B2G_HIP(hipGetLastError());
             hipLaunchKernelGGL(jacobi_update_kernel, dim3((unsigned)s.n_upd),
                                dim3(256), 0, st, s.d_blk, s.d_upd, s.A,
                                s.V, s.Q, s.qflag, (int)r);
             B2G_HIP(hipGetLastError());
         }
-        B2G_HIP(hipMemcpyAsync(s.h_nrot, s.nrot, sizeof(unsigned),
-                               hipMemcpyDeviceToHost, st));
-        B2G_HIP(hipStreamSynchronize(st));
-        if (getenv("B2G_JACOBI_TRACE") != nullptr)
+        if (trace) {
+            B2G_HIP(hipMemcpyAsync(s.h_nrot, s.nrot, sizeof(unsigned),
+                                   hipMemcpyDeviceToHost, st));
+            B2G_HIP(hipStreamSynchronize(st));
             fprintf(stderr, "b2g jacobi sweep %d: %u rotating pair subproblems\n",
                     sweep, *s.h_nrot);
-        if (*s.h_nrot == 0)
-            break;
+        }
     }
     if (sweeps)
         *sweeps = sweep + 1;

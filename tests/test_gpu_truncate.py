@@ -97,6 +97,39 @@ def test_syev_batched_matches_numpy(gpu_ctx):
                 assert np.abs(v[j] - vo[j]).max() < 1e-9, (name, j)
 
 
+@pytest.mark.parametrize("sizes", [
+    (1, 2, 15, 16, 17), (31, 32, 33, 128, 129), (255, 257, 20),
+    (385, 400, 3), (641, 64, 1), (1152, 1153)])
+def test_syev_batched_orders(gpu_ctx, sizes):
+    # orders around the panels (16 columns), the register sizes of the QR
+    # step (256, 640 and 1152 rows; 8, 24 and 40 column tiles) and past the
+    # largest it takes; graded, rank-deficient, indefinite and zero matrices.
+    # Backward error of either method a small multiple of n eps ||A||, n eps
+    # = 2.6e-13 at n = 1153: 1e-12 on the eigenvalues (Rayleigh quotients),
+    # 1e-11 on residual and orthogonality
+    rng = np.random.default_rng(sum(sizes))
+    mats = []
+    for i, n in enumerate(sizes):
+        q = np.linalg.qr(rng.standard_normal((n, n)))[0]
+        w = 10.0 ** (-14.0 * np.arange(n) / n)
+        if i % 3 == 1:
+            w[n // 2:] = 0.0
+        elif i % 3 == 2:
+            w *= np.where(np.arange(n) % 2, -1.0, 1.0)
+        a = (q * w) @ q.T
+        mats.append((a + a.T) / 2)
+    mats.append(np.zeros((5, 5)))
+    print("orders", sizes, flush=True)
+    ws, vs, sweeps = TR.eigh_batched(gpu_ctx, [dev(m) for m in mats])
+    for a, w, v in zip(mats, ws, vs):
+        w, v = w.cpu().numpy(), v.cpu().numpy()
+        wn = np.linalg.eigvalsh(a)
+        nrm = max(np.abs(wn).max(), 1e-300)
+        assert np.abs(w - wn).max() <= 1e-12 * nrm, len(w)
+        assert np.abs(a @ v.T - v.T * w).max() <= 1e-11 * nrm, len(w)
+        assert np.abs(v @ v.T - np.eye(len(w))).max() < 1e-11, len(w)
+
+
 def test_syev_batched_repeatable(gpu_ctx):
     mats = [dev(m) for _, m in sym_mats()]
     w1, v1, _ = TR.eigh_batched(gpu_ctx, mats)
