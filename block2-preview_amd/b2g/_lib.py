@@ -172,6 +172,7 @@ _SIGS = {
     "b2g_ctx_create": (C.c_int, [C.c_int, C.c_uint, C.POINTER(_vp)]),
     "b2g_ctx_destroy": (C.c_int, [_vp]),
     "b2g_ctx_synchronize": (C.c_int, [_vp]),
+    "b2g_ctx_trim": (C.c_int, [_vp]),
     "b2g_ctx_stream": (_vp, [_vp]),
     "b2g_plan_set_timing": (C.c_int, [_vp, C.c_int]),
     "b2g_plan_timing": (C.c_int, [_vp, f64p, u64p]),

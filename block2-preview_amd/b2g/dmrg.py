@@ -913,12 +913,13 @@ class DMRG:
         """Under device-memory pressure (less than 45 % of the device free:
         one step of an n=40, M=3000 ab initio sweep allocates about 100 GB)
         drops the plans kept across sweeps (rebuilt on demand) and hands
-        torch's cached blocks back to the device, so that library
-        allocations can use them."""
+        the context's and torch's kept blocks back to the device, so that
+        either can use them."""
         free, total = torch.cuda.mem_get_info(self.dev)
         if free >= 0.45 * total:
             return
         self.close()
+        L.check(self.lib.b2g_ctx_trim(self.ctx.h))
         torch.cuda.empty_cache()
 
     def update_two_dot(self, i, forward, bond_dim, noise, conv):

@@ -44,17 +44,17 @@ struct DavCache {
                     e = nullptr;
                 }
     }
+    b2g_ctx ctx = nullptr;
     void release() {
         drop_graphs();
-        for (double **p : {&B, &S, &q, &t, &qn, &sn, &partial})
-            if (*p) {
-                hipFree(*p);
-                *p = nullptr;
-            }
-        if (dst)
-            hipFree(dst);
-        if (hdr)
-            hipHostFree(hdr);
+        if (ctx == nullptr)
+            return;
+        for (double **p : {&B, &S, &q, &t, &qn, &sn, &partial}) {
+            ctx->pool.put(*p);
+            *p = nullptr;
+        }
+        ctx->pool.put(dst);
+        ctx->pinned.put(hdr);
         dst = hdr = nullptr;
         n = nv = 0;
     }
@@ -445,7 +445,7 @@ extern "C" int b2g_effham_create(b2g_ctx ctx, const b2g_problem *pb,
     tm.mark("plan upload");
     if (r == B2G_OK) {
         const size_t dl = std::max<uint64_t>(p.ket.total(), 1);
-        if (hipMalloc(&h->diag, dl * sizeof(double)) != hipSuccess) {
+        if (ctx->alloc(&h->diag, dl * sizeof(double)) != hipSuccess) {
             set_error("diagonal allocation failed");
             r = B2G_ERR_MEMORY;
         } else
@@ -470,7 +470,7 @@ extern "C" int b2g_effham_destroy(b2g_effham h) {
     b2g_buf_destroy(h->lbuf);
     b2g_buf_destroy(h->rbuf);
     if (h->diag)
-        hipFree(h->diag);
+        h->ctx->pool.put(h->diag);
     delete h;
     return B2G_OK;
 }
@@ -590,6 +590,7 @@ extern "C" int b2g_effham_data(b2g_effham h, double **left, size_t *left_len,
     B2G_REQUIRE(h && left && left_len && right && right_len, B2G_ERR_ARG,
                 "NULL arg");
     B2G_REQUIRE(h->plan, B2G_ERR_STATE, "effham was built host-only");
+    h->lbuf->shown = h->rbuf->shown = true;
     *left = (double *)h->lbuf->ptr;
     *left_len = h->lbuf->n;
     *right = (double *)h->rbuf->ptr;
@@ -629,19 +630,11 @@ struct DavWork {
     double *B = nullptr, *S = nullptr, *q = nullptr, *t = nullptr;
     double *O = nullptr;    // orthogonal states
     double *scal = nullptr; // device scalars (>= 64*64 + 16)
+    b2g_ctx ctx;
+    explicit DavWork(b2g_ctx c) : ctx(c) {}
     ~DavWork() {
-        if (O)
-            hipFree(O);
-        if (B)
-            hipFree(B);
-        if (S)
-            hipFree(S);
-        if (q)
-            hipFree(q);
-        if (t)
-            hipFree(t);
-        if (scal)
-            hipFree(scal);
+        for (double *p : {O, B, S, q, t, scal})
+            ctx->pool.put(p);
     }
 };
 
@@ -748,14 +741,14 @@ static int davidson(b2g_effham h, double *x, int k, const DavOpts &o,
         nwg = nor, nor = 0;
     const int nv = std::max(nor, nwg);
     const double rel2 = o.rel * o.rel;
-    DavWork w;
-    B2G_HIP(hipMalloc(&w.B, (size_t)def_max * n * sizeof(double)));
-    B2G_HIP(hipMalloc(&w.S, (size_t)def_max * n * sizeof(double)));
-    B2G_HIP(hipMalloc(&w.q, n * sizeof(double)));
-    B2G_HIP(hipMalloc(&w.t, n * sizeof(double)));
-    B2G_HIP(hipMalloc(&w.scal, (64 * 64 + 64) * sizeof(double)));
+    DavWork w(ctx);
+    B2G_HIP(ctx->alloc(&w.B, (size_t)def_max * n * sizeof(double)));
+    B2G_HIP(ctx->alloc(&w.S, (size_t)def_max * n * sizeof(double)));
+    B2G_HIP(ctx->alloc(&w.q, n * sizeof(double)));
+    B2G_HIP(ctx->alloc(&w.t, n * sizeof(double)));
+    B2G_HIP(ctx->alloc(&w.scal, (64 * 64 + 64) * sizeof(double)));
     if (nv)
-        B2G_HIP(hipMalloc(&w.O, (size_t)nv * n * sizeof(double)));
+        B2G_HIP(ctx->alloc(&w.O, (size_t)nv * n * sizeof(double)));
     double *Bv = w.B, *Sv = w.S;
     auto bv = [&](int i) { return Bv + (size_t)i * n; };
     auto sv = [&](int i) { return Sv + (size_t)i * n; };
@@ -919,9 +912,8 @@ static int davidson(b2g_effham h, double *x, int k, const DavOpts &o,
                 // keep the targeted Ritz pairs first (:1105-1133): vector j
                 // of B and S becomes the one of idx[j], through a buffer
                 double *T = nullptr;
-                B2G_HIP(hipMalloc(&T, (size_t)m * n * sizeof(double)));
-                std::unique_ptr<double, int (*)(void *)> tg(
-                    T, [](void *p) { return (int)hipFree(p); });
+                B2G_HIP(ctx->alloc(&T, (size_t)m * n * sizeof(double)));
+                PoolGuard tg(ctx, T);
                 for (double *X : {Bv, Sv}) {
                     for (int j = 0; j < m; j++)
                         B2G_HIP(launch_copy(X + (size_t)idx[j] * n,
@@ -991,21 +983,22 @@ static int davidson_graph(b2g_effham h, double *x, int k, const DavOpts &o,
     if (c.n != n || c.nv != nv) {
         B2G_HIP(hipStreamSynchronize(st));
         c.release();
+        c.ctx = ctx;
         auto fail = [&c](hipError_t e) {
             if (e != hipSuccess)
                 c.release();
             return e;
         };
-        B2G_HIP(fail(hipMalloc(&c.B, nv * n * sizeof(double))));
-        B2G_HIP(fail(hipMalloc(&c.S, nv * n * sizeof(double))));
-        B2G_HIP(fail(hipMalloc(&c.q, n * sizeof(double))));
-        B2G_HIP(fail(hipMalloc(&c.t, n * sizeof(double))));
-        B2G_HIP(fail(hipMalloc(&c.qn, n * sizeof(double))));
-        B2G_HIP(fail(hipMalloc(&c.sn, n * sizeof(double))));
-        B2G_HIP(fail(hipMalloc(&c.partial,
+        B2G_HIP(fail(ctx->alloc(&c.B, nv * n * sizeof(double))));
+        B2G_HIP(fail(ctx->alloc(&c.S, nv * n * sizeof(double))));
+        B2G_HIP(fail(ctx->alloc(&c.q, n * sizeof(double))));
+        B2G_HIP(fail(ctx->alloc(&c.t, n * sizeof(double))));
+        B2G_HIP(fail(ctx->alloc(&c.qn, n * sizeof(double))));
+        B2G_HIP(fail(ctx->alloc(&c.sn, n * sizeof(double))));
+        B2G_HIP(fail(ctx->alloc(&c.partial,
                                davidson_partial_len() * sizeof(double))));
-        B2G_HIP(fail(hipMalloc(&c.dst, sizeof(DavState))));
-        B2G_HIP(fail(hipHostMalloc(&c.hdr, sizeof(DavState))));
+        B2G_HIP(fail(ctx->alloc(&c.dst, sizeof(DavState))));
+        B2G_HIP(fail(ctx->pinned.get(sizeof(DavState), (void **)&c.hdr)));
         c.n = n;
         c.nv = nv;
         tm.mark("workspace");
@@ -1152,15 +1145,12 @@ static int exact_diag(b2g_effham h, double *x, int k, const DavOpts &o,
     B2G_REQUIRE(h->kernel == nullptr, B2G_ERR_STATE,
                 "exact diagonalisation with a matvec hook is not supported");
     double *E = nullptr, *Hm = nullptr, *w = nullptr;
-    B2G_HIP(hipMalloc(&Hm, n * n * sizeof(double)));
-    std::unique_ptr<double, int (*)(void *)> g1(
-        Hm, [](void *p) { return (int)hipFree(p); });
-    B2G_HIP(hipMalloc(&E, n * n * sizeof(double)));
-    std::unique_ptr<double, int (*)(void *)> g2(
-        E, [](void *p) { return (int)hipFree(p); });
-    B2G_HIP(hipMalloc(&w, n * sizeof(double)));
-    std::unique_ptr<double, int (*)(void *)> g3(
-        w, [](void *p) { return (int)hipFree(p); });
+    B2G_HIP(ctx->alloc(&Hm, n * n * sizeof(double)));
+    PoolGuard g1(ctx, Hm);
+    B2G_HIP(ctx->alloc(&E, n * n * sizeof(double)));
+    PoolGuard g2(ctx, E);
+    B2G_HIP(ctx->alloc(&w, n * sizeof(double)));
+    PoolGuard g3(ctx, w);
     // rows of the identity, 64 at a time (staged in E), their products as
     // rows of Hm (H is symmetric: row i of Hm = (H e_i)^T = column i)
     const size_t batch = 64;

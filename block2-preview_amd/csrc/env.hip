@@ -202,7 +202,6 @@ struct b2g_winplan_s {
     bool host_only = false;
     bool b_is_one = false; // B is the plan's own 1.0 (transforms, swaps)
     void *dev = nullptr;
-    size_t dev_len = 0; // bytes of the block (from the context's pool)
     b2g::WinGroup *d_groups = nullptr;
     b2g::WinRec *d_recs = nullptr;
     b2g::WinChunk *d_chunks = nullptr;
@@ -211,42 +210,6 @@ struct b2g_winplan_s {
 };
 
 namespace b2g {
-
-// A device block of at least `bytes` from the context's pool of released
-// window-plan blocks (smallest that fits), else a new allocation.
-static int win_block(b2g_ctx ctx, size_t bytes, void **out, size_t *len) {
-    auto &pool = ctx->win_pool;
-    size_t best = pool.size();
-    for (size_t i = 0; i < pool.size(); i++)
-        if (pool[i].first >= bytes &&
-            (best == pool.size() || pool[i].first < pool[best].first))
-            best = i;
-    if (best != pool.size()) {
-        *len = pool[best].first;
-        *out = pool[best].second;
-        pool.erase(pool.begin() + best);
-        return B2G_OK;
-    }
-    const size_t mib = (size_t)1 << 20;
-    const size_t n = (bytes + mib - 1) / mib * mib;
-    hipError_t e = hipMalloc(out, n);
-    if (e != hipSuccess && !pool.empty()) {
-        // none of the released blocks fits: give them back and retry
-        (void)hipGetLastError();
-        for (auto &b : pool)
-            hipFree(b.second);
-        pool.clear();
-        e = hipMalloc(out, n);
-    }
-    B2G_HIP(e);
-    *len = n;
-    return B2G_OK;
-}
-
-// bytes of released window-plan blocks a context keeps for reuse; beyond
-// it the smallest are freed (a sweep whose bond dimension grows releases
-// plans smaller than every later request)
-constexpr size_t kWinPoolCap = (size_t)8 << 30;
 
 static int winplan_finish(b2g_winplan w,
                           WinItems &items) {
@@ -272,11 +235,7 @@ static int winplan_finish(b2g_winplan w,
     const size_t bytes = ng * sizeof(WinGroup) + nr * sizeof(WinRec) +
                          nc * sizeof(WinChunk) + 64;
     B2G_HIP(hipSetDevice(w->ctx->device));
-    {
-        const int r = win_block(w->ctx, bytes, &w->dev, &w->dev_len);
-        if (r != B2G_OK)
-            return r;
-    }
+    B2G_HIP(w->ctx->alloc(&w->dev, bytes));
     char *p = (char *)w->dev;
     w->d_one = (double *)p;
     w->d_groups = (WinGroup *)(p + 64);
@@ -942,17 +901,7 @@ extern "C" int b2g_winplan_destroy(b2g_winplan w) {
         // the plan's launches are done before its block serves another
         hipSetDevice(w->ctx->device);
         hipStreamSynchronize(w->ctx->stream);
-        auto &pool = w->ctx->win_pool;
-        pool.emplace_back(w->dev_len, w->dev);
-        size_t total = 0;
-        for (const auto &b : pool)
-            total += b.first;
-        while (total > kWinPoolCap) {
-            auto it = std::min_element(pool.begin(), pool.end());
-            total -= it->first;
-            hipFree(it->second);
-            pool.erase(it);
-        }
+        w->ctx->pool.put(w->dev);
     }
     delete w;
     return B2G_OK;
@@ -1109,7 +1058,7 @@ extern "C" int b2g_contract_wfn_plan(b2g_ctx ctx, int symmetry,
         bytes += g->tasks[c].size() * sizeof(Task);
     if (bytes) {
         B2G_HIP(hipSetDevice(ctx->device));
-        B2G_HIP(hipMalloc(&g->dev, bytes));
+        B2G_HIP(ctx->alloc(&g->dev, bytes));
         std::vector<char> host(bytes);
         size_t off = 0;
         for (int c = 0; c < kTileConfigs; c++) {
@@ -1164,7 +1113,7 @@ extern "C" int b2g_gemmlist_destroy(b2g_gemmlist g) {
     if (g->dev) {
         hipSetDevice(g->ctx->device);
         hipStreamSynchronize(g->ctx->stream);
-        hipFree(g->dev);
+        g->ctx->pool.put(g->dev);
     }
     delete g;
     return B2G_OK;

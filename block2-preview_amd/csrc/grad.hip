@@ -50,13 +50,11 @@ struct GradPlan {
     double flops = 0; // algorithmic FLOPs per right-hand side
 };
 
-void grad_plan_destroy(GradPlan *g) {
+void grad_plan_destroy(b2g_ctx ctx, GradPlan *g) {
     if (g == nullptr)
         return;
-    if (g->dev)
-        hipFree(g->dev);
-    if (g->scratch)
-        hipFree(g->scratch);
+    ctx->pool.put(g->dev);
+    ctx->pool.put(g->scratch);
     delete g;
 }
 
@@ -266,15 +264,15 @@ static int grad_plan_build(b2g_plan p, GradPlan **out) {
         offs.push_back(off);
         off += (L.s.size() * sizeof(Seg) + 255) & ~size_t(255);
     });
-    hipError_t e = hipMalloc(&g->dev, std::max<size_t>(bytes, 1));
+    hipError_t e = p->ctx->alloc(&g->dev, std::max<size_t>(bytes, 1));
     if (e == hipSuccess)
         e = hipMemcpy(g->dev, host.data(), std::max<size_t>(bytes, 1),
                       hipMemcpyHostToDevice);
     if (e == hipSuccess)
-        e = hipMalloc(&g->scratch,
-                      std::max<uint64_t>(g->s_max, 1) * sizeof(double));
+        e = p->ctx->alloc(&g->scratch,
+                          std::max<uint64_t>(g->s_max, 1) * sizeof(double));
     if (e != hipSuccess) {
-        grad_plan_destroy(g);
+        grad_plan_destroy(p->ctx, g);
         set_error(std::string("gradient plan upload: ") + hipGetErrorString(e));
         return B2G_ERR_MEMORY;
     }

@@ -105,15 +105,11 @@ struct HostChunk {
 
 } // namespace
 
-void pk_destroy(PkPlan *k) {
+void pk_destroy(b2g_ctx ctx, PkPlan *k) {
     if (k == nullptr)
         return;
-    if (k->dev)
-        hipFree(k->dev);
-    if (k->op)
-        hipFree(k->op);
-    if (k->scratch)
-        hipFree(k->scratch);
+    for (void *q : {k->dev, (void *)k->op, (void *)k->scratch})
+        ctx->pool.put(q);
     delete k;
 }
 
@@ -305,7 +301,7 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
     const int rs = ctx_stage(p->ctx, bytes + 16, &host);
     if (rs != B2G_OK)
         return rs;
-    B2G_HIP(hipMalloc(&k->dev, bytes + 16));
+    B2G_HIP(p->ctx->alloc(&k->dev, bytes + 16));
     size_t off = 0;
     auto put = [&](const void *src, size_t nb) {
         const size_t o = off;
@@ -326,8 +322,9 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
     if (mat_bytes)
         B2G_HIP(hipMemcpyAsync(k->dev, host, mat_bytes, hipMemcpyHostToDevice,
                                p->ctx->stream));
-    B2G_HIP(hipMalloc(&k->op, std::max<uint64_t>(2 * (k->l_len + k->r_len), 8) *
-                                  sizeof(uint16_t)));
+    B2G_HIP(p->ctx->alloc(&k->op,
+                          std::max<uint64_t>(2 * (k->l_len + k->r_len), 8) *
+                              sizeof(uint16_t)));
     tm.mark("pack lists uploaded, planes allocated");
     {
         const int r = pk_pack_ops(p, k);
@@ -413,7 +410,7 @@ int pk_build(b2g_plan p) {
     const int r = pk_build_into(p, k);
     if (r != B2G_OK) {
         hipStreamSynchronize(p->ctx->stream);
-        pk_destroy(k);
+        pk_destroy(p->ctx, k);
         return r;
     }
     p->pk = k;
@@ -427,12 +424,12 @@ int pk_reserve(b2g_plan p, int n_rhs) {
         return B2G_OK;
     if (k->scratch) {
         B2G_HIP(hipStreamSynchronize(p->ctx->stream));
-        B2G_HIP(hipFree(k->scratch));
+        p->ctx->pool.put(k->scratch);
         k->scratch = nullptr;
         k->scratch_rhs = 0;
     }
     const size_t n = std::max<uint64_t>(2 * (k->x_len + k->w_max), 8) * n_rhs;
-    B2G_HIP(hipMalloc(&k->scratch, n * sizeof(uint16_t)));
+    B2G_HIP(p->ctx->alloc(&k->scratch, n * sizeof(uint16_t)));
     k->scratch_rhs = n_rhs;
     p->scratch_gen++;
     return B2G_OK;

@@ -10,9 +10,9 @@
 namespace b2g {
 
 struct GradPlan; // grad.hip
-void grad_plan_destroy(GradPlan *g);
+void grad_plan_destroy(b2g_ctx ctx, GradPlan *g);
 struct PkPlan; // pkplan.hip
-void pk_destroy(PkPlan *k);
+void pk_destroy(b2g_ctx ctx, PkPlan *k);
 
 // one phase-2 output block (or window) and its segments [sb, se)
 struct BlockJob {

@@ -66,6 +66,88 @@ static int scratch_setup(int device) {
     return B2G_OK;
 }
 
+// ------------------------------------------------------------- block pool
+constexpr size_t kPoolCap = (size_t)16 << 30;
+
+hipError_t BlockPool::make(size_t bytes, void **out) {
+    return pinned_ ? hipHostMalloc(out, bytes) : hipMalloc(out, bytes);
+}
+void BlockPool::drop(void *p) {
+    if (pinned_)
+        (void)hipHostFree(p);
+    else
+        (void)hipFree(p);
+}
+
+hipError_t BlockPool::get(size_t bytes, void **out) {
+    *out = nullptr;
+    // whole 4 KiB or 2 MiB, so that nearly equal requests share blocks
+    const size_t unit = bytes <= ((size_t)1 << 20) ? 4096 : (size_t)2 << 20;
+    const size_t n = (std::max<size_t>(bytes, 1) + unit - 1) / unit * unit;
+    std::lock_guard<std::mutex> lock(m_);
+    size_t best = free_.size();
+    for (size_t i = 0; i < free_.size(); i++)
+        if (free_[i].first >= n && free_[i].first <= n + n / 4 + unit &&
+            (best == free_.size() || free_[i].first < free_[best].first))
+            best = i;
+    size_t len = n;
+    if (best != free_.size()) {
+        len = free_[best].first;
+        *out = free_[best].second;
+        kept_ -= len;
+        free_.erase(free_.begin() + best);
+    } else {
+        hipError_t e = make(n, out);
+        if (e != hipSuccess && !free_.empty()) {
+            (void)hipGetLastError();
+            for (auto &b : free_)
+                drop(b.second);
+            free_.clear();
+            kept_ = 0;
+            e = make(n, out);
+        }
+        if (e != hipSuccess) {
+            *out = nullptr;
+            return e;
+        }
+    }
+    size_[*out] = len;
+    return hipSuccess;
+}
+
+void BlockPool::put(void *p) {
+    if (p == nullptr)
+        return;
+    std::lock_guard<std::mutex> lock(m_);
+    auto it = size_.find(p);
+    if (it == size_.end())
+        return;
+    const size_t n = it->second;
+    size_.erase(it);
+    free_.emplace_back(n, p);
+    kept_ += n;
+    size_t cap = kPoolCap;
+    if (!pinned_ && n >= ((size_t)64 << 20)) {
+        size_t avail = 0, total = 0;
+        if (hipMemGetInfo(&avail, &total) == hipSuccess && avail < total / 4)
+            cap = 0;
+    }
+    size_t i = 0;
+    for (; i < free_.size() && kept_ > cap; i++) {
+        kept_ -= free_[i].first;
+        drop(free_[i].second);
+    }
+    free_.erase(free_.begin(), free_.begin() + i);
+}
+
+void BlockPool::trim() {
+    std::lock_guard<std::mutex> lock(m_);
+    for (auto &b : free_)
+        drop(b.second);
+    free_.clear();
+    kept_ = 0;
+}
+
 static void *scratch_ptr(int device) {
     std::lock_guard<std::mutex> lock(g_scratch_mu);
     return device >= 0 && device < kMaxDevices ? g_scratch_ptr[device]
@@ -188,10 +270,17 @@ extern "C" int b2g_ctx_destroy(b2g_ctx ctx) {
     hipHostFree(ctx->red_host);
     if (ctx->stage)
         hipHostFree(ctx->stage);
-    for (auto &b : ctx->win_pool)
-        hipFree(b.second);
     hipStreamDestroy(ctx->stream);
     delete ctx;
+    return B2G_OK;
+}
+
+extern "C" int b2g_ctx_trim(b2g_ctx ctx) {
+    B2G_REQUIRE(ctx != nullptr, B2G_ERR_ARG, "ctx is NULL");
+    B2G_HIP(hipSetDevice(ctx->device));
+    B2G_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->pool.trim();
+    ctx->pinned.trim();
     return B2G_OK;
 }
 
@@ -224,7 +313,7 @@ extern "C" int b2g_buf_create(b2g_ctx ctx, size_t n, int dtype, b2g_buf *out) {
     b->ctx = ctx;
     b->n = n;
     b->dtype = dtype;
-    if (n != 0 && hipMalloc(&b->ptr, n * dtype_size(dtype)) != hipSuccess) {
+    if (n != 0 && ctx->alloc(&b->ptr, n * dtype_size(dtype)) != hipSuccess) {
         delete b;
         set_error("b2g_buf_create: hipMalloc failed");
         return B2G_ERR_MEMORY;
@@ -237,9 +326,12 @@ extern "C" int b2g_buf_destroy(b2g_buf buf) {
     if (buf == nullptr)
         return B2G_OK;
     hipSetDevice(buf->ctx->device);
-    hipStreamSynchronize(buf->ctx->stream);
+    if (buf->shown) // the caller may have used it on streams of its own
+        hipDeviceSynchronize();
+    else
+        hipStreamSynchronize(buf->ctx->stream);
     if (buf->ptr && buf->owned)
-        hipFree(buf->ptr);
+        buf->ctx->pool.put(buf->ptr);
     delete buf;
     return B2G_OK;
 }
@@ -300,6 +392,8 @@ extern "C" int b2g_upload_blocks(b2g_ctx ctx, const void *host, size_t n,
 }
 
 extern "C" void *b2g_buf_device_ptr(b2g_buf buf) {
+    if (buf)
+        buf->shown = true;
     return buf ? buf->ptr : nullptr;
 }
 extern "C" size_t b2g_buf_size(b2g_buf buf) { return buf ? buf->n : 0; }
@@ -904,7 +998,7 @@ static int upload_chunks(b2g_plan p) {
     const int rs = ctx_stage(p->ctx, bytes + 16, &host);
     if (rs != B2G_OK)
         return rs;
-    B2G_HIP(hipMalloc(&p->dev, bytes + 16));
+    B2G_HIP(p->ctx->alloc(&p->dev, bytes + 16));
     size_t off = 0;
     auto put = [&](const void *src, size_t nb) -> size_t {
         size_t o = off;
@@ -1223,9 +1317,9 @@ extern "C" int b2g_upload_plan(b2g_ctx ctx, b2g_buf lbuf, b2g_buf rbuf,
     if (r == B2G_OK)
         p->pairs.assign(pairs, pairs + n_pairs);
     if (r == B2G_OK && (flags & 3)) {
-        if (hipMalloc(&p->l32, std::max<size_t>(lbuf->n, 1) * 4) !=
+        if (ctx->alloc(&p->l32, std::max<size_t>(lbuf->n, 1) * 4) !=
                 hipSuccess ||
-            hipMalloc(&p->r32, std::max<size_t>(rbuf->n, 1) * 4) !=
+            ctx->alloc(&p->r32, std::max<size_t>(rbuf->n, 1) * 4) !=
                 hipSuccess) {
             set_error("b2g_upload_plan: FP32 shadow allocation failed");
             r = B2G_ERR_MEMORY;
@@ -1267,18 +1361,10 @@ extern "C" int b2g_plan_destroy(b2g_plan p) {
         hipEventDestroy(st.start);
         hipEventDestroy(st.stop);
     }
-    if (p->dev)
-        hipFree(p->dev);
-    if (p->l32)
-        hipFree(p->l32);
-    if (p->r32)
-        hipFree(p->r32);
-    if (p->w)
-        hipFree(p->w);
-    if (p->pbuf)
-        hipFree(p->pbuf);
-    grad_plan_destroy(p->grad);
-    pk_destroy(p->pk);
+    for (void *q : {p->dev, (void *)p->l32, (void *)p->r32, p->w, p->pbuf})
+        p->ctx->pool.put(q);
+    grad_plan_destroy(p->ctx, p->grad);
+    pk_destroy(p->ctx, p->pk);
     delete p;
     return B2G_OK;
 }
@@ -1418,11 +1504,11 @@ int plan_reserve(b2g_plan p, int n_rhs, int precision) {
     } else if (need > p->w_bytes) {
         if (p->w) {
             B2G_HIP(hipStreamSynchronize(ctx->stream));
-            B2G_HIP(hipFree(p->w));
+            ctx->pool.put(p->w);
             p->w = nullptr;
             p->w_bytes = 0;
         }
-        B2G_HIP(hipMalloc(&p->w, need));
+        B2G_HIP(ctx->alloc(&p->w, need));
         p->w_bytes = need;
         p->scratch_gen++;
     }
@@ -1432,11 +1518,11 @@ int plan_reserve(b2g_plan p, int n_rhs, int precision) {
     if (pneed > p->p_bytes) {
         if (p->pbuf) {
             B2G_HIP(hipStreamSynchronize(ctx->stream));
-            B2G_HIP(hipFree(p->pbuf));
+            ctx->pool.put(p->pbuf);
             p->pbuf = nullptr;
             p->p_bytes = 0;
         }
-        B2G_HIP(hipMalloc(&p->pbuf, pneed));
+        B2G_HIP(ctx->alloc(&p->pbuf, pneed));
         p->p_bytes = pneed;
         p->scratch_gen++;
     }
@@ -1795,7 +1881,8 @@ extern "C" int b2g_diag(b2g_ctx ctx, b2g_buf lbuf, b2g_buf rbuf,
     const size_t nb1 = blocks.size() * sizeof(DiagBlock),
                  nb2 = dterms.size() * sizeof(DiagTermDev);
     char *dev = nullptr;
-    B2G_HIP(hipMalloc(&dev, nb1 + nb2 + 16));
+    B2G_HIP(ctx->alloc(&dev, nb1 + nb2 + 16));
+    PoolGuard guard(ctx, dev);
     if (nb1)
         B2G_HIP(hipMemcpyAsync(dev, blocks.data(), nb1, hipMemcpyHostToDevice,
                                ctx->stream));
@@ -1809,7 +1896,6 @@ extern "C" int b2g_diag(b2g_ctx ctx, b2g_buf lbuf, b2g_buf rbuf,
                         (const DiagTermDev *)(dev + nb1), ctx->num_cu * 4,
                         ctx->stream);
     hipError_t e2 = hipStreamSynchronize(ctx->stream);
-    hipFree(dev);
     B2G_HIP(e);
     B2G_HIP(e2);
     return B2G_OK;

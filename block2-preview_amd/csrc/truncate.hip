@@ -946,14 +946,16 @@ __global__ __launch_bounds__(256) void dm_noise_kernel(
 struct TaskSet {
     std::vector<Task> t[kTileConfigs];
     std::vector<Seg> s;
+    b2g_ctx ctx = nullptr; // of dev
     void *dev = nullptr;
     Task *d_t[kTileConfigs] = {};
     Seg *d_s = nullptr;
     ~TaskSet() {
         if (dev)
-            hipFree(dev);
+            ctx->pool.put(dev);
     }
-    int upload(b2g_ctx ctx) {
+    int upload(b2g_ctx c) {
+        ctx = c;
         for (int c = 0; c < kTileConfigs; c++)
             sort_tasks(t[c], s);
         size_t bytes = s.size() * sizeof(Seg);
@@ -963,7 +965,7 @@ struct TaskSet {
         int r = ctx_stage(ctx, bytes + 16, &host);
         if (r != B2G_OK)
             return r;
-        B2G_HIP(hipMalloc(&dev, bytes + 16));
+        B2G_HIP(ctx->alloc(&dev, bytes + 16));
         size_t off = 0;
         auto put = [&](const void *src, size_t nb) {
             if (nb)
@@ -1007,16 +1009,15 @@ struct Syev {
     uint64_t *d_src_off = nullptr, *d_w_off = nullptr;
     size_t n_pair = 0, n_upd = 0;
     int sweeps = 0;
+    b2g_ctx ctx;
+    explicit Syev(b2g_ctx c) : ctx(c) {}
     ~Syev() {
         for (void *p : {(void *)A, (void *)V, (void *)Q, (void *)w,
-                        (void *)H, (void *)A1,
-                        (void *)qflag, (void *)nrot, (void *)d_blk,
-                        (void *)d_pair, (void *)d_upd, (void *)d_src_off,
-                        (void *)d_w_off})
-            if (p)
-                hipFree(p);
-        if (h_nrot)
-            hipHostFree(h_nrot);
+                        (void *)H, (void *)A1, (void *)qflag, (void *)nrot,
+                        (void *)d_blk, (void *)d_pair, (void *)d_upd,
+                        (void *)d_src_off, (void *)d_w_off})
+            ctx->pool.put(p);
+        ctx->pinned.put(h_nrot);
     }
 };
 
@@ -1031,8 +1032,8 @@ static int qr_precondition(b2g_ctx ctx, Syev &s) {
             nb = std::max(nb, (int)b.nb);
     if (nb == 0) // nothing to precondition
         return B2G_OK;
-    B2G_HIP(hipMalloc(&s.H, s.a_len * sizeof(double)));
-    B2G_HIP(hipMalloc(&s.A1, s.a_len * sizeof(double)));
+    B2G_HIP(ctx->alloc(&s.H, s.a_len * sizeof(double)));
+    B2G_HIP(ctx->alloc(&s.A1, s.a_len * sizeof(double)));
     for (int p = 0; p < nb; p++) {
         const int rows = (nb - p) * kJB;
 #define B2G_PANEL(R_)                                                          \
@@ -1075,7 +1076,7 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
                     const std::vector<uint64_t> &src_off, const double *src,
                     double *E, std::vector<double> &w_sorted, int *sweeps) {
     hipStream_t st = ctx->stream;
-    Syev s;
+    Syev s(ctx);
     const size_t nm = n.size();
     s.w_off.resize(nm + 1, 0);
     for (size_t i = 0; i < nm; i++) {
@@ -1126,18 +1127,18 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
     s.n_upd = upd.size();
     B2G_REQUIRE(s.n_pair < (1u << 31) && s.n_upd < (1u << 31), B2G_ERR_ARG,
                 "eigensolver: too many blocks");
-    B2G_HIP(hipMalloc(&s.A, s.a_len * sizeof(double)));
-    B2G_HIP(hipMalloc(&s.V, s.a_len * sizeof(double)));
-    B2G_HIP(hipMalloc(&s.Q, s.q_len * sizeof(double)));
-    B2G_HIP(hipMalloc(&s.w, std::max<uint64_t>(s.w_len, 1) * sizeof(double)));
-    B2G_HIP(hipMalloc(&s.qflag, s.f_len * sizeof(int)));
-    B2G_HIP(hipMalloc(&s.d_blk, nm * sizeof(JacBlock)));
-    B2G_HIP(hipMalloc(&s.d_pair, s.n_pair * sizeof(JacTask)));
-    B2G_HIP(hipMalloc(&s.d_upd, s.n_upd * sizeof(JacTask)));
-    B2G_HIP(hipMalloc(&s.d_src_off, nm * sizeof(uint64_t)));
-    B2G_HIP(hipMalloc(&s.d_w_off, nm * sizeof(uint64_t)));
-    B2G_HIP(hipMalloc(&s.nrot, sizeof(unsigned)));
-    B2G_HIP(hipHostMalloc((void **)&s.h_nrot, sizeof(unsigned)));
+    B2G_HIP(ctx->alloc(&s.A, s.a_len * sizeof(double)));
+    B2G_HIP(ctx->alloc(&s.V, s.a_len * sizeof(double)));
+    B2G_HIP(ctx->alloc(&s.Q, s.q_len * sizeof(double)));
+    B2G_HIP(ctx->alloc(&s.w, std::max<uint64_t>(s.w_len, 1) * sizeof(double)));
+    B2G_HIP(ctx->alloc(&s.qflag, s.f_len * sizeof(int)));
+    B2G_HIP(ctx->alloc(&s.d_blk, nm * sizeof(JacBlock)));
+    B2G_HIP(ctx->alloc(&s.d_pair, s.n_pair * sizeof(JacTask)));
+    B2G_HIP(ctx->alloc(&s.d_upd, s.n_upd * sizeof(JacTask)));
+    B2G_HIP(ctx->alloc(&s.d_src_off, nm * sizeof(uint64_t)));
+    B2G_HIP(ctx->alloc(&s.d_w_off, nm * sizeof(uint64_t)));
+    B2G_HIP(ctx->alloc(&s.nrot, sizeof(unsigned)));
+    B2G_HIP(ctx->pinned.get(sizeof(unsigned), (void **)&s.h_nrot));
     B2G_HIP(hipMemcpyAsync(s.d_blk, s.blk.data(), nm * sizeof(JacBlock),
                            hipMemcpyHostToDevice, st));
     B2G_HIP(hipMemcpyAsync(s.d_pair, pairs.data(), s.n_pair * sizeof(JacTask),
@@ -1157,9 +1158,8 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
         B2G_HIP(hipGetLastError());
         const unsigned nparts = 32;
         double *part = nullptr;
-        B2G_HIP(hipMalloc(&part, nm * nparts * sizeof(double)));
-        std::unique_ptr<double, int (*)(void *)> part_guard(
-            part, [](void *p) { return (int)hipFree(p); });
+        B2G_HIP(ctx->alloc(&part, nm * nparts * sizeof(double)));
+        PoolGuard part_guard(ctx, part);
         hipLaunchKernelGGL(jacobi_norm_kernel, dim3(nparts, (unsigned)nm),
                            dim3(256), 0, st, s.d_blk, s.A, part);
         B2G_HIP(hipGetLastError());
@@ -1243,9 +1243,8 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
         for (size_t i = 0; i < nm; i++)
             y_len = std::max<uint64_t>(y_len, src_off[i] + (uint64_t)n[i] * n[i]);
         double *Y = nullptr;
-        B2G_HIP(hipMalloc(&Y, std::max<uint64_t>(y_len, 1) * sizeof(double)));
-        std::unique_ptr<double, int (*)(void *)> y_guard(
-            Y, [](void *p) { return (int)hipFree(p); });
+        B2G_HIP(ctx->alloc(&Y, std::max<uint64_t>(y_len, 1) * sizeof(double)));
+        PoolGuard y_guard(ctx, Y);
         int r = ts.upload(ctx);
         if (r == B2G_OK)
             r = ts.run(ctx, src, s.V, Y);
@@ -1280,7 +1279,8 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
     }
     if (!jobs.empty()) {
         VecJob *d_jobs = nullptr;
-        B2G_HIP(hipMalloc(&d_jobs, jobs.size() * sizeof(VecJob)));
+        B2G_HIP(ctx->alloc(&d_jobs, jobs.size() * sizeof(VecJob)));
+        PoolGuard jobs_guard(ctx, d_jobs);
         hipError_t e = hipMemcpyAsync(d_jobs, jobs.data(),
                                       jobs.size() * sizeof(VecJob),
                                       hipMemcpyHostToDevice, st);
@@ -1290,7 +1290,6 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
             e = hipGetLastError();
         }
         const hipError_t e2 = hipStreamSynchronize(st);
-        hipFree(d_jobs);
         B2G_HIP(e);
         B2G_HIP(e2);
     }
@@ -1350,7 +1349,7 @@ struct b2g_split_s {
     ~b2g_split_s() {
         for (Part &p : part)
             if (p.data)
-                hipFree(p.data);
+                ctx->pool.put(p.data);
     }
 };
 
@@ -1449,9 +1448,8 @@ static int add_noise(b2g_ctx ctx, const b2g_sparse_info *wfn, uint64_t psi_len,
         T.resize(len);
     }
     double *dT = nullptr;
-    B2G_HIP(hipMalloc(&dT, T.size() * sizeof(double)));
-    std::unique_ptr<double, int (*)(void *)> t_guard(
-        dT, [](void *p) { return (int)hipFree(p); });
+    B2G_HIP(ctx->alloc(&dT, T.size() * sizeof(double)));
+    PoolGuard t_guard(ctx, dT);
     B2G_HIP(hipMemcpy(dT, T.data(), T.size() * sizeof(double),
                       hipMemcpyHostToDevice));
     if (wav) {
@@ -1481,9 +1479,8 @@ static int add_noise(b2g_ctx ctx, const b2g_sparse_info *wfn, uint64_t psi_len,
     std::vector<uint32_t> dim(dm.nb.begin(), dm.nb.end());
     const size_t bytes = nd * (sizeof(uint64_t) + sizeof(uint32_t) + sizeof(double));
     char *dbuf = nullptr;
-    B2G_HIP(hipMalloc(&dbuf, bytes));
-    std::unique_ptr<char, int (*)(void *)> b_guard(
-        dbuf, [](void *p) { return (int)hipFree(p); });
+    B2G_HIP(ctx->alloc(&dbuf, bytes));
+    PoolGuard b_guard(ctx, dbuf);
     uint64_t *d_off = (uint64_t *)dbuf;
     double *d_coef = (double *)(dbuf + nd * sizeof(uint64_t));
     uint32_t *d_dim = (uint32_t *)(dbuf + nd * (sizeof(uint64_t) + sizeof(double)));
@@ -1664,8 +1661,8 @@ static int split_impl(b2g_ctx ctx, int symmetry, const b2g_sparse_info *wfn,
                 add_tiles(ts.t, dm.shift[b], dm.nb[b], dm.nb[b], K, sb,
                           (uint32_t)ts.s.size(), 0);
         }
-        B2G_HIP(hipMalloc(&dm.data, std::max<uint64_t>(dm.len, 1) *
-                                        sizeof(double)));
+        B2G_HIP(ctx->alloc(&dm.data, std::max<uint64_t>(dm.len, 1) *
+                                         sizeof(double)));
         int r = ts.upload(ctx);
         if (r == B2G_OK)
             r = ts.run(ctx, psi, psi, dm.data);
@@ -1683,9 +1680,8 @@ static int split_impl(b2g_ctx ctx, int symmetry, const b2g_sparse_info *wfn,
     tm.mark("density matrix");
     // ---- eigen-decomposition of every block
     double *E = nullptr;
-    B2G_HIP(hipMalloc(&E, std::max<uint64_t>(dm.len, 1) * sizeof(double)));
-    std::unique_ptr<double, int (*)(void *)> e_guard(
-        E, [](void *p) { return (int)hipFree(p); });
+    B2G_HIP(ctx->alloc(&E, std::max<uint64_t>(dm.len, 1) * sizeof(double)));
+    PoolGuard e_guard(ctx, E);
     std::vector<double> w;
     {
         std::vector<uint32_t> n(dm.nb.begin(), dm.nb.end());
@@ -1800,9 +1796,10 @@ static int split_impl(b2g_ctx ctx, int symmetry, const b2g_sparse_info *wfn,
         }
     sort_part(wav);
     set_shifts(wav);
-    B2G_HIP(hipMalloc(&rot.data, std::max<uint64_t>(rot.len, 1) * sizeof(double)));
-    B2G_HIP(hipMalloc(&wav.data, std::max<uint64_t>(wav.len * n_roots, 1) *
-                                     sizeof(double)));
+    B2G_HIP(ctx->alloc(&rot.data,
+                       std::max<uint64_t>(rot.len, 1) * sizeof(double)));
+    B2G_HIP(ctx->alloc(&wav.data, std::max<uint64_t>(wav.len * n_roots, 1) *
+                                      sizeof(double)));
     // ---- rotation matrix: kept eigenvectors (rows of E) as columns
     // (trace_right) or rows
     {
@@ -1823,7 +1820,8 @@ static int split_impl(b2g_ctx ctx, int symmetry, const b2g_sparse_info *wfn,
         }
         if (!jobs.empty()) {
             RowCopy *d_jobs = nullptr;
-            B2G_HIP(hipMalloc(&d_jobs, jobs.size() * sizeof(RowCopy)));
+            B2G_HIP(ctx->alloc(&d_jobs, jobs.size() * sizeof(RowCopy)));
+            PoolGuard jobs_guard(ctx, d_jobs);
             hipError_t e = hipMemcpyAsync(d_jobs, jobs.data(),
                                           jobs.size() * sizeof(RowCopy),
                                           hipMemcpyHostToDevice, ctx->stream);
@@ -1835,7 +1833,6 @@ static int split_impl(b2g_ctx ctx, int symmetry, const b2g_sparse_info *wfn,
                 e = hipGetLastError();
             }
             const hipError_t e2 = hipStreamSynchronize(ctx->stream);
-            hipFree(d_jobs);
             B2G_HIP(e);
             B2G_HIP(e2);
         }
@@ -2025,8 +2022,10 @@ extern "C" int b2g_split_values(b2g_split s, int which, double *out,
 extern "C" int b2g_split_destroy(b2g_split s) {
     if (s == nullptr)
         return B2G_OK;
-    if (s->ctx)
-        hipStreamSynchronize(s->ctx->stream);
+    // the caller had the parts' addresses and may have used them on streams
+    // of its own
+    hipSetDevice(s->ctx->device);
+    hipDeviceSynchronize();
     delete s;
     return B2G_OK;
 }

@@ -79,6 +79,10 @@ const char *b2g_last_error(void);
 int b2g_ctx_create(int device, unsigned flags, b2g_ctx *out);
 int b2g_ctx_destroy(b2g_ctx ctx);
 int b2g_ctx_synchronize(b2g_ctx ctx);
+/* gives the device memory that the context keeps of released objects back
+ * (at most 16 GiB; it does so by itself when an allocation fails or when
+ * less than a quarter of the device is free as memory is released)        */
+int b2g_ctx_trim(b2g_ctx ctx);
 /* the context's hipStream_t (for callers that order their own work or
  * record events against it)                                              */
 void *b2g_ctx_stream(b2g_ctx ctx);
