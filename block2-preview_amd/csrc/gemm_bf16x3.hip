@@ -155,25 +155,30 @@ hipError_t launch_pack_bf16(const double *src, __bf16 *hi, __bf16 *lo,
 // ------------------------------------------------------------- tile loader
 // One workgroup = 4 waves (2x2); K staged through two LDS buffers in steps
 // of 32 (one MFMA k-step).  An LDS row holds the 32 k values of one tile row
-// (A) or tile column (B) plus 8 of padding, so that a lane's 8 k values are
-// one 16-byte read and the 16 rows of a fragment fall on distinct banks.
+// (A) or tile column (B), so that a lane's 8 k values (a k group) are one
+// 16-byte read; the k groups of a row are permuted by the row (slot) so that
+// one k group of 16 consecutive rows falls on distinct banks without padding:
+// two 128 x 128 workgroups fit a compute unit.
 template <int TM, int TN> struct PkTile {
-    static constexpr int TK = 32, LDK = TK + 8;
+    static constexpr int TK = 32;
     static constexpr int VA = TM * TK / 8, VB = TN * TK / 8; // 16 B vectors
     static constexpr int GA = (VA + 255) / 256, GB = (VB + 255) / 256;
-    static constexpr int ASZ = TM * LDK, BSZ = TN * LDK;
+    static constexpr int ASZ = TM * TK, BSZ = TN * TK;
     static constexpr int BUF = 2 * ASZ + 2 * BSZ; // A hi, A lo, B hi, B lo
     u32x4 ah[GA], al[GA], bh[GB], bl[GB];
 
-    // vector e of a tile: row and k group.  Sixteen consecutive lanes take
-    // one k group of sixteen consecutive rows, so that a wave's 16-byte LDS
-    // stores follow the bank pattern of the fragment reads (rows 80 bytes
-    // apart: any 16 of them cover distinct 16-byte bank groups of 256
-    // bytes); a wave still covers 16 whole rows of 64 bytes per global load.
-    static __device__ __forceinline__ int vrow(int e) {
-        return (e & 15) + 16 * (e >> 6);
+    // element offset of k group g of a row
+    static __device__ __forceinline__ int slot(int row, int g) {
+        const int j = (row >> 2) & 3;
+        return row * TK + 8 * (g ^ (((j ^ (j >> 1)) & 1) << 1 | j >> 1));
     }
-    static __device__ __forceinline__ int vgrp(int e) { return (e >> 4) & 3; }
+    // vector e of a tile: row and k group.  Four consecutive lanes take the
+    // 64 contiguous bytes of one row, so that a wave's load touches 16 cache
+    // lines (a lane per row of one k group touched a line per lane, and the
+    // address units, busy 70 to 80 % of the time, bound both phases), and its
+    // 16-byte LDS stores fill 1 KiB in order.
+    static __device__ __forceinline__ int vrow(int e) { return e >> 2; }
+    static __device__ __forceinline__ int vgrp(int e) { return e & 3; }
 
     __device__ __forceinline__ void load(
         __amdgpu_buffer_rsrc_t rAh, __amdgpu_buffer_rsrc_t rAl,
@@ -212,7 +217,7 @@ template <int TM, int TN> struct PkTile {
         for (int g = 0; g < GA; g++) {
             const int e = tid + 256 * g;
             if (VA % 256 == 0 || e < VA) {
-                const int o = vrow(e) * LDK + 8 * vgrp(e);
+                const int o = slot(vrow(e), vgrp(e));
                 *(u32x4 *)(buf + o) = ah[g];
                 *(u32x4 *)(buf + ASZ + o) = al[g];
             }
@@ -221,7 +226,7 @@ template <int TM, int TN> struct PkTile {
         for (int g = 0; g < GB; g++) {
             const int e = tid + 256 * g;
             if (VB % 256 == 0 || e < VB) {
-                const int o = vrow(e) * LDK + 8 * vgrp(e);
+                const int o = slot(vrow(e), vgrp(e));
                 *(u32x4 *)(buf + 2 * ASZ + o) = bh[g];
                 *(u32x4 *)(buf + 2 * ASZ + BSZ + o) = bl[g];
             }
@@ -243,29 +248,19 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
     void *__restrict__ D0, void *__restrict__ D1,
     const Task *__restrict__ tasks, int ntasks, const Seg *__restrict__ segs,
     uint64_t a_rs, uint64_t b_rs, uint64_t d_rs, uint64_t p_rs, double scale,
-    int beta0, XcdSplit xs) {
+    int beta0, int nrhs, XcdSplit xs) {
     typedef PkTile<TM, TN> T;
     constexpr int WM = TM / 2, WN = TN / 2;
     constexpr int FM = WM / 16, FN = WN / 16;
     __shared__ __attribute__((aligned(16))) __bf16 smem[2 * T::BUF];
-    const int rhs = blockIdx.y;
-    Ah += rhs * a_rs;
-    Al += rhs * a_rs;
-    Bh += rhs * b_rs;
-    Bl += rhs * b_rs;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int lr = lane & 15, lk = lane >> 4;
     T ld;
-    int t0 = blockIdx.x, tend = ntasks, tstep = gridDim.x;
-    if (xs.off[8] != 0) { // per-XCD task ranges, as in seg_gemm_kernel
-        const int x = blockIdx.x & 7;
-        t0 = (int)xs.off[x] + (int)(blockIdx.x >> 3);
-        tend = (int)xs.off[x + 1];
-        tstep = gridDim.x >> 3;
-    }
-    for (int t = t0; t < tend; t += tstep) {
-        const Task task = tasks[t];
+    for (TaskRange tr(ntasks, nrhs, xs); tr.more(); tr.next()) {
+        const Task task = tasks[tr.task()];
+        const int rhs = tr.rhs();
+        const uint64_t ao = rhs * a_rs, bo = rhs * b_rs;
         // acc: the tile's sum; part: the running segment's unscaled sum
         // (phase 1 tasks have one segment with alpha = 1: part is the sum)
         f32x4 acc[FM][FN], part[FM][FN];
@@ -286,10 +281,10 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
                           __amdgpu_buffer_rsrc_t &a1,
                           __amdgpu_buffer_rsrc_t &b0,
                           __amdgpu_buffer_rsrc_t &b1) {
-                a0 = pk_rsrc(Ah + sg.a_off);
-                a1 = pk_rsrc(Al + sg.a_off);
-                b0 = pk_rsrc(Bh + sg.b_off);
-                b1 = pk_rsrc(Bl + sg.b_off);
+                a0 = pk_rsrc(Ah + ao + sg.a_off);
+                a1 = pk_rsrc(Al + ao + sg.a_off);
+                b0 = pk_rsrc(Bh + bo + sg.b_off);
+                b1 = pk_rsrc(Bl + bo + sg.b_off);
             };
             __amdgpu_buffer_rsrc_t rAh, rAl, rBh, rBl;
             rs(cur, rAh, rAl, rBh, rBl);
@@ -321,13 +316,13 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
                 bf16x8 fah[FM], fal[FM], fbh[FN], fbl[FN];
 #pragma unroll
                 for (int i = 0; i < FM; i++) {
-                    const int o = (wm * WM + i * 16 + lr) * T::LDK + 8 * lk;
+                    const int o = T::slot(wm * WM + i * 16 + lr, lk);
                     fah[i] = *(const bf16x8 *)(sAh + o);
                     fal[i] = *(const bf16x8 *)(sAl + o);
                 }
 #pragma unroll
                 for (int j = 0; j < FN; j++) {
-                    const int o = (wn * WN + j * 16 + lr) * T::LDK + 8 * lk;
+                    const int o = T::slot(wn * WN + j * 16 + lr, lk);
                     fbh[j] = *(const bf16x8 *)(sBh + o);
                     fbl[j] = *(const bf16x8 *)(sBl + o);
                 }
@@ -360,13 +355,17 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
         }
         if constexpr (OUT == 0) {
             // W^T through LDS: the tile (row m, column n) lands in a float
-            // [TM][TN + 4] array in the (free) staging buffers, then every
-            // thread writes 8 consecutive m of one W^T row as a 16-byte
-            // vector per plane (whole rows of 256 bytes per 16 lanes)
+            // [TM][TN] array in the (free) staging buffers (columns permuted
+            // by the group of 8 rows, for the banks of the reads), then
+            // every thread writes 8 consecutive m of one W^T row as a
+            // 16-byte vector per plane (whole rows of 256 bytes per 16
+            // lanes)
             mfma_settle<f32x4, FM * FN>(&part[0][0]);
-            constexpr int LDT = TN + 4;
-            static_assert(TM * LDT * 4 <= 2 * T::BUF * 2, "W^T staging");
+            static_assert(TM * TN * 4 <= 2 * T::BUF * 2, "W^T staging");
             float *tile = (float *)smem;
+            auto at = [](int m, int n) {
+                return m * TN + (n ^ (((m >> 3) << 2) & (TN - 1)));
+            };
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < FM; i++)
@@ -374,8 +373,8 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
                 for (int j = 0; j < FN; j++)
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        tile[(wm * WM + i * 16 + 4 * lk + r) * LDT + wn * WN +
-                             j * 16 + lr] = part[i][j][r];
+                        tile[at(wm * WM + i * 16 + 4 * lk + r,
+                                wn * WN + j * 16 + lr)] = part[i][j][r];
             __syncthreads();
             __bf16 *Wh = (__bf16 *)D0 + rhs * d_rs;
             __bf16 *Wl = (__bf16 *)D1 + rhs * d_rs;
@@ -387,7 +386,7 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
                     bf16x8 h, l;
 #pragma unroll
                     for (int q = 0; q < 8; q++) {
-                        const float x = tile[(m0 + q) * LDT + n];
+                        const float x = tile[at(m0 + q, n)];
                         const __bf16 xh = (__bf16)x;
                         h[q] = xh;
                         l[q] = (__bf16)(x - (float)xh);
@@ -437,11 +436,11 @@ hipError_t launch_seg_gemm_pk(int cfg, const __bf16 *Ah, const __bf16 *Al,
                               XcdSplit xs) {
     if (ntasks <= 0)
         return hipSuccess;
-    dim3 g(task_grid(grid, ntasks, xs), (unsigned)n_rhs);
+    const dim3 g(task_grid(grid, ntasks, n_rhs));
 #define B2G_LAUNCH(TM_, TN_)                                                   \
     hipLaunchKernelGGL((seg_gemm_pk_kernel<TM_, TN_, OUT>), g, dim3(256), 0,   \
                        st, Ah, Al, Bh, Bl, D0, D1, tasks, ntasks, segs, a_rs,  \
-                       b_rs, d_rs, p_rs, scale, beta0, xs)
+                       b_rs, d_rs, p_rs, scale, beta0, n_rhs, xs)
     switch (cfg) {
     case 0: B2G_LAUNCH(32, 32); break;
     case 1: B2G_LAUNCH(32, 64); break;

@@ -72,7 +72,7 @@ __device__ __forceinline__ float buf_load_s<float>(__amdgpu_buffer_rsrc_t r,
 // Element q of thread tid is e = tid + 256 q; since 256 is a multiple of TK,
 // TM and TN, one coordinate of e is the same for all q and the other
 // advances by a constant.  Tasks are strided over the grid (persistent
-// launch); blockIdx.y selects the right-hand side.
+// launch, TaskRange).
 //
 // The registers of one chunk, with the flags and alpha of its segment, and
 // their store to LDS ([k][m] and [k][n] layouts, one padding column), alpha
@@ -341,20 +341,6 @@ __device__ __forceinline__ void seg_gemm_task(
             }
 }
 
-// Tasks of one launch: first index, end and stride of this workgroup
-struct TaskRange {
-    int t0, tend, tstep;
-    __device__ __forceinline__ TaskRange(int ntasks, const XcdSplit &xs)
-        : t0(blockIdx.x), tend(ntasks), tstep(gridDim.x) {
-        if (xs.off[8] != 0) {
-            const int x = blockIdx.x & 7;
-            t0 = (int)xs.off[x] + (int)(blockIdx.x >> 3);
-            tend = (int)xs.off[x + 1];
-            tstep = gridDim.x >> 3;
-        }
-    }
-};
-
 // tiles with a side of 128: one launch per shape
 template <typename TA, typename TB, typename TD, typename TC, int TM, int TN,
           int TK, int PHASE>
@@ -362,12 +348,11 @@ __global__ __launch_bounds__(256) void seg_gemm_kernel(
     const TA *__restrict__ A, const TB *__restrict__ B, TD *__restrict__ D,
     TD *__restrict__ P, const Task *__restrict__ tasks, int ntasks,
     const Seg *__restrict__ segs, uint64_t a_rs, uint64_t b_rs, uint64_t d_rs,
-    uint64_t p_rs, double scale, int beta0, XcdSplit xs) {
+    uint64_t p_rs, double scale, int beta0, int nrhs, XcdSplit xs) {
     __shared__ TC smem[2 * TK * (TM + TN + 2)];
-    const int rhs = blockIdx.y;
-    const TaskRange tr(ntasks, xs);
-    for (int t = tr.t0; t < tr.tend; t += tr.tstep) {
-        const Task task = tasks[t];
+    for (TaskRange tr(ntasks, nrhs, xs); tr.more(); tr.next()) {
+        const Task task = tasks[tr.task()];
+        const int rhs = tr.rhs();
         seg_gemm_task<TA, TB, TD, TC, TM, TN, TK>(
             A + rhs * a_rs, B + rhs * b_rs, D + rhs * d_rs, P + rhs * p_rs,
             task, segs, scale, beta0, smem);
@@ -391,19 +376,15 @@ __global__ __launch_bounds__(256, 4) void seg_gemm_small_kernel(
     const TA *__restrict__ A, const TB *__restrict__ B, TD *__restrict__ D,
     TD *__restrict__ P, const Task *__restrict__ tasks, int ntasks,
     const Seg *__restrict__ segs, uint64_t a_rs, uint64_t b_rs, uint64_t d_rs,
-    uint64_t p_rs, double scale, int beta0, XcdSplit xs) {
+    uint64_t p_rs, double scale, int beta0, int nrhs, XcdSplit xs) {
     __shared__ TC smem[2 * 32 * (32 + 32 + 2)]; // >= 2 * 16 * (64 + 64 + 2)
-    const int rhs = blockIdx.y;
-    A += rhs * a_rs;
-    B += rhs * b_rs;
-    D += rhs * d_rs;
-    P += rhs * p_rs;
-    const TaskRange tr(ntasks, xs);
-    for (int t = tr.t0; t < tr.tend; t += tr.tstep) {
-        const Task task = tasks[t];
+    for (TaskRange tr(ntasks, nrhs, xs); tr.more(); tr.next()) {
+        const Task task = tasks[tr.task()];
+        const int rhs = tr.rhs();
 #define B2G_TASK(TM_, TN_, TK_)                                                \
-    seg_gemm_task<TA, TB, TD, TC, TM_, TN_, TK_>(A, B, D, P, task, segs,       \
-                                                 scale, beta0, smem)
+    seg_gemm_task<TA, TB, TD, TC, TM_, TN_, TK_>(                              \
+        A + rhs * a_rs, B + rhs * b_rs, D + rhs * d_rs, P + rhs * p_rs, task,  \
+        segs, scale, beta0, smem)
         switch (__builtin_amdgcn_readfirstlane(task_cfg(task))) {
         case 0: B2G_TASK(32, 32, 32); break;
         case 1: B2G_TASK(32, 64, 16); break;
@@ -483,10 +464,11 @@ template hipError_t launch_splitk_reduce<double>(double *, const double *,
 int tile_m(int cfg) { return 32 << (cfg / 3); }
 int tile_n(int cfg) { return 32 << (cfg % 3); }
 
-// persistent grid: min(grid, ntasks) workgroups
-unsigned task_grid(int grid, int ntasks, const XcdSplit &xs) {
-    const int g = grid < ntasks ? grid : ntasks;
-    return (unsigned)(xs.off[8] != 0 ? (g + 7) & ~7 : g);
+// persistent grid: min(grid, ntasks) workgroups per right-hand side, a
+// multiple of 8
+unsigned task_grid(int grid, int ntasks, int n_rhs) {
+    const int64_t g = (int64_t)(grid < ntasks ? grid : ntasks) * n_rhs;
+    return (unsigned)((g < (1 << 30) ? g : (1 << 30)) + 7) & ~7u;
 }
 
 template <typename TA, typename TB, typename TD, typename TC, int PHASE>
@@ -497,12 +479,12 @@ hipError_t launch_seg_gemm(int cfg, const TA *A, const TB *B, TD *D, TD *P,
                            int grid, hipStream_t st, XcdSplit xs) {
     if (ntasks <= 0)
         return hipSuccess;
-    dim3 g(task_grid(grid, ntasks, xs), (unsigned)n_rhs);
+    const dim3 g(task_grid(grid, ntasks, n_rhs));
 #define B2G_LAUNCH(TM_, TN_, TK_)                                              \
     hipLaunchKernelGGL((seg_gemm_kernel<TA, TB, TD, TC, TM_, TN_, TK_, PHASE>), \
                        g,                                                      \
                        dim3(256), 0, st, A, B, D, P, tasks, ntasks, segs,      \
-                       a_rs, b_rs, d_rs, p_rs, scale, beta0, xs)
+                       a_rs, b_rs, d_rs, p_rs, scale, beta0, n_rhs, xs)
     switch (cfg) {
     case 2: B2G_LAUNCH(32, 128, 16); break;
     case 5: B2G_LAUNCH(64, 128, 16); break;
@@ -512,7 +494,7 @@ hipError_t launch_seg_gemm(int cfg, const TA *A, const TB *B, TD *D, TD *P,
     default:
         hipLaunchKernelGGL((seg_gemm_small_kernel<TA, TB, TD, TC, PHASE>), g,
                            dim3(256), 0, st, A, B, D, P, tasks, ntasks, segs,
-                           a_rs, b_rs, d_rs, p_rs, scale, beta0, xs);
+                           a_rs, b_rs, d_rs, p_rs, scale, beta0, n_rhs, xs);
         break;
     }
 #undef B2G_LAUNCH

@@ -86,6 +86,32 @@ struct XcdSplit {
     uint32_t off[9];
 };
 
+// The (task, right-hand side) items of one launch, walked by a workgroup.
+// The right-hand sides of a task run next to one another on one XCD
+// (workgroup b runs on XCD b % 8), where the operator panels they share stay
+// in its L2.  The grid is a multiple of 8 workgroups (task_grid).
+struct TaskRange {
+    int i, end, step, nrhs, x; // item of the XCD's own sequence
+    bool split;
+    __device__ __forceinline__ TaskRange(int ntasks, int nrhs_,
+                                         const XcdSplit &xs)
+        : nrhs(nrhs_), x(blockIdx.x & 7), split(xs.off[8] != 0) {
+        const int t0 = split ? (int)xs.off[x] : 0;
+        const int t1 = split ? (int)xs.off[x + 1] : (ntasks - x + 7) / 8;
+        i = t0 * nrhs + (int)(blockIdx.x >> 3);
+        end = t1 * nrhs;
+        step = (int)(gridDim.x >> 3);
+    }
+    __device__ __forceinline__ bool more() const { return i < end; }
+    __device__ __forceinline__ void next() { i += step; }
+    // task index and right-hand side of the current item
+    __device__ __forceinline__ int task() const {
+        const int t = i / nrhs;
+        return split ? t : 8 * t + x;
+    }
+    __device__ __forceinline__ int rhs() const { return i % nrhs; }
+};
+
 // Deterministic split-K reduction of one output tile:
 //   D[tile] = (beta ? D[tile] : 0) + sum_{p < nparts} P[p_off + p*tm*tn + ...]
 struct RedTask {

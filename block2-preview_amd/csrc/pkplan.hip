@@ -242,7 +242,7 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
         // one W^T block per phase-1 segment, tiled with the split-BF16
         // rates (segment K from the plan's own segments)
         jobs.emplace_back([&]() {
-            tile_env_refresh(~0ull, ~0ull, p->ctx->num_cu);
+            tile_env_refresh(p->macs, p->macs2, p->ctx->num_cu, 1);
             for (size_t si = 0; si < ch.s1.size(); si++)
                 for (const Tile &t :
                      tile_cover(m1[si], n1[si], ch.s1[si].K, 1))
@@ -253,7 +253,7 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
         // output blocks re-tiled likewise, with split-K partial slots and
         // reductions of their own
         jobs.emplace_back([&]() {
-            tile_env_refresh(~0ull, ~0ull, p->ctx->num_cu);
+            tile_env_refresh(p->macs, p->macs2, p->ctx->num_cu, 1);
             for (const BlockJob &j : ch.jobs2)
                 add_split_tiles(ch.s2, j, 1, h.t2, h.red, h.p_len);
         });

@@ -89,8 +89,10 @@ struct Tile {
 // Tiling settings for the plan this host thread builds next; every plan
 // builder calls it first.  macs: multiply-adds of the plan's products (both
 // phases), macs2 those of the phase that is split along K (0: none), on
-// num_cu compute units.  B2G_TILE, B2G_TILE_CAP and B2G_KSPLIT override.
-void tile_env_refresh(uint64_t macs, uint64_t macs2, int num_cu);
+// num_cu compute units; table: 0 FP64 / FP32 kernels, 1 split-BF16 kernels.
+// B2G_TILE, B2G_TILE_CAP and B2G_KSPLIT override.
+void tile_env_refresh(uint64_t macs, uint64_t macs2, int num_cu,
+                      int table = 0);
 // 1024-element slices of the largest tile of a reduction list
 int red_slices(const std::vector<RedTask> &red);
 // tiling of an M x N output block for tasks of depth K (measured tile

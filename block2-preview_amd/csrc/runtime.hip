@@ -494,7 +494,7 @@ constexpr uint64_t kSmallPlanMacs = 25000000000ull;
 // at n=8 M=50 depths 64 / 256 / 1024 take 48 / 59 / 107 us.
 constexpr uint64_t kSplitTasksPerCu = 6;
 
-void tile_env_refresh(uint64_t macs, uint64_t macs2, int num_cu) {
+void tile_env_refresh(uint64_t macs, uint64_t macs2, int num_cu, int table) {
     TileEnv v;
     if (const char *e = getenv("B2G_TILE")) {
         // "T" (square) or "TMxTN", sizes from {32, 64, 128}
@@ -517,10 +517,14 @@ void tile_env_refresh(uint64_t macs, uint64_t macs2, int num_cu) {
     if (const char *e = getenv("B2G_TILE_CAP"))
         if (atoi(e) == 64 || atoi(e) == 128)
             v.cap = (uint32_t)atoi(e);
-    if (ks == nullptr)
+    // (split-BF16: k-steps of 32 and half the time per step: no shallower
+    // than 256, and large plans as deep as they were: M=200 depths 64 / 256 /
+    // 2048 take 71 / 64 / 133 us, M=2000 512 / 1024 / 2048 966 / 897 / 887)
+    if (ks == nullptr && (table == 0 || v.cap == 64))
         v.ksplit = std::min<uint64_t>(
-            2048, std::max<uint64_t>(64, macs2 / (kSplitTasksPerCu * num_cu *
-                                                  v.cap * v.cap)));
+            2048, std::max<uint64_t>(table == 0 ? 64 : 256,
+                                     macs2 / (kSplitTasksPerCu * num_cu *
+                                              v.cap * v.cap)));
     t_env = v;
 }
 
