@@ -10,19 +10,24 @@
 // 3 * 16 cycles per 16x16x32 block against 8 * 32 cycles for the same block
 // with FP32 16x16x4 MFMAs; the Davidson that uses them refines in FP64.
 //
-// Packed planes.  A GEMM operand is held as a row-major R x ld matrix whose
-// rows run along the contraction index k (ld = K rounded up to 8, columns
-// [K, ld) zero), stored twice with identical layout: the hi plane and the lo
-// plane.  Eight consecutive k of a row are one aligned 16-byte vector, so the
-// tile loader issues 16-byte buffer loads and 16-byte LDS stores and does no
-// arithmetic.  The constant operators are packed once per plan (in the
-// orientation each pair reads them), the wavefunction once per H*psi, and
-// phase 1 writes its product W directly as packed W^T planes for phase 2.
+// Packed operands.  A GEMM operand is held as a row-major matrix whose rows
+// run along the contraction index k, K rounded up to 32 with zeros; every 32
+// k of a row are one aligned 128-byte line, the 32 hi values and then the 32
+// lo values.  A k-step of a tile row is therefore one whole cache line: the
+// loader reads it with eight lanes' 16-byte buffer loads and does no
+// arithmetic.  (As two planes, a k-step read half of two lines, twice the
+// requests between a compute unit's L1 and L2, whose number in flight bounds
+// these kernels: H*psi at M=3000 with four right-hand sides 14.4 against
+// 11.9 ms, matrix cores busy 33 against 46 % of phase 2.)  The constant
+// operators are packed once per plan (in the orientation each pair reads
+// them), the wavefunction once per H*psi, and phase 1 writes its product W
+// directly as packed W^T for phase 2.
 //
 // Task / segment semantics are those of seg_gemm_kernel (kernels.hip): a
 // task is one TM x TN output tile accumulating sum_s alpha_s A_s B_s^T over
-// its segments (A_s: M x K_s, B_s: N x K_s, both packed), the tile owned by
-// exactly one task (no atomics).  alpha_s is applied to each segment's FP32
+// its segments (A_s: M x K_s, B_s: N x K_s, both packed, lda / ldb the packed
+// row stride in elements, hi and lo counted), the tile owned by exactly one
+// task (no atomics).  alpha_s is applied to each segment's FP32
 // partial sum when the segment ends.
 #include "kernels.hpp"
 #include "launch.hpp"
@@ -41,18 +46,27 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// raw buffer resource over one packed matrix: offsets are 32-bit byte
-// offsets below 2^31 (matrices hold fewer than 2^28 elements); an offset of
-// kPkMasked lies past the record count and reads as zero
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t pk_rsrc(const __bf16 *p) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16 *>(p),
-                                             (short)0, 0x7FFFFFF0, 0x00020000);
+// Raw buffer resource over rows row0 .. row0 + tile of a packed matrix of
+// `rows` rows and stride ld.  Rows from `rows` on lie past its end and read
+// as zero.  (A packed matrix has rows * round8(K) < 2^28, so `tile` <= 128
+// rows are fewer than 2^31 bytes.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t
+pk_rsrc(const __bf16 *p, uint32_t row0, uint32_t rows, uint32_t ld, int tile) {
+    const uint32_t n = min(rows - row0, (uint32_t)tile);
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<__bf16 *>(p + (uint64_t)row0 * ld), (short)0,
+        (int)(2 * ld * n), 0x00020000);
 }
-constexpr uint32_t kPkMasked = 0x80000000u;
-
 __device__ __forceinline__ u32x4 pk_load(__amdgpu_buffer_rsrc_t r,
-                                         uint32_t off) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+                                         uint32_t off, uint32_t soff) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)soff, 0);
+}
+
+// element offset of the hi value (r, k) of a packed matrix of row stride ld;
+// its lo value is 32 elements on
+__device__ __forceinline__ uint64_t pk_offset(uint32_t r, uint32_t k,
+                                              uint32_t ld) {
+    return (uint64_t)r * ld + (k >> 5) * 64 + (k & 31);
 }
 
 // ------------------------------------------------------------------ packing
@@ -66,16 +80,15 @@ __device__ __forceinline__ u32x4 pk_load(__amdgpu_buffer_rsrc_t r,
 constexpr int kPackGPT = 4;
 
 __global__ __launch_bounds__(256) void pack_bf16_kernel(
-    const double *__restrict__ src, __bf16 *__restrict__ hi,
-    __bf16 *__restrict__ lo, const PackMat *__restrict__ mats, int nmats,
-    uint64_t ngroups, uint64_t src_rs, uint64_t dst_rs) {
+    const double *__restrict__ src, __bf16 *__restrict__ dst,
+    const PackMat *__restrict__ mats, int nmats, uint64_t ngroups,
+    uint64_t src_rs, uint64_t dst_rs) {
     constexpr int G = 256 * kPackGPT;
     __shared__ uint64_t sg0[G + 1];
     __shared__ int sm[2];
     const int rhs = blockIdx.y;
     src += rhs * src_rs;
-    hi += rhs * dst_rs;
-    lo += rhs * dst_rs;
+    dst += rhs * dst_rs;
     const uint64_t base = (uint64_t)blockIdx.x * G;
     if (base >= ngroups)
         return;
@@ -130,13 +143,13 @@ __global__ __launch_bounds__(256) void pack_bf16_kernel(
             h[i] = vh;
             lw[i] = (__bf16)(float)(v - (double)(float)vh);
         }
-        const uint64_t o = pm.dst + (uint64_t)r * pm.dst_ld + k;
-        *(bf16x8 *)(hi + o) = h;
-        *(bf16x8 *)(lo + o) = lw;
+        __bf16 *o = dst + pm.dst + pk_offset(r, k, 2 * pm.dst_ld);
+        *(bf16x8 *)o = h;
+        *(bf16x8 *)(o + 32) = lw;
     }
 }
 
-hipError_t launch_pack_bf16(const double *src, __bf16 *hi, __bf16 *lo,
+hipError_t launch_pack_bf16(const double *src, __bf16 *dst,
                             const PackMat *mats, int nmats, uint64_t ngroups,
                             uint64_t src_rs, uint64_t dst_rs, int n_rhs,
                             int grid, hipStream_t st) {
@@ -147,7 +160,7 @@ hipError_t launch_pack_bf16(const double *src, __bf16 *hi, __bf16 *lo,
     if (g >= (1ull << 31))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(pack_bf16_kernel, dim3((unsigned)g, (unsigned)n_rhs),
-                       dim3(256), 0, st, src, hi, lo, mats, nmats, ngroups,
+                       dim3(256), 0, st, src, dst, mats, nmats, ngroups,
                        src_rs, dst_rs);
     return hipGetLastError();
 }
@@ -161,90 +174,77 @@ hipError_t launch_pack_bf16(const double *src, __bf16 *hi, __bf16 *lo,
 // two 128 x 128 workgroups fit a compute unit.
 template <int TM, int TN> struct PkTile {
     static constexpr int TK = 32;
-    static constexpr int VA = TM * TK / 8, VB = TN * TK / 8; // 16 B vectors
-    static constexpr int GA = (VA + 255) / 256, GB = (VB + 255) / 256;
+    static constexpr int VA = TM * 8, VB = TN * 8; // 16-byte vectors
+    static_assert(VA % 256 == 0 && VB % 256 == 0, "whole loads per thread");
+    static constexpr int GA = VA / 256, GB = VB / 256; // per thread
     static constexpr int ASZ = TM * TK, BSZ = TN * TK;
     static constexpr int BUF = 2 * ASZ + 2 * BSZ; // A hi, A lo, B hi, B lo
-    u32x4 ah[GA], al[GA], bh[GB], bl[GB];
+    u32x4 a[GA], b[GB];
+    uint32_t va, vb, sa, sb;
 
     // element offset of k group g of a row
     static __device__ __forceinline__ int slot(int row, int g) {
         const int j = (row >> 2) & 3;
         return row * TK + 8 * (g ^ (((j ^ (j >> 1)) & 1) << 1 | j >> 1));
     }
-    // vector e of a tile: row and k group.  Four consecutive lanes take the
-    // 64 contiguous bytes of one row, so that a wave's load touches 16 cache
-    // lines (a lane per row of one k group touched a line per lane, and the
-    // address units, busy 70 to 80 % of the time, bound both phases), and its
-    // 16-byte LDS stores fill 1 KiB in order.
-    static __device__ __forceinline__ int vrow(int e) { return e >> 2; }
-    static __device__ __forceinline__ int vgrp(int e) { return e & 3; }
-
-    __device__ __forceinline__ void load(
-        __amdgpu_buffer_rsrc_t rAh, __amdgpu_buffer_rsrc_t rAl,
-        __amdgpu_buffer_rsrc_t rBh, __amdgpu_buffer_rsrc_t rBl, const Seg &sg,
-        uint32_t k0, const Task &task, int tid) {
+    // Vector e of a tile: row e / 8, and part e % 8 of the row's line (hi
+    // groups 0..3, lo groups 4..7).  Where it goes in LDS: the planes lie
+    // one after the other; the lo plane reverses every four rows, so that
+    // the eight lanes of a row, and the sixteen of two, meet no bank twice
+    // (rows in their order: a third of the LDS cycles are conflicts).
+    static __device__ __forceinline__ int place(int e, int plane) {
+        const int row = e >> 3, g = e & 3;
+        return (e & 4) ? plane + slot(row ^ 3, g) : slot(row, g);
+    }
+    // Offsets of one segment, in bytes from the tile's first row: the
+    // thread's first vector, and 32 rows (a workgroup's reach).  Sums
+    // saturate, so a row past the resource's end stays past it.
+    __device__ __forceinline__ void setup(const Seg &sg, int tid) {
+        va = sat32(2 * (uint64_t)sg.lda * (tid >> 3)) + 16 * (tid & 7);
+        vb = sat32(2 * (uint64_t)sg.ldb * (tid >> 3)) + 16 * (tid & 7);
+        sa = sat32(64 * (uint64_t)sg.lda), sb = sat32(64 * (uint64_t)sg.ldb);
+    }
+    static __device__ __forceinline__ uint32_t sat32(uint64_t v) {
+        return v < 0xFFFFFF00u ? (uint32_t)v : 0xFFFFFF00u;
+    }
+    // k0 a multiple of 32: four bytes per k
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rA,
+                                         __amdgpu_buffer_rsrc_t rB,
+                                         uint32_t k0) {
 #pragma unroll
-        for (int g = 0; g < GA; g++) {
-            const int e = tid + 256 * g;
-            if (VA % 256 == 0 || e < VA) {
-                const uint32_t r = task.row0 + vrow(e);
-                const uint32_t k = k0 + 8 * vgrp(e);
-                const uint32_t off = (r < task.M && k < sg.K)
-                                         ? 2 * (r * sg.lda + k)
-                                         : kPkMasked;
-                ah[g] = pk_load(rAh, off);
-                al[g] = pk_load(rAl, off);
-            }
-        }
+        for (int g = 0; g < GA; g++)
+            a[g] = pk_load(rA, reach(va, sa, g), 4 * k0);
 #pragma unroll
-        for (int g = 0; g < GB; g++) {
-            const int e = tid + 256 * g;
-            if (VB % 256 == 0 || e < VB) {
-                const uint32_t c = task.col0 + vrow(e);
-                const uint32_t k = k0 + 8 * vgrp(e);
-                const uint32_t off = (c < task.N && k < sg.K)
-                                         ? 2 * (c * sg.ldb + k)
-                                         : kPkMasked;
-                bh[g] = pk_load(rBh, off);
-                bl[g] = pk_load(rBl, off);
-            }
-        }
+        for (int g = 0; g < GB; g++)
+            b[g] = pk_load(rB, reach(vb, sb, g), 4 * k0);
+    }
+    static __device__ __forceinline__ uint32_t reach(uint32_t v, uint32_t s,
+                                                     int g) {
+        for (int i = 0; i < g; i++)
+            v = __builtin_elementwise_add_sat(v, s);
+        return v;
     }
 
     __device__ __forceinline__ void store(__bf16 *buf, int tid) const {
 #pragma unroll
-        for (int g = 0; g < GA; g++) {
-            const int e = tid + 256 * g;
-            if (VA % 256 == 0 || e < VA) {
-                const int o = slot(vrow(e), vgrp(e));
-                *(u32x4 *)(buf + o) = ah[g];
-                *(u32x4 *)(buf + ASZ + o) = al[g];
-            }
-        }
+        for (int g = 0; g < GA; g++)
+            *(u32x4 *)(buf + place(tid + 256 * g, ASZ)) = a[g];
 #pragma unroll
-        for (int g = 0; g < GB; g++) {
-            const int e = tid + 256 * g;
-            if (VB % 256 == 0 || e < VB) {
-                const int o = slot(vrow(e), vgrp(e));
-                *(u32x4 *)(buf + 2 * ASZ + o) = bh[g];
-                *(u32x4 *)(buf + 2 * ASZ + BSZ + o) = bl[g];
-            }
-        }
+        for (int g = 0; g < GB; g++)
+            *(u32x4 *)(buf + 2 * ASZ + place(tid + 256 * g, BSZ)) = b[g];
     }
 };
 
-// OUT 0: D0/D1 are the hi/lo planes of the packed transpose of the output
-//        (element (m, n) of a task's block at d_off + n*ldd + m, ldd the
-//        packed row length; rows M <= m < ldd receive the zeros of the
-//        masked A rows, so the padding of W^T is rewritten by every launch),
-//        written through LDS as 16-byte vectors along m;
+// OUT 0: D0 is the packed transpose of the output (row n, k index m, of a
+//        task's block at d_off, ldd the packed row stride; rows M <= m <
+//        ldd / 2 receive the zeros of the masked A rows, so the padding of
+//        W^T is rewritten by every launch), written through LDS as 16-byte
+//        vectors along m;
 // OUT 1: D0 is the FP64 output (row-major, ldd), D1 the FP64 split-K
 //        partial buffer (task.beta bit 1), as in seg_gemm_kernel.
 template <int TM, int TN, int OUT>
 __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
-    const __bf16 *__restrict__ Ah, const __bf16 *__restrict__ Al,
-    const __bf16 *__restrict__ Bh, const __bf16 *__restrict__ Bl,
+    const __bf16 *__restrict__ A, const __bf16 *__restrict__ B,
     void *__restrict__ D0, void *__restrict__ D1,
     const Task *__restrict__ tasks, int ntasks, const Seg *__restrict__ segs,
     uint64_t a_rs, uint64_t b_rs, uint64_t d_rs, uint64_t p_rs, double scale,
@@ -277,19 +277,13 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
             Seg nxt = cur;
             if (s + 1 < task.seg_end)
                 nxt = segs[s + 1];
-            auto rs = [&](const Seg &sg, __amdgpu_buffer_rsrc_t &a0,
-                          __amdgpu_buffer_rsrc_t &a1,
-                          __amdgpu_buffer_rsrc_t &b0,
-                          __amdgpu_buffer_rsrc_t &b1) {
-                a0 = pk_rsrc(Ah + ao + sg.a_off);
-                a1 = pk_rsrc(Al + ao + sg.a_off);
-                b0 = pk_rsrc(Bh + bo + sg.b_off);
-                b1 = pk_rsrc(Bl + bo + sg.b_off);
-            };
-            __amdgpu_buffer_rsrc_t rAh, rAl, rBh, rBl;
-            rs(cur, rAh, rAl, rBh, rBl);
+            __amdgpu_buffer_rsrc_t rA =
+                pk_rsrc(A + ao + cur.a_off, task.row0, task.M, cur.lda, TM);
+            __amdgpu_buffer_rsrc_t rB =
+                pk_rsrc(B + bo + cur.b_off, task.col0, task.N, cur.ldb, TN);
             int buf = 0;
-            ld.load(rAh, rAl, rBh, rBl, cur, k0, task, tid);
+            ld.setup(cur, tid);
+            ld.load(rA, rB, 0);
             ld.store(smem, tid);
             __syncthreads();
             float alpha = (float)cur.alpha; // of the segment in LDS
@@ -303,12 +297,16 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
                     cur = nxt;
                     if (s + 1 < task.seg_end)
                         nxt = segs[s + 1];
-                    rs(cur, rAh, rAl, rBh, rBl);
+                    rA =
+                pk_rsrc(A + ao + cur.a_off, task.row0, task.M, cur.lda, TM);
+                    rB =
+                pk_rsrc(B + bo + cur.b_off, task.col0, task.N, cur.ldb, TN);
                     alpha = (float)cur.alpha;
+                    ld.setup(cur, tid);
                 }
                 const bool more = s < task.seg_end;
                 if (more)
-                    ld.load(rAh, rAl, rBh, rBl, cur, k0, task, tid);
+                    ld.load(rA, rB, k0);
                 const __bf16 *sAh = smem + buf * T::BUF;
                 const __bf16 *sAl = sAh + T::ASZ;
                 const __bf16 *sBh = sAh + 2 * T::ASZ;
@@ -316,15 +314,15 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
                 bf16x8 fah[FM], fal[FM], fbh[FN], fbl[FN];
 #pragma unroll
                 for (int i = 0; i < FM; i++) {
-                    const int o = T::slot(wm * WM + i * 16 + lr, lk);
-                    fah[i] = *(const bf16x8 *)(sAh + o);
-                    fal[i] = *(const bf16x8 *)(sAl + o);
+                    const int r = wm * WM + i * 16 + lr;
+                    fah[i] = *(const bf16x8 *)(sAh + T::slot(r, lk));
+                    fal[i] = *(const bf16x8 *)(sAl + T::slot(r ^ 3, lk));
                 }
 #pragma unroll
                 for (int j = 0; j < FN; j++) {
-                    const int o = T::slot(wn * WN + j * 16 + lr, lk);
-                    fbh[j] = *(const bf16x8 *)(sBh + o);
-                    fbl[j] = *(const bf16x8 *)(sBl + o);
+                    const int r = wn * WN + j * 16 + lr;
+                    fbh[j] = *(const bf16x8 *)(sBh + T::slot(r, lk));
+                    fbl[j] = *(const bf16x8 *)(sBl + T::slot(r ^ 3, lk));
                 }
                 // small cross terms first, then the leading term
 #pragma unroll
@@ -376,13 +374,12 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
                         tile[at(wm * WM + i * 16 + 4 * lk + r,
                                 wn * WN + j * 16 + lr)] = part[i][j][r];
             __syncthreads();
-            __bf16 *Wh = (__bf16 *)D0 + rhs * d_rs;
-            __bf16 *Wl = (__bf16 *)D1 + rhs * d_rs;
+            __bf16 *W = (__bf16 *)D0 + rhs * d_rs;
             constexpr int MG = TM / 8;
             for (int v = tid; v < TN * MG; v += 256) {
                 const int n = v / MG, m0 = 8 * (v % MG);
                 const uint32_t row = task.row0 + m0, col = task.col0 + n;
-                if (row < task.ldd && col < task.N) {
+                if (row < task.ldd / 2 && col < task.N) {
                     bf16x8 h, l;
 #pragma unroll
                     for (int q = 0; q < 8; q++) {
@@ -391,10 +388,9 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
                         h[q] = xh;
                         l[q] = (__bf16)(x - (float)xh);
                     }
-                    const uint64_t o =
-                        task.d_off + (uint64_t)col * task.ldd + row;
-                    *(bf16x8 *)(Wh + o) = h;
-                    *(bf16x8 *)(Wl + o) = l;
+                    __bf16 *o = W + task.d_off + pk_offset(col, row, task.ldd);
+                    *(bf16x8 *)o = h;
+                    *(bf16x8 *)(o + 32) = l;
                 }
             }
             __syncthreads(); // the staging buffers are the next task's
@@ -427,9 +423,8 @@ __global__ __launch_bounds__(256) void seg_gemm_pk_kernel(
 }
 
 template <int OUT>
-hipError_t launch_seg_gemm_pk(int cfg, const __bf16 *Ah, const __bf16 *Al,
-                              const __bf16 *Bh, const __bf16 *Bl, void *D0,
-                              void *D1, const Task *tasks, int ntasks,
+hipError_t launch_seg_gemm_pk(int cfg, const __bf16 *A, const __bf16 *B,
+                              void *D0, void *D1, const Task *tasks, int ntasks,
                               const Seg *segs, uint64_t a_rs, uint64_t b_rs,
                               uint64_t d_rs, uint64_t p_rs, double scale,
                               int beta0, int n_rhs, int grid, hipStream_t st,
@@ -439,7 +434,7 @@ hipError_t launch_seg_gemm_pk(int cfg, const __bf16 *Ah, const __bf16 *Al,
     const dim3 g(task_grid(grid, ntasks, n_rhs));
 #define B2G_LAUNCH(TM_, TN_)                                                   \
     hipLaunchKernelGGL((seg_gemm_pk_kernel<TM_, TN_, OUT>), g, dim3(256), 0,   \
-                       st, Ah, Al, Bh, Bl, D0, D1, tasks, ntasks, segs, a_rs,  \
+                       st, A, B, D0, D1, tasks, ntasks, segs, a_rs,            \
                        b_rs, d_rs, p_rs, scale, beta0, n_rhs, xs)
     switch (cfg) {
     case 0: B2G_LAUNCH(32, 32); break;
@@ -457,13 +452,11 @@ hipError_t launch_seg_gemm_pk(int cfg, const __bf16 *Ah, const __bf16 *Al,
 }
 
 template hipError_t launch_seg_gemm_pk<0>(int, const __bf16 *, const __bf16 *,
-                                          const __bf16 *, const __bf16 *,
                                           void *, void *, const Task *, int,
                                           const Seg *, uint64_t, uint64_t,
                                           uint64_t, uint64_t, double, int, int,
                                           int, hipStream_t, XcdSplit);
 template hipError_t launch_seg_gemm_pk<1>(int, const __bf16 *, const __bf16 *,
-                                          const __bf16 *, const __bf16 *,
                                           void *, void *, const Task *, int,
                                           const Seg *, uint64_t, uint64_t,
                                           uint64_t, uint64_t, double, int, int,

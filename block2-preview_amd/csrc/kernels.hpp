@@ -119,9 +119,9 @@ struct RedTask {
     uint32_t ldd, M, N, row0, col0, tm, tn, nparts, beta, pad;
 };
 
-// One matrix of a packing job (split-BF16 operand planes, gemm_bf16x3.hip):
-// a rows x dst_ld packed matrix at element offset dst (dst_ld = cols rounded
-// up to 8), element (r, k) = src[src + r*src_ld + k] (trans:
+// One matrix of a packing job (split-BF16 operands, gemm_bf16x3.hip): a
+// rows x dst_ld packed matrix at element offset dst (dst_ld = cols rounded
+// up to 32; two elements, hi and lo, per value), value (r, k) = src[src + r*src_ld + k] (trans:
 // src[src + k*src_ld + r]) for k < cols and zero for cols <= k < dst_ld.  It
 // is packed in groups of 8 consecutive k of one row, rows * dst_ld / 8 of
 // them numbered from g0 on; the matrices of a job are sorted by g0.

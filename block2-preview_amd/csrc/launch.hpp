@@ -35,20 +35,19 @@ hipError_t launch_splitk_reduce(TD *D, const TD *P, const RedTask *tasks,
                                 hipStream_t st);
 
 // split-BF16 three-term variant on packed operand planes (gemm_bf16x3.hip):
-// segments address packed A (M x lda) and packed B (N x ldb) planes, both
-// k-contiguous; OUT 0 writes the packed transpose of the product as hi / lo
-// planes (D0 / D1), OUT 1 writes FP64 D0 with split-K partials in D1
+// segments address packed A (M x lda) and packed B (N x ldb), both
+// k-contiguous; OUT 0 writes the packed transpose of the product (D0), OUT 1
+// writes FP64 D0 with split-K partials in D1
 template <int OUT>
-hipError_t launch_seg_gemm_pk(int cfg, const __bf16 *Ah, const __bf16 *Al,
-                              const __bf16 *Bh, const __bf16 *Bl, void *D0,
-                              void *D1, const Task *tasks, int ntasks,
+hipError_t launch_seg_gemm_pk(int cfg, const __bf16 *A, const __bf16 *B,
+                              void *D0, void *D1, const Task *tasks, int ntasks,
                               const Seg *segs, uint64_t a_rs, uint64_t b_rs,
                               uint64_t d_rs, uint64_t p_rs, double scale,
                               int beta0, int n_rhs, int grid, hipStream_t st,
                               XcdSplit xs = XcdSplit{});
-// FP64 -> packed hi / lo BF16 planes, per right-hand side (src_rs, dst_rs):
+// FP64 -> packed hi / lo BF16, per right-hand side (src_rs, dst_rs):
 // the nmats matrices of `mats` (ngroups 8-element groups in all)
-hipError_t launch_pack_bf16(const double *src, __bf16 *hi, __bf16 *lo,
+hipError_t launch_pack_bf16(const double *src, __bf16 *dst,
                             const PackMat *mats, int nmats, uint64_t ngroups,
                             uint64_t src_rs, uint64_t dst_rs, int n_rhs,
                             int grid, hipStream_t st);

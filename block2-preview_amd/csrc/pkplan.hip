@@ -2,17 +2,17 @@
 // plan, device upload, scratch and operator re-packing.
 //
 // Every GEMM operand of the split-BF16 kernels is a packed matrix (rows run
-// along the contraction index, row length K rounded up to 8, hi and lo BF16
-// planes; gemm_bf16x3.hip).  From the plan's chunks:
+// along the contraction index, K rounded up to 32, hi and lo BF16 values;
+// gemm_bf16x3.hip).  From the plan's chunks:
 //   * phase 1 (W = C op(B)): A = the packed wavefunction window C (c_m x c_n,
 //     packed per H*psi), B = the packed right-operator block in the
 //     orientation op(B)^T (v_n x c_n); the product is written as packed W^T
-//     (v_n x round8(c_m));
+//     (v_n x round32(c_m));
 //   * phase 2 (V += alpha op(A) W): A = the packed left-operator block in the
 //     orientation op(A) (v_m x c_m), B = packed W^T; the FP64 output tasks,
 //     split-K reductions and partial buffer are the plan's own.
-// A block read in both orientations is packed twice; operator planes cost
-// 4 bytes per packed element (half of the FP64 buffers they come from).
+// A block read in both orientations is packed twice; packed operators cost
+// 4 bytes per value (half of the FP64 buffers they come from).
 #include "common.hpp"
 #include "launch.hpp"
 #include "replay.hpp"
@@ -31,7 +31,11 @@ namespace b2g {
 
 namespace {
 
-uint64_t round8(uint64_t v) { return (v + 7) & ~(uint64_t)7; }
+uint64_t round32(uint64_t v) { return (v + 31) & ~(uint64_t)31; }
+// 128 rows of a packed matrix stay below 2^31 bytes
+bool pk_fits(uint64_t rows, uint64_t K) {
+    return rows * ((K + 7) & ~(uint64_t)7) < ((uint64_t)1 << 28);
+}
 
 // packed matrices of one source buffer, deduplicated by
 // (offset, row stride, orientation, rows, K)
@@ -66,8 +70,8 @@ struct Packer {
                          : (uint64_t)(rows - 1) * ld + (K - 1));
         if (last >= src_len)
             return -1;
-        const uint64_t pld = round8(K);
-        if ((uint64_t)rows * pld >= ((uint64_t)1 << 28))
+        const uint64_t pld = round32(K);
+        if (!pk_fits(rows, K))
             return -1;
         const uint64_t base = len;
         PackMat m;
@@ -82,7 +86,7 @@ struct Packer {
         m.g0 = ngroups;
         mats.push_back(m);
         ngroups += (uint64_t)rows * (pld / 8);
-        len += (uint64_t)rows * pld;
+        len += (uint64_t)rows * pld * 2;
         where.emplace(key, base);
         return (int64_t)base;
     }
@@ -117,12 +121,11 @@ static int pk_pack_ops(b2g_plan p, PkPlan *k) {
     const int grid = p->ctx->num_cu * 8;
     hipStream_t st = p->ctx->stream;
     __bf16 *op = (__bf16 *)k->op;
-    B2G_HIP(launch_pack_bf16((const double *)p->lbuf->ptr, op, op + k->l_len,
-                             k->d_lmats, k->n_lmats, k->n_lgroups, 0, 0, 1,
+    B2G_HIP(launch_pack_bf16((const double *)p->lbuf->ptr, op, k->d_lmats,
+                             k->n_lmats, k->n_lgroups, 0, 0, 1, grid, st));
+    B2G_HIP(launch_pack_bf16((const double *)p->rbuf->ptr, op + k->l_len,
+                             k->d_rmats, k->n_rmats, k->n_rgroups, 0, 0, 1,
                              grid, st));
-    B2G_HIP(launch_pack_bf16((const double *)p->rbuf->ptr, op + 2 * k->l_len,
-                             op + 2 * k->l_len + k->r_len, k->d_rmats,
-                             k->n_rmats, k->n_rgroups, 0, 0, 1, grid, st));
     return B2G_OK;
 }
 
@@ -176,9 +179,9 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
         for (size_t si = 0; si < ch.s1.size(); si++) {
             B2G_REQUIRE(m1[si] > 0 && n1[si] > 0, B2G_ERR_STATE,
                         "packed plan: phase-1 segment without a task");
-            const uint32_t ldw = (uint32_t)round8(m1[si]);
-            B2G_REQUIRE((uint64_t)n1[si] * ldw < ((uint64_t)1 << 28),
-                        B2G_ERR_ARG, "packed plan: W block of 2^28 elements");
+            const uint32_t ldw = (uint32_t)(2 * round32(m1[si]));
+            B2G_REQUIRE(pk_fits(n1[si], m1[si]), B2G_ERR_ARG,
+                        "packed plan: W block of 2^28 elements");
             wpk[si] = wlen;
             *wmap.emplace(w1[si], std::make_pair(wlen, ldw)).first =
                 std::make_pair(wlen, ldw);
@@ -218,7 +221,7 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
             for (size_t si = 0; si < ch.s2.size(); si++) {
                 const Seg &s = ch.s2[si];
                 const std::pair<uint64_t, uint32_t> *wp = wmap.find(s.b_off);
-                if (wp == nullptr || wp->second != round8(s.K)) {
+                if (wp == nullptr || wp->second != 2 * round32(s.K)) {
                     err[2] = "packed plan: phase-2 W not found";
                     return;
                 }
@@ -233,7 +236,7 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
                     return;
                 }
                 Seg q = s;
-                q.a_off = (uint64_t)a, q.lda = (uint32_t)round8(s.K);
+                q.a_off = (uint64_t)a, q.lda = (uint32_t)(2 * round32(s.K));
                 q.b_off = wp->first, q.ldb = wp->second;
                 q.flags = 0;
                 h.s2.push_back(q);
@@ -247,8 +250,8 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
                 for (const Tile &t :
                      tile_cover(m1[si], n1[si], ch.s1[si].K, 1))
                     h.t1[cfg_of(t)].push_back(make_task(
-                        wpk[si], (uint32_t)round8(m1[si]), m1[si], n1[si], t,
-                        (uint32_t)si, (uint32_t)si + 1, 0));
+                        wpk[si], (uint32_t)(2 * round32(m1[si])), m1[si],
+                        n1[si], t, (uint32_t)si, (uint32_t)si + 1, 0));
         });
         // output blocks re-tiled likewise, with split-K partial slots and
         // reductions of their own
@@ -263,8 +266,8 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
         h.s1.reserve(ch.s1.size());
         for (size_t si = 0; si < ch.s1.size(); si++) {
             Seg q = ch.s1[si];
-            q.a_off = (uint64_t)xa[si], q.lda = (uint32_t)round8(q.K);
-            q.b_off = (uint64_t)rb[si], q.ldb = (uint32_t)round8(q.K);
+            q.a_off = (uint64_t)xa[si], q.lda = (uint32_t)(2 * round32(q.K));
+            q.b_off = (uint64_t)rb[si], q.ldb = (uint32_t)(2 * round32(q.K));
             q.flags = 0, q.alpha = 1.0;
             h.s1.push_back(q);
         }
@@ -323,9 +326,9 @@ static int pk_build_into(b2g_plan p, PkPlan *k) {
         B2G_HIP(hipMemcpyAsync(k->dev, host, mat_bytes, hipMemcpyHostToDevice,
                                p->ctx->stream));
     B2G_HIP(p->ctx->alloc(&k->op,
-                          std::max<uint64_t>(2 * (k->l_len + k->r_len), 8) *
+                          std::max<uint64_t>(k->l_len + k->r_len, 64) *
                               sizeof(uint16_t)));
-    tm.mark("pack lists uploaded, planes allocated");
+    tm.mark("pack lists uploaded, operators allocated");
     {
         const int r = pk_pack_ops(p, k);
         if (r != B2G_OK) {
@@ -428,7 +431,7 @@ int pk_reserve(b2g_plan p, int n_rhs) {
         k->scratch = nullptr;
         k->scratch_rhs = 0;
     }
-    const size_t n = std::max<uint64_t>(2 * (k->x_len + k->w_max), 8) * n_rhs;
+    const size_t n = std::max<uint64_t>(k->x_len + k->w_max, 64) * n_rhs;
     B2G_HIP(p->ctx->alloc(&k->scratch, n * sizeof(uint16_t)));
     k->scratch_rhs = n_rhs;
     p->scratch_gen++;

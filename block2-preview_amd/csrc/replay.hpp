@@ -149,7 +149,8 @@ struct PkChunk {
 struct PkPlan {
     std::vector<PkChunk> chunks;
     void *dev = nullptr;     // task, segment and pack-tile arrays
-    uint16_t *op = nullptr;  // packed operator planes: L hi, L lo, R hi, R lo
+    // packed operators, L then R (lengths in elements, hi and lo counted)
+    uint16_t *op = nullptr;
     uint64_t l_len = 0, r_len = 0;
     // pack jobs: operator blocks (L, R) and wavefunction windows (X)
     PackMat *d_lmats = nullptr, *d_rmats = nullptr, *d_xmats = nullptr;
@@ -158,20 +159,13 @@ struct PkPlan {
     uint64_t x_len = 0; // packed wavefunction elements per right-hand side
     uint64_t w_max = 0; // packed W^T elements per right-hand side
     uint64_t p_max = 0; // split-K partial elements per right-hand side
-    // packed wavefunction and W^T planes for scratch_rhs right-hand sides:
-    // x hi, x lo (x_len * rhs each), W hi, W lo (w_max * rhs each)
+    // packed wavefunction and W^T for scratch_rhs right-hand sides
     uint16_t *scratch = nullptr;
     int scratch_rhs = 0;
-    const uint16_t *lh() const { return op; }
-    const uint16_t *ll() const { return op + l_len; }
-    const uint16_t *rh() const { return op + 2 * l_len; }
-    const uint16_t *rl() const { return op + 2 * l_len + r_len; }
-    uint16_t *xh() const { return scratch; }
-    uint16_t *xl() const { return scratch + x_len * scratch_rhs; }
-    uint16_t *wh() const { return scratch + 2 * x_len * scratch_rhs; }
-    uint16_t *wl() const {
-        return scratch + (2 * x_len + w_max) * scratch_rhs;
-    }
+    const uint16_t *l() const { return op; }
+    const uint16_t *r() const { return op + l_len; }
+    uint16_t *x() const { return scratch; }
+    uint16_t *w() const { return scratch + x_len * scratch_rhs; }
 };
 // build p->pk from the plan (packs the operator planes); no-op if built
 int pk_build(b2g_plan p);

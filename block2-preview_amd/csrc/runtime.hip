@@ -1635,8 +1635,8 @@ static int hpsi_run(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
     typedef const __bf16 *cbf;
     if (pk != nullptr)
         B2G_HIP(timed(B2G_K_PACK, ctx->stream, [&](hipStream_t st) {
-            return launch_pack_bf16(x, (__bf16 *)pk->xh(), (__bf16 *)pk->xl(),
-                                    pk->d_xmats, pk->n_xmats, pk->n_xgroups,
+            return launch_pack_bf16(x, (__bf16 *)pk->x(), pk->d_xmats,
+                                    pk->n_xmats, pk->n_xgroups,
                                     p->x_len,
                                     pk->x_len, n_rhs, grid, st);
         }));
@@ -1649,16 +1649,15 @@ static int hpsi_run(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
             B2G_HIP(phase(kc.n1, kc.f1, B2G_K_PHASE1,
                           [&](int c, hipStream_t st) {
                 return launch_seg_gemm_pk<0>(
-                    c, (cbf)pk->xh(), (cbf)pk->xl(), (cbf)pk->rh(),
-                    (cbf)pk->rl(), pk->wh(), pk->wl(), kc.d_t1[c],
+                    c, (cbf)pk->x(), (cbf)pk->r(), pk->w(), nullptr, kc.d_t1[c],
                     (int)kc.n1[c], kc.d_s1, pk->x_len, 0, pk->w_max, 0, 1.0,
                     0, n_rhs, grid, st, kc.x1[c]);
             }));
             B2G_HIP(phase(kc.n2, kc.f2, B2G_K_PHASE2,
                           [&](int c, hipStream_t st) {
                 return launch_seg_gemm_pk<1>(
-                    c, (cbf)pk->lh(), (cbf)pk->ll(), (cbf)pk->wh(),
-                    (cbf)pk->wl(), y, P, kc.d_t2[c], (int)kc.n2[c], kc.d_s2,
+                    c, (cbf)pk->l(), (cbf)pk->w(), y, P, kc.d_t2[c],
+                    (int)kc.n2[c], kc.d_s2,
                     0, pk->w_max, p->y_len, pstride, scale, beta0, n_rhs,
                     grid, st, kc.x2[c]);
             }));
