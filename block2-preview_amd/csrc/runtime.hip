@@ -631,24 +631,28 @@ void add_tiles(std::vector<Task> *tasks, uint64_t d_off, uint32_t M,
 // TM x TN slot of the partial buffer, and a reduction task sums the slots in
 // group order (deterministic) into the output.
 typedef std::vector<std::pair<uint32_t, uint32_t>> SegGroups;
-static SegGroups split_groups(const std::vector<Seg> &s2, const BlockJob &j,
-                              int table, uint64_t kmax) {
-    SegGroups groups;
+// The number of groups; the groups themselves where `groups` is given
+static size_t split_groups(const std::vector<Seg> &s2, const BlockJob &j,
+                           int table, uint64_t kmax,
+                           SegGroups *groups = nullptr) {
     // depth as the kernels walk it: every segment takes whole k-steps
     // (16 deep for the FP64 / FP32 kernels, 32 for the split-BF16 ones), so
     // that a long list of shallow segments is split like a deep one
     const uint64_t step = table == 1 ? 32 : 16;
     uint64_t acc = 0;
+    size_t n = 1;
     uint32_t g0 = j.sb;
-    for (uint32_t k = j.sb; k < j.se; k++) {
+    for (uint32_t k = j.sb; k + 1 < j.se; k++) {
         acc += (s2[k].K + step - 1) / step * step;
-        if (acc >= kmax && k + 1 < j.se) {
-            groups.emplace_back(g0, k + 1);
-            g0 = k + 1, acc = 0;
+        if (acc >= kmax) {
+            if (groups)
+                groups->emplace_back(g0, k + 1);
+            g0 = k + 1, acc = 0, n++;
         }
     }
-    groups.emplace_back(g0, j.se);
-    return groups;
+    if (groups)
+        groups->emplace_back(g0, j.se);
+    return n;
 }
 
 // partial elements of the jobs under the settings `v`
@@ -659,7 +663,7 @@ static uint64_t partial_len(const std::vector<Seg> &s2,
     t_env = v;
     uint64_t len = 0;
     for (const BlockJob &j : jobs) {
-        const size_t n = split_groups(s2, j, 0, v.ksplit).size();
+        const size_t n = split_groups(s2, j, 0, v.ksplit);
         if (n > 1)
             for (const Tile &t : tile_cover(j.M, j.N, 1, 0))
                 len += n * t.tm * t.tn;
@@ -671,15 +675,16 @@ static uint64_t partial_len(const std::vector<Seg> &s2,
 void add_split_tiles(const std::vector<Seg> &s2, const BlockJob &j, int table,
                      std::vector<Task> *t2, std::vector<RedTask> &red,
                      uint64_t &p_len) {
-    const SegGroups groups = split_groups(s2, j, table, t_env.ksplit);
     const std::vector<Tile> &tiles =
         tile_cover(j.M, j.N, 1, table);
-    if (groups.size() == 1) {
+    if (split_groups(s2, j, table, t_env.ksplit) == 1) {
         for (const Tile &t : tiles)
             t2[launch_of(t, table)].push_back(
                 make_task(j.d_off, j.ldd, j.M, j.N, t, j.sb, j.se, j.beta));
         return;
     }
+    SegGroups groups;
+    split_groups(s2, j, table, t_env.ksplit, &groups);
     for (const Tile &t : tiles) {
         const uint64_t tsz = (uint64_t)t.tm * t.tn;
         const uint64_t p0 = p_len;
