@@ -40,6 +40,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0,
                                              0x7FFFFFF0, 0x00020000);
 }
+// ... over no bytes: every load returns zero
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t empty_rsrc(const void *p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, 0,
+                                             0x00020000);
+}
 constexpr uint32_t kMasked = 0x80000000u; // offset past the record count
 
 // buffer load at byte offset off + soff (off past the record count: zero)
@@ -69,6 +74,17 @@ __device__ __forceinline__ float buf_load_s<float>(__amdgpu_buffer_rsrc_t r,
 // (a second chunk in flight gained nothing on tiles of up to 64 x 64, whose
 // four workgroups per compute unit cover the latency: n=26 M=1000 product
 // 407 us against 397 us).
+// The loads are issued one by one between the MFMAs of the chunk's first
+// k-step and the stores between those of its last, and fragments are read one
+// k-step ahead: between two barriers the matrix cores hardly wait for a
+// wave's other work.  (With the loads before and the stores after all MFMAs,
+// the two workgroups of a compute unit, in step with one another, left them
+// idle for 27 % of the 128 x 128 launches.  H*psi, n=40 M=3000, four
+// right-hand sides: 45.9 against 41.7 ms; M=2000 8.26 against 7.66 ms; n=26
+// M=1000 395 against 377 us, in FP32 with two right-hand sides 403 against
+// 398 us.  Vector arithmetic does hold up the FP64 MFMAs, about 12 cycles for
+// a multiplication and 3 for an integer operation; LDS and memory
+// instructions do not.)
 // Element q of thread tid is e = tid + 256 q; since 256 is a multiple of TK,
 // TM and TN, one coordinate of e is the same for all q and the other
 // advances by a constant.  Tasks are strided over the grid (persistent
@@ -86,33 +102,26 @@ struct TileRegs {
     TB rb[NB];
     uint32_t flags;
     double alpha;
-    // registers -> LDS buffer ([k][m] and [k][n] layouts), alpha applied;
-    // per layout, element q sits at a per-thread base plus a constant
+    // Registers -> LDS buffer ([k][m] and [k][n] layouts), alpha applied,
+    // without branches: element q at a per-thread base plus q times a stride
+    // that the operand's layout selects.  Not transposed, A has
+    // m = tid / TK + q * 256 / TK, k = tid % TK; transposed, m = tid % TM,
+    // k = tid / TM + q * 256 / TM; B the other way round.
     __device__ __forceinline__ void store(TC *As, TC *Bs, int tid) const {
         const bool ta = flags & 1, tb = (flags >> 1) & 1;
         const TC al = (TC)alpha;
-        if (!ta) { // m = tid / TK + q * 256 / TK, k = tid % TK
-            TC *p = As + (tid % TK) * (TM + 1) + tid / TK;
+        const int da = ta ? (256 / TM) * (TM + 1) : 256 / TK;
+        const int db = tb ? 256 / TK : (256 / TN) * (TN + 1);
+        TC *pa = As + (ta ? (tid / TM) * (TM + 1) + tid % TM
+                          : (tid % TK) * (TM + 1) + tid / TK);
+        TC *pb = Bs + (tb ? (tid % TK) * (TN + 1) + tid / TK
+                          : (tid / TN) * (TN + 1) + tid % TN);
 #pragma unroll
-            for (int q = 0; q < NA; q++)
-                p[q * (256 / TK)] = (TC)ra[q] * al;
-        } else { // m = tid % TM, k = tid / TM + q * 256 / TM
-            TC *p = As + (tid / TM) * (TM + 1) + tid % TM;
+        for (int q = 0; q < NA; q++)
+            pa[q * da] = (TC)ra[q] * al;
 #pragma unroll
-            for (int q = 0; q < NA; q++)
-                p[q * (256 / TM) * (TM + 1)] = (TC)ra[q] * al;
-        }
-        if (!tb) { // n = tid % TN, k = tid / TN + q * 256 / TN
-            TC *p = Bs + (tid / TN) * (TN + 1) + tid % TN;
-#pragma unroll
-            for (int q = 0; q < NB; q++)
-                p[q * (256 / TN) * (TN + 1)] = (TC)rb[q];
-        } else { // n = tid / TK + q * 256 / TK, k = tid % TK
-            TC *p = Bs + (tid % TK) * (TN + 1) + tid / TK;
-#pragma unroll
-            for (int q = 0; q < NB; q++)
-                p[q * (256 / TK)] = (TC)rb[q];
-        }
+        for (int q = 0; q < NB; q++)
+            pb[q * db] = (TC)rb[q];
     }
 };
 
@@ -200,40 +209,47 @@ struct TileLoader {
         sa = __builtin_amdgcn_readfirstlane(sa);
         sb = __builtin_amdgcn_readfirstlane(sb);
     }
-    // starts the loads of the current chunk into r and steps to the next
-    __device__ __forceinline__ void load(Regs &r, const Task &task, int tid) {
+    // The current chunk: begin() prepares its offsets, elements past K masked
+    // in place (a partial chunk is its segment's last, the next segment's
+    // offsets are computed anew); issue() starts its loads, without a branch,
+    // so that they can be placed among MFMAs (`any` false, no chunk left: the
+    // resources are empty); advance() steps to the next chunk.
+    __device__ __forceinline__ void begin(Regs &r, const Task &task, int tid) {
         if (k0 == 0)
             setup(task, tid);
-        const Seg &sg = cur;
-        r.flags = sg.flags;
-        r.alpha = sg.alpha;
-        const uint32_t soa = __builtin_amdgcn_readfirstlane(k0 * sa);
-        const uint32_t sob = __builtin_amdgcn_readfirstlane(k0 * sb);
-        if (k0 + TK <= sg.K) {
-#pragma unroll
-            for (int q = 0; q < NA; q++)
-                r.ra[q] = buf_load_s<TA>(rA, va[q], soa);
-#pragma unroll
-            for (int q = 0; q < NB; q++)
-                r.rb[q] = buf_load_s<TB>(rB, vb[q], sob);
-        } else {
-            // partial chunk: the k of element q, per storage order
-            const bool ta = sg.flags & 1, tb = (sg.flags >> 1) & 1;
+        r.flags = cur.flags;
+        r.alpha = cur.alpha;
+        if (k0 + TK > cur.K) {
+            const bool ta = cur.flags & 1, tb = (cur.flags >> 1) & 1;
 #pragma unroll
             for (int q = 0; q < NA; q++) {
                 const uint32_t k =
                     k0 + (ta ? tid / TM + q * (256 / TM) : tid % TK);
-                r.ra[q] = buf_load_s<TA>(rA, k < sg.K ? va[q] : kMasked, soa);
+                va[q] = k < cur.K ? va[q] : kMasked;
             }
 #pragma unroll
             for (int q = 0; q < NB; q++) {
                 const uint32_t k =
                     k0 + (tb ? tid % TK : tid / TN + q * (256 / TN));
-                r.rb[q] = buf_load_s<TB>(rB, k < sg.K ? vb[q] : kMasked, sob);
+                vb[q] = k < cur.K ? vb[q] : kMasked;
             }
         }
+    }
+    __device__ __forceinline__ void issue(Regs &r, bool any) {
+        const uint32_t soa = __builtin_amdgcn_readfirstlane(k0 * sa);
+        const uint32_t sob = __builtin_amdgcn_readfirstlane(k0 * sb);
+        const __amdgpu_buffer_rsrc_t qa = any ? rA : empty_rsrc(A);
+        const __amdgpu_buffer_rsrc_t qb = any ? rB : empty_rsrc(B);
+#pragma unroll
+        for (int q = 0; q < NA; q++)
+            r.ra[q] = buf_load_s<TA>(qa, va[q], soa);
+#pragma unroll
+        for (int q = 0; q < NB; q++)
+            r.rb[q] = buf_load_s<TB>(qb, vb[q], sob);
+    }
+    __device__ __forceinline__ void advance() {
         k0 += TK;
-        if (k0 >= sg.K) {
+        if (k0 >= cur.K) {
             k0 = 0;
             s++;
             cur = nxt;
@@ -265,18 +281,19 @@ __device__ __forceinline__ void seg_gemm_task(
 #pragma unroll
         for (int j = 0; j < FN; j++)
             acc[i][j] = acc_t{0, 0, 0, 0};
-    // MFMAs on one LDS buffer, fragment reads one k-step ahead
-    auto mac = [&](const TC *As) {
+    Loader ld(A, B, segs, task);
+    typename Loader::Regs r;
+    // MFMAs on one LDS buffer, fragment reads one k-step ahead; the next
+    // chunk's loads lie between the MFMAs of the first k-step, its stores to
+    // `fill` (released by the barrier that ended the previous chunk) between
+    // those of the last
+    auto mac = [&](const TC *As, TC *fill, bool more) {
+        constexpr int NM = FM * FN, NL = Loader::NA + Loader::NB;
+        constexpr int PER = (NL + NM - 1) / NM;
         const TC *Bs = As + ASZ;
         TC a[2][FM], b[2][FN];
 #pragma unroll
-        for (int i = 0; i < FM; i++)
-            a[0][i] = As[lk * (TM + 1) + wm * WM + i * 16 + lr];
-#pragma unroll
-        for (int j = 0; j < FN; j++)
-            b[0][j] = Bs[lk * (TN + 1) + wn * WN + j * 16 + lr];
-#pragma unroll
-        for (int ks = 0; ks < TK / 4; ks++) {
+        for (int ks = -1; ks < TK / 4; ks++) {
             const int cb = ks & 1, nb = cb ^ 1;
             if (ks + 1 < TK / 4) {
                 const int kr = (ks + 1) * 4 + lk;
@@ -287,30 +304,50 @@ __device__ __forceinline__ void seg_gemm_task(
                 for (int j = 0; j < FN; j++)
                     b[nb][j] = Bs[kr * (TN + 1) + wn * WN + j * 16 + lr];
             }
+            if (ks < 0)
+                continue;
+            __builtin_amdgcn_sched_barrier(0);
+            if (ks == 0)
+                ld.issue(r, more);
+            if (ks == TK / 4 - 1)
+                r.store(fill, fill + ASZ, tid);
 #pragma unroll
             for (int i = 0; i < FM; i++)
 #pragma unroll
                 for (int j = 0; j < FN; j++)
                     acc[i][j] = Mfma<TC>::op(a[cb][i], b[cb][j], acc[i][j]);
+            if (ks == 0) {
+#pragma unroll
+                for (int i = 0; i < NM; i++) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x20, PER, 0);
+                }
+            }
+            if (ks == TK / 4 - 1) {
+#pragma unroll
+                for (int i = 0; i < NM; i++) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x200, PER, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
-    Loader ld(A, B, segs, task);
     if (ld.more()) {
         TC *use = smem, *fill = smem + ASZ + BSZ;
-        typename Loader::Regs r;
-        ld.load(r, task, tid);
+        ld.begin(r, task, tid);
+        ld.issue(r, true);
+        ld.advance();
         r.store(use, use + ASZ, tid);
         __syncthreads();
         while (true) {
             const bool more = ld.more();
             if (more)
-                ld.load(r, task, tid);
-            mac(use);
+                ld.begin(r, task, tid);
+            mac(use, fill, more);
             if (!more)
                 break;
-            // `fill` was released by the barrier that ended the previous
-            // chunk
-            r.store(fill, fill + ASZ, tid);
+            ld.advance();
             TC *t = use;
             use = fill, fill = t;
             __syncthreads();
@@ -341,10 +378,11 @@ __device__ __forceinline__ void seg_gemm_task(
             }
 }
 
-// tiles with a side of 128: one launch per shape
+// tiles with a side of 128: one launch per shape (two workgroups per compute
+// unit: 240 VGPRs for 128 x 128 in FP64)
 template <typename TA, typename TB, typename TD, typename TC, int TM, int TN,
           int TK, int PHASE>
-__global__ __launch_bounds__(256) void seg_gemm_kernel(
+__global__ __launch_bounds__(256, 2) void seg_gemm_kernel(
     const TA *__restrict__ A, const TB *__restrict__ B, TD *__restrict__ D,
     TD *__restrict__ P, const Task *__restrict__ tasks, int ntasks,
     const Seg *__restrict__ segs, uint64_t a_rs, uint64_t b_rs, uint64_t d_rs,
