@@ -34,7 +34,7 @@ hipError_t launch_splitk_reduce(TD *D, const TD *P, const RedTask *tasks,
                                 uint64_t p_rs, int beta0, int n_rhs, int grid,
                                 hipStream_t st);
 
-// split-BF16 three-term variant on packed operand planes (gemm_bf16x3.hip):
+// split-BF16 three-term variant on packed operands (gemm_bf16x3.hip):
 // segments address packed A (M x lda) and packed B (N x ldb), both
 // k-contiguous; OUT 0 writes the packed transpose of the product (D0), OUT 1
 // writes FP64 D0 with split-K partials in D1

@@ -1,4 +1,4 @@
-// Split-BF16 replay on packed operand planes: derivation from the replay
+// Split-BF16 replay on packed operands: derivation from the replay
 // plan, device upload, scratch and operator re-packing.
 //
 // Every GEMM operand of the split-BF16 kernels is a packed matrix (rows run

@@ -72,10 +72,10 @@ struct b2g_plan_s {
     // use) and that plan
     std::vector<b2g_pair> pairs;
     b2g::GradPlan *grad = nullptr;
-    // the split-BF16 replay on packed operand planes (built on first use)
+    // the split-BF16 replay on packed operands (built on first use)
     b2g::PkPlan *pk = nullptr;
     // bumped whenever scratch that launches address (W, partials, packed
-    // planes) is reallocated: captured graphs of older generations are stale
+    // operands) is reallocated: captured graphs of older generations are stale
     uint64_t scratch_gen = 0;
 };
 
@@ -130,7 +130,7 @@ int plan_reserve(b2g_plan p, int n_rhs, int precision);
 // are written there, copied on the context stream and waited for)
 int ctx_stage(b2g_ctx ctx, size_t bytes, char **out);
 
-// Split-BF16 replay on packed operand planes (pkplan.hip).  Derived from the
+// Split-BF16 replay on packed operands (pkplan.hip).  Derived from the
 // plan's chunks: phase 1 reads the packed wavefunction windows and packed
 // right-operator blocks and writes packed W^T; phase 2 reads packed
 // left-operator blocks and packed W^T and keeps the FP64 tasks, split-K
@@ -167,11 +167,11 @@ struct PkPlan {
     uint16_t *x() const { return scratch; }
     uint16_t *w() const { return scratch + x_len * scratch_rhs; }
 };
-// build p->pk from the plan (packs the operator planes); no-op if built
+// build p->pk from the plan (packs the operators); no-op if built
 int pk_build(b2g_plan p);
 // packed scratch for n_rhs right-hand sides (grows only)
 int pk_reserve(b2g_plan p, int n_rhs);
-// re-pack the operator planes after the operator buffers changed
+// re-pack the operators after the operator buffers changed
 int pk_refresh(b2g_plan p);
 
 } // namespace b2g

@@ -1504,7 +1504,7 @@ int plan_reserve(b2g_plan p, int n_rhs, int precision) {
     const size_t es = precision == B2G_PREC_F64 ? 8 : 4;
     const size_t need = std::max<uint64_t>(p->w_max, 1) * n_rhs * es;
     if (precision == B2G_PREC_BF16X3) {
-        // packed planes replace the W scratch
+        // packed operands replace the W scratch
         int r = pk_build(p);
         if (r == B2G_OK)
             r = pk_reserve(p, n_rhs);
@@ -1553,7 +1553,7 @@ extern "C" int b2g_plan_reserve(b2g_plan p, int n_rhs, int precision) {
 namespace b2g {
 
 // One H*psi with the FP64 / FP32 W scratch at `W` and the split-K partials
-// at `P` (for split-BF16 the packed planes of the plan); allocates nothing
+// at `P` (for split-BF16 the packed operands of the plan); allocates nothing
 // itself.
 static int hpsi_run(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
                     int n_rhs, double scale, int accumulate, int precision,

@@ -152,18 +152,18 @@ typedef struct {
  * (FP64); x_len / y_len are the input/output vector lengths.  `flags` bit 0
  * or bit 1 also builds FP32 shadows of the operator buffers, which
  * B2G_PREC_F32 reads.  B2G_PREC_BF16X3 reads packed split-BF16 copies of the
- * operator blocks (hi + lo planes, 4 bytes per element, in the orientation
+ * operator blocks (hi and lo, 4 bytes per element, in the orientation
  * each pair uses), built on its first use or by b2g_plan_reserve.          */
 int b2g_upload_plan(b2g_ctx ctx, b2g_buf lbuf, b2g_buf rbuf,
                     const b2g_pair *pairs, size_t n_pairs,
                     const b2g_block *yblocks, size_t n_yblocks, size_t x_len,
                     size_t y_len, unsigned flags, b2g_plan *out);
 int b2g_plan_destroy(b2g_plan plan);
-/* Re-derive the plan's reduced-precision shadows and packed planes after
+/* Re-derive the plan's reduced-precision shadows and packed copies after
  * the operator buffers' contents changed (same structure, new numbers).   */
 int b2g_plan_refresh(b2g_plan plan);
 /* Allocate what b2g_hpsi needs for n_rhs right-hand sides at `precision`
- * (scratch, and the packed operator planes of B2G_PREC_BF16X3), so that a
+ * (scratch, and the packed operators of B2G_PREC_BF16X3), so that a
  * following b2g_hpsi allocates nothing (e.g. under stream capture).        */
 int b2g_plan_reserve(b2g_plan plan, int n_rhs, int precision);
 /* Reference-order work of one H*psi, in multiply-adds
@@ -227,7 +227,7 @@ int b2g_hpsi(b2g_ctx ctx, b2g_plan plan, const double *x, double *y,
  * the process ends) instead of plan-owned memory.  No counterpart in the
  * reference: for callers that cannot allocate (code under stream capture,
  * serving loops, harnesses that forbid hipMalloc).  FP64 and FP32 only
- * (split-BF16 reads packed planes the plan allocates); a product needing
+ * (split-BF16 reads packed copies the plan allocates); a product needing
  * more than 64 MiB for its W windows and the partials of a split into tasks
  * 2048 deep is refused (B2G_ERR_ARG).  Every call on one
  * device shares that array: calls that overlap on one device (other
