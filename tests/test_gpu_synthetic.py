@@ -118,3 +118,30 @@ def test_fp32(gpu_ctx, problem):
     y = run(gpu_ctx, pb, xs, {}, precision="f32")
     for r in range(4):
         assert rel(y[r], ys[r]) < 2e-6, r
+
+
+@pytest.fixture(scope="module")
+def small_blocks():
+    # blocks of 1 to 33: depths on both sides of a k-chunk (16) and of a
+    # packed line (32), most tiles partly outside their block
+    pb = synth.middle_site(n_orb=12, m=120, max_dim=33, seed=5)
+    xs = np.random.default_rng(4).standard_normal((3, pb.ket_len))
+    orc = O.Oracle(pb)
+    return pb, xs, np.stack([orc.hpsi(x, nthreads=8) for x in xs])
+
+
+@pytest.mark.parametrize("tile", ["auto", "32", "128"])
+@pytest.mark.parametrize("precision", ["f64", "f32", "bf16x3"])
+def test_chunk_edges(gpu_ctx, small_blocks, precision, tile):
+    # one and three right-hand sides (tasks dealt with their right-hand sides
+    # next to one another); a vector's result does not depend on the others.
+    # Tolerances as above (split-BF16: 2^-16 dropped per product, and sums)
+    pb, xs, ys = small_blocks
+    print(precision, "tile", tile, flush=True)
+    env = {} if tile == "auto" else {"B2G_TILE": tile}
+    y = run(gpu_ctx, pb, xs, env, precision=precision)
+    tol = {"f64": 1e-12, "f32": 2e-6, "bf16x3": 1e-4}[precision]
+    for r in range(3):
+        assert rel(y[r], ys[r]) < tol, r
+        one = run(gpu_ctx, pb, xs[r:r + 1], env, precision=precision)
+        assert np.array_equal(one[0], y[r]), r
