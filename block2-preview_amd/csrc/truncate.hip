@@ -64,13 +64,15 @@ static_assert((uint64_t)kMaxSyevOrder * kMaxSyevOrder < ((uint64_t)1 << 28) &&
                   kMaxSyevOrder % (2 * kJB) == 0,
               "kMaxSyevOrder");
 constexpr int kJLD = kJS + 1;
+constexpr int kMaxQrBlocks = 72; // orders above 1152: no QR step
 
 // one matrix of a batch: A and V are N x N (N = 32 nb) from a_off; the
 // round's Qs are nb / 2 matrices of 64 x 64 from q_off, their flags from
 // f_off
 struct JacBlock {
     uint64_t a_off, q_off;
-    uint32_t nb, n, f_off, pad;
+    uint32_t nb, n, f_off;
+    uint32_t qr;      // takes part in the QR step (jacobi_floor_kernel)
     double floor_abs; // off-diagonal entries below this are not rotated
 };
 // pair task (kind 0): x = pair index; region task (kind 1): x = row pair,
@@ -156,7 +158,12 @@ __global__ void jacobi_floor_kernel(JacBlock *__restrict__ blocks, int nblocks,
     double s = 0.0;
     for (int c = 0; c < nparts; c++)
         s += part[(size_t)b * nparts + c];
-    blocks[b].floor_abs = 64.0 * 2.220446049250313e-16 * sqrt(s);
+    const double f = 64.0 * 2.220446049250313e-16 * sqrt(s);
+    blocks[b].floor_abs = f;
+    // A matrix with an element that is not finite has no reflectors (0 * Inf
+    // and 0 * NaN would spread through all of V): it is iterated as it is,
+    // and since no entry exceeds its floor it rotates nothing, V = I.
+    blocks[b].qr = blocks[b].nb <= kMaxQrBlocks && isfinite(f);
 }
 
 // One kJS x kJS pair subproblem per workgroup: a cyclic Jacobi sweep in LDS;
@@ -496,7 +503,6 @@ __global__ __launch_bounds__(256) void jacobi_update_kernel(
 // |w|^2 = 2), H_1 .. H_16 = I - W T W^T with T^-1 = I + the strictly upper
 // part of W^T W.  W of column c sits in column c of H (rows >= c).
 constexpr int kQrWaves = 8;      // of a panel's workgroup
-constexpr int kMaxQrBlocks = 72; // orders above 1152 are iterated as they are
 
 // value of lane C of each row of 16 lanes
 template <int C> __device__ __forceinline__ double row_bcast(double v) {
@@ -589,7 +595,7 @@ __global__ __launch_bounds__(64 * kQrWaves) void qr_panel_kernel(
     double *__restrict__ H, double *__restrict__ T, int p) {
     __shared__ double red[2][kQrWaves][16], piv[2][16], G[16][17];
     const JacBlock bl = blocks[blockIdx.x];
-    if (p >= (int)bl.nb || bl.nb > kMaxQrBlocks)
+    if (p >= (int)bl.nb || !bl.qr)
         return;
     const int N = (int)bl.nb * kJB, c0 = p * kJB;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -645,7 +651,7 @@ __global__ __launch_bounds__(512) void qr_update_kernel(
     const JacBlock bl = blocks[blockIdx.y];
     const int N = (int)bl.nb * kJB, c0 = p * kJB;
     const int c1 = c0 + kJB + 32 * (int)blockIdx.x;
-    if (c1 >= N || bl.nb > kMaxQrBlocks)
+    if (c1 >= N || !bl.qr)
         return;
     const bool two = c1 + 16 < N;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -713,7 +719,7 @@ __global__ __launch_bounds__(512) void qr_update_kernel(
 // accumulator tile of S^T is the B operand of its own product).  Wave w
 // holds the column tiles w, w + 4, ...; one launch per range (lo, hi] of nb,
 // so that small matrices run with few registers.  Out: A1 (= R Q, symmetric, written
-// transposed) and V = Q; matrices too large for it are copied, V = I.
+// transposed) and V = Q; matrices it does not take are copied, V = I.
 template <int NT>
 __global__ __launch_bounds__(256) void qr_apply_kernel(
     const JacBlock *__restrict__ blocks, const double *__restrict__ A,
@@ -727,7 +733,7 @@ __global__ __launch_bounds__(256) void qr_apply_kernel(
     const bool ident = blockIdx.z == 1;
     if (i0 >= N || nb <= lo || nb > hi)
         return;
-    if (nb > kMaxQrBlocks) {
+    if (!bl.qr) {
         for (int e = tid; e < 16 * N; e += 256) {
             const uint64_t o = bl.a_off + (uint64_t)i0 * N + e;
             if (ident)
@@ -854,7 +860,8 @@ __global__ __launch_bounds__(256) void rayleigh_kernel(
 // One workgroup per eigenvector: out row j of matrix b = V column perm[j],
 // scaled to unit 2-norm (the accumulated rotations leave norms off by
 // O(sweeps * eps)) with the sign that makes its largest-magnitude
-// component positive (the first such component on ties).
+// component positive (the first such component on ties; of a column of NaN
+// the first component).
 struct VecJob {
     uint32_t blk, col;
     uint64_t dst; // row start in the output
@@ -868,7 +875,7 @@ __global__ __launch_bounds__(256) void eigvec_rows_kernel(
     const JacBlock bl = blocks[jb.blk];
     const uint32_t N = bl.nb * kJB;
     double best = -1.0, ss = 0.0;
-    int bi = 0x7FFFFFFF;
+    int bi = 0; // a row of the matrix in any case
     for (uint32_t i = threadIdx.x; i < bl.n; i += 256) {
         const double v = V[bl.a_off + (uint64_t)i * N + jb.col];
         ss = fma(v, v, ss);
@@ -1095,7 +1102,7 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
         b.a_off = s.a_len;
         b.q_off = s.q_len;
         b.f_off = (uint32_t)s.f_len;
-        b.pad = 0;
+        b.qr = 0;
         b.floor_abs = 0.0;
         s.a_len += N * N;
         s.q_len += (uint64_t)(b.nb / 2) * kJS * kJS;

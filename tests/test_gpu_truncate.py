@@ -130,6 +130,34 @@ def test_syev_batched_orders(gpu_ctx, sizes):
         assert np.abs(v @ v.T - np.eye(len(w))).max() < 1e-11, len(w)
 
 
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("n", [1, 17, 100, 300, 1153])
+def test_syev_batched_not_finite(gpu_ctx, n, bad):
+    # a matrix with one element that is not finite rotates nothing: its
+    # vectors are the unit vectors and its values are not finite.  The other
+    # matrices of the batch are solved as ever (tolerances as above)
+    rng = np.random.default_rng(n)
+    mats = []
+    for k in (33, n, 64, n):
+        a = rng.standard_normal((k, k))
+        mats.append((a + a.T) / 2)
+    i, j = n // 2, n // 3
+    mats[1][i, j] = mats[1][j, i] = bad
+    mats[3][n - 1, n - 1] = bad
+    print("order", n, "element", bad, flush=True)
+    ws, vs, _ = TR.eigh_batched(gpu_ctx, [dev(m) for m in mats])
+    for b, (a, w, v) in enumerate(zip(mats, ws, vs)):
+        w, v = w.cpu().numpy(), v.cpu().numpy()
+        if b % 2:
+            assert not np.isfinite(w).any(), b
+            assert np.array_equal(v, np.eye(n)), b
+        else:
+            wn = np.linalg.eigvalsh(a)
+            nrm = np.abs(wn).max()
+            assert np.abs(w - wn).max() < 1e-12 * nrm, b
+            assert np.abs(a @ v.T - v.T * w).max() < 1e-11 * nrm, b
+
+
 def test_syev_batched_repeatable(gpu_ctx):
     mats = [dev(m) for _, m in sym_mats()]
     w1, v1, _ = TR.eigh_batched(gpu_ctx, mats)
