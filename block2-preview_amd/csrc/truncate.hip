@@ -74,7 +74,10 @@ struct JacBlock {
     uint32_t nb, n, f_off;
     uint32_t qr;      // takes part in the QR step (jacobi_floor_kernel)
     double floor_abs; // off-diagonal entries below this are not rotated
+    // largest |a_ij| of the matrix, as bits (of NaN: above those of Inf)
+    unsigned long long amax;
 };
+static_assert(sizeof(unsigned long long) == sizeof(double), "bits of amax");
 // pair task (kind 0): x = pair index; region task (kind 1): x = row pair,
 // y = column pair; V task (kind 2): x = pair, y = slice of kJS rows
 struct JacTask {
@@ -102,40 +105,56 @@ __device__ __forceinline__ int pair_index(int bi, int bj, int l) {
     return l < kJB ? bi * kJB + l : bj * kJB + (l - kJB);
 }
 
-// A: padded copy of the compact symmetric matrices, V = I
+// A: padded copy of the compact symmetric matrices, V = I, amax (0 before)
 __global__ __launch_bounds__(256) void jacobi_init_kernel(
-    const JacBlock *__restrict__ blocks, int nblocks,
+    JacBlock *__restrict__ blocks, int nblocks,
     const uint64_t *__restrict__ src_off, const double *__restrict__ src,
     double *__restrict__ A, double *__restrict__ V) {
     for (int b = blockIdx.y; b < nblocks; b += gridDim.y) {
         const JacBlock bl = blocks[b];
         const uint32_t N = bl.nb * kJB;
         const uint64_t NN = (uint64_t)N * N;
+        unsigned long long top = 0;
         for (uint64_t e = blockIdx.x * 256ull + threadIdx.x; e < NN;
              e += (uint64_t)gridDim.x * 256) {
             const uint32_t i = (uint32_t)(e / N), j = (uint32_t)(e % N);
-            A[bl.a_off + e] =
+            const double a =
                 (i < bl.n && j < bl.n) ? src[src_off[b] + (uint64_t)i * bl.n + j]
                                        : 0.0;
+            A[bl.a_off + e] = a;
             V[bl.a_off + e] = i == j ? 1.0 : 0.0;
+            top = max(top, __builtin_bit_cast(unsigned long long, fabs(a)));
         }
+        for (int w = 32; w > 0; w >>= 1)
+            top = max(top, __shfl_xor(top, w));
+        if ((threadIdx.x & 63) == 0 && top != 0)
+            atomicMax(&blocks[b].amax, top);
     }
 }
 
-// floor_abs of each matrix: 64 eps ||A_b||_F.  Stage 1: workgroup
-// (chunk, b) sums the squares of rows chunk, chunk + gridDim.x, ... of
-// matrix b into part[b * gridDim.x + chunk]; stage 2 (jacobi_floor_kernel)
-// adds the parts of each matrix in order (deterministic).
+// Each matrix is scaled by the power of two that brings its largest element
+// into [1, 2), so that the squares which norms, reflectors and rotations
+// take of its elements neither overflow nor vanish (unscaled, norms below
+// 1e-153 counted as zero and above 6e153 as infinite); the eigenvectors are
+// those of A and the eigenvalues are taken from A itself (rayleigh_kernel).
+// Then floor_abs: 64 eps ||A_b||_F.  Stage 1: workgroup (chunk, b) scales and
+// sums the squares of rows chunk, chunk + gridDim.x, ... of matrix b into
+// part[b * gridDim.x + chunk]; stage 2 (jacobi_floor_kernel) adds the parts
+// of each matrix in order (deterministic).
 __global__ __launch_bounds__(256) void jacobi_norm_kernel(
-    const JacBlock *__restrict__ blocks, const double *__restrict__ A,
+    const JacBlock *__restrict__ blocks, double *__restrict__ A,
     double *__restrict__ part) {
     __shared__ double sh[256];
     const JacBlock bl = blocks[blockIdx.y];
     const uint32_t N = bl.nb * kJB;
+    const double amax = __builtin_bit_cast(double, bl.amax);
+    const int sc = amax > 0.0 && isfinite(amax) ? -ilogb(amax) : 0;
     double s = 0.0;
     for (uint32_t i = blockIdx.x; i < N; i += gridDim.x)
         for (uint32_t j = threadIdx.x; j < N; j += 256) {
-            const double v = A[bl.a_off + (uint64_t)i * N + j];
+            double *a = A + bl.a_off + (uint64_t)i * N + j;
+            const double v = ldexp(*a, sc);
+            *a = v;
             s = fma(v, v, s);
         }
     sh[threadIdx.x] = s;
@@ -1104,6 +1123,7 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
         b.f_off = (uint32_t)s.f_len;
         b.qr = 0;
         b.floor_abs = 0.0;
+        b.amax = 0;
         s.a_len += N * N;
         s.q_len += (uint64_t)(b.nb / 2) * kJS * kJS;
         s.f_len += b.nb / 2;

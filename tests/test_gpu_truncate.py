@@ -158,6 +158,28 @@ def test_syev_batched_not_finite(gpu_ctx, n, bad):
             assert np.abs(a @ v.T - v.T * w).max() < 1e-11 * nrm, b
 
 
+@pytest.mark.parametrize("power", [-1000, -530, -400, 400, 508, 515, 1000])
+def test_syev_batched_scale(gpu_ctx, power):
+    # a power of two in front changes neither the vectors nor, but for the
+    # factor, the values; the squares of these elements over- or underflow
+    # (2^508: only those of their differences)
+    rng = np.random.default_rng(4)
+    mats = []
+    for n in (1, 20, 100, 300, 1153):
+        a = rng.standard_normal((n, n))
+        mats.append((a + a.T) / 2)
+    print("2 ^", power, flush=True)
+    w1, v1, _ = TR.eigh_batched(gpu_ctx, [dev(m) for m in mats])
+    w2, v2, _ = TR.eigh_batched(gpu_ctx, [dev(m * 2.0 ** power)
+                                          for m in mats])
+    for a, b in zip(v1, v2):
+        assert torch.equal(a, b), len(a)
+    for a, b in zip(w1, w2):
+        # products with the smallest vector elements may round as denormals
+        a, b = a.cpu().numpy(), b.cpu().numpy() * 2.0 ** -power
+        assert np.abs(a - b).max() <= 1e-14 * np.abs(a).max(), len(a)
+
+
 def test_syev_batched_repeatable(gpu_ctx):
     mats = [dev(m) for _, m in sym_mats()]
     w1, v1, _ = TR.eigh_batched(gpu_ctx, mats)
