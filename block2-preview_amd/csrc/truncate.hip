@@ -45,6 +45,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <limits>
 #include <memory>
 #include <numeric>
 #include <random>
@@ -1297,7 +1298,11 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
         std::vector<std::pair<double, uint32_t>> o(n[i]);
         for (uint32_t j = 0; j < n[i]; j++)
             o[j] = std::make_pair(w[s.w_off[i] + j], j);
-        std::sort(o.begin(), o.end());
+        // values with a NaN among them have no order: left in place (comparing
+        // it, std::sort may leave its range)
+        if (std::none_of(o.begin(), o.end(),
+                         [](const auto &x) { return std::isnan(x.first); }))
+            std::sort(o.begin(), o.end());
         for (uint32_t j = 0; j < n[i]; j++) {
             w_sorted[s.w_off[i] + j] = o[j].first;
             jobs.push_back(VecJob{(uint32_t)i, o[j].second,
@@ -1752,9 +1757,15 @@ static int split_impl(b2g_ctx ctx, int symmetry, const b2g_sparse_info *wfn,
     };
     double error = 0.0;
     if (k != -1) {
+        // NaN as +Inf (comparing it, std::sort may leave its range): states of
+        // a block that is not finite are kept, so that they show in the result
+        auto rank = [&](const std::pair<int, int> &x) {
+            const double v = wrv(x);
+            return std::isnan(v) ? std::numeric_limits<double>::infinity() : v;
+        };
         std::sort(ss.begin(), ss.end(),
                   [&](const std::pair<int, int> &a, const std::pair<int, int> &b) {
-                      return wrv(a) > wrv(b);
+                      return rank(a) > rank(b);
                   });
         const unsigned keep = trunc_type / 16u;
         if (keep == 0) {

@@ -40,6 +40,7 @@ import torch
 import truncate_oracle as T
 from conftest import FIXTURES, DELAYED_FIXTURES, fixture_path
 
+from b2g import synth
 from b2g import truncate as TR
 from sweep_common import (SWEEP_SPLIT_CASES, load_sweep_split,
                           sweep_split_fixtures)
@@ -195,6 +196,35 @@ def load(name):
     info = TR.BlockInfo(z["ket_quanta"], z["ket_nbra"], z["ket_nket"],
                         z["ket_shift"], int(z["ket_dq"][0]))
     return z, sym, info
+
+
+@pytest.mark.parametrize("tr", [True, False])
+def test_split_not_finite(gpu_ctx, tr):
+    # one NaN in the wavefunction: the weights of its sector are NaN and
+    # rank first, the other sectors' are as without it (1e-12: as the
+    # eigenvalues above), and as many states are kept as asked for
+    pb = synth.middle_site(n_orb=12, m=200, max_dim=80, seed=5)
+    k = pb.ket
+    info = TR.BlockInfo(k.quanta, k.nbra, k.nket, k.shift, int(k.dq[0]))
+    x = np.random.default_rng(8).standard_normal(pb.ket_len)
+    x /= np.linalg.norm(x)
+    y = x.copy()
+    b = int(np.argmax(info.nbra))
+    info.block(y, b)[0, 0] = np.nan
+    print("trace right", tr, flush=True)
+    a, c = (TR.split_density_matrix(gpu_ctx, T.SU2, info, dev(v), 150,
+                                    trace_right=tr) for v in (x, y))
+    dm = a.dm[0]
+    o = np.concatenate([[0], np.cumsum(dm.nbra.astype(int))])
+    nan = np.isnan(c.eigvals)
+    (i,) = {int(np.searchsorted(o, p, "right")) - 1
+            for p in np.flatnonzero(nan)}
+    assert nan.sum() == dm.nbra[i] == (info.nbra if tr else info.nket)[b]
+    assert np.abs(c.eigvals - a.eigvals)[~nan].max() <= 1e-12
+    r = c.left[0] if tr else c.right[0]
+    kept = dict(zip(r.quanta.tolist(), r.nket if tr else r.nbra))
+    assert sum(kept.values()) == 150
+    assert kept[int(dm.quanta[i])] == dm.nbra[i]
 
 
 def part_blocks(bi, data):
