@@ -1627,10 +1627,17 @@ static int hpsi_run(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
             e = timed(kbase + c, st,
                       [&](hipStream_t s) { return launch(c, s); });
         }
-        for (int i = 0; e == hipSuccess && i < naux; i++) {
-            e = hipEventRecord(ctx->join[i], ctx->aux[i]);
+        // joined after an error as well: the launches before it still use the
+        // plan's blocks, which are given back to the context once its own
+        // stream is done
+        for (int i = 0; i < naux; i++) {
+            hipError_t j = hipEventRecord(ctx->join[i], ctx->aux[i]);
+            if (j == hipSuccess)
+                j = hipStreamWaitEvent(ctx->stream, ctx->join[i], 0);
+            if (j != hipSuccess)
+                (void)hipStreamSynchronize(ctx->aux[i]);
             if (e == hipSuccess)
-                e = hipStreamWaitEvent(ctx->stream, ctx->join[i], 0);
+                e = j;
         }
         return e;
     };
