@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
+#include <atomic>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -216,5 +217,7 @@ struct b2g_buf_s {
     size_t n = 0;
     int dtype = B2G_F64;
     bool owned = true; // false: a view of memory it must not free
-    bool shown = false; // the caller has its address: may use it on any stream
+    // used outside its context's stream: the caller has its address, or another
+    // context's plan reads it
+    std::atomic<bool> shown{false};
 };

@@ -313,6 +313,7 @@ extern "C" int b2g_grad_ops(b2g_ctx ctx, b2g_plan p, const double *v,
     B2G_REQUIRE(ctx && p && v && c && gl && gr, B2G_ERR_ARG, "NULL arg");
     B2G_REQUIRE(n_rhs >= 1, B2G_ERR_ARG, "bad n_rhs");
     B2G_HIP(hipSetDevice(ctx->device));
+    B2G_HIP(plan_launched_by(p, ctx));
     if (p->grad == nullptr) {
         const int r = grad_plan_build(p, &p->grad);
         if (r != B2G_OK)

@@ -426,13 +426,14 @@ int pk_reserve(b2g_plan p, int n_rhs) {
     if (n_rhs <= k->scratch_rhs)
         return B2G_OK;
     if (k->scratch) {
-        B2G_HIP(hipStreamSynchronize(p->ctx->stream));
+        B2G_HIP(plan_wait(p));
         p->ctx->pool.put(k->scratch);
         k->scratch = nullptr;
         k->scratch_rhs = 0;
     }
     const size_t n = std::max<uint64_t>(k->x_len + k->w_max, 64) * n_rhs;
     B2G_HIP(p->ctx->alloc(&k->scratch, n * sizeof(uint16_t)));
+    B2G_HIP(plan_publish(p));
     k->scratch_rhs = n_rhs;
     p->scratch_gen++;
     return B2G_OK;

@@ -5,6 +5,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 
+#include <atomic>
 #include <vector>
 
 namespace b2g {
@@ -77,6 +78,9 @@ struct b2g_plan_s {
     // bumped whenever scratch that launches address (W, partials, packed
     // operands) is reallocated: captured graphs of older generations are stale
     uint64_t scratch_gen = 0;
+    // launched by another context too: its blocks may be in use outside this
+    // one's stream
+    std::atomic<bool> elsewhere{false};
 };
 
 
@@ -126,6 +130,14 @@ XcdSplit xcd_order(std::vector<Task> &tasks, const std::vector<Seg> &segs,
 uint64_t w_cap_elems();
 // allocate the H*psi scratch for n_rhs at precision ahead of a capture
 int plan_reserve(b2g_plan p, int n_rhs, int precision);
+// A plan may be launched by another context (b2g_hpsi, b2g_grad_ops) than the
+// one its blocks come from.  plan_launched_by notes that; plan_publish, for
+// blocks just taken from the pool, waits for what their last user may still
+// have under way on this context's stream; plan_wait waits for the work on
+// the plan's blocks before they are given back.
+hipError_t plan_launched_by(b2g_plan p, b2g_ctx ctx);
+hipError_t plan_publish(b2g_plan p);
+hipError_t plan_wait(b2g_plan p);
 // the context's pinned staging buffer, at least `bytes` long (host uploads
 // are written there, copied on the context stream and waited for)
 int ctx_stage(b2g_ctx ctx, size_t bytes, char **out);

@@ -326,7 +326,7 @@ extern "C" int b2g_buf_destroy(b2g_buf buf) {
     if (buf == nullptr)
         return B2G_OK;
     hipSetDevice(buf->ctx->device);
-    if (buf->shown) // the caller may have used it on streams of its own
+    if (buf->shown)
         hipDeviceSynchronize();
     else
         hipStreamSynchronize(buf->ctx->stream);
@@ -392,8 +392,9 @@ extern "C" int b2g_upload_blocks(b2g_ctx ctx, const void *host, size_t n,
 }
 
 extern "C" void *b2g_buf_device_ptr(b2g_buf buf) {
-    if (buf)
-        buf->shown = true;
+    // its block may have work of its last user under way on the stream
+    if (buf && !buf->shown.exchange(true))
+        (void)hipStreamSynchronize(buf->ctx->stream);
     return buf ? buf->ptr : nullptr;
 }
 extern "C" size_t b2g_buf_size(b2g_buf buf) { return buf ? buf->n : 0; }
@@ -1319,6 +1320,7 @@ extern "C" int b2g_upload_plan(b2g_ctx ctx, b2g_buf lbuf, b2g_buf rbuf,
     p->ctx = ctx;
     p->lbuf = lbuf;
     p->rbuf = rbuf;
+    (void)plan_launched_by(p, ctx);
     p->x_len = x_len;
     p->y_len = y_len;
     p->flags = flags;
@@ -1365,7 +1367,7 @@ extern "C" int b2g_plan_destroy(b2g_plan p) {
     if (p == nullptr)
         return B2G_OK;
     hipSetDevice(p->ctx->device);
-    hipStreamSynchronize(p->ctx->stream);
+    (void)plan_wait(p);
     for (auto &st : p->stamps) {
         hipEventDestroy(st.start);
         hipEventDestroy(st.stop);
@@ -1497,6 +1499,21 @@ extern "C" int b2g_plan_stats(b2g_plan p, uint64_t *n1, uint64_t *n2,
 
 namespace b2g {
 
+hipError_t plan_wait(b2g_plan p) {
+    return p->elsewhere ? hipDeviceSynchronize()
+                        : hipStreamSynchronize(p->ctx->stream);
+}
+hipError_t plan_publish(b2g_plan p) {
+    return p->elsewhere ? hipStreamSynchronize(p->ctx->stream) : hipSuccess;
+}
+hipError_t plan_launched_by(b2g_plan p, b2g_ctx ctx) {
+    for (b2g_buf b : {p->lbuf, p->rbuf})
+        if (b->ctx != ctx)
+            b->shown = true;
+    return p->ctx != ctx && !p->elsewhere.exchange(true) ? plan_publish(p)
+                                                         : hipSuccess;
+}
+
 // scratch (W, split-K partials) for n_rhs right-hand sides at `precision`;
 // reallocates only when growing (not allowed while a stream is captured)
 int plan_reserve(b2g_plan p, int n_rhs, int precision) {
@@ -1512,12 +1529,13 @@ int plan_reserve(b2g_plan p, int n_rhs, int precision) {
             return r;
     } else if (need > p->w_bytes) {
         if (p->w) {
-            B2G_HIP(hipStreamSynchronize(ctx->stream));
+            B2G_HIP(plan_wait(p));
             ctx->pool.put(p->w);
             p->w = nullptr;
             p->w_bytes = 0;
         }
         B2G_HIP(ctx->alloc(&p->w, need));
+        B2G_HIP(plan_publish(p));
         p->w_bytes = need;
         p->scratch_gen++;
     }
@@ -1526,12 +1544,13 @@ int plan_reserve(b2g_plan p, int n_rhs, int precision) {
     const size_t pneed = std::max<uint64_t>(pmax, 1) * n_rhs * 8;
     if (pneed > p->p_bytes) {
         if (p->pbuf) {
-            B2G_HIP(hipStreamSynchronize(ctx->stream));
+            B2G_HIP(plan_wait(p));
             ctx->pool.put(p->pbuf);
             p->pbuf = nullptr;
             p->p_bytes = 0;
         }
         B2G_HIP(ctx->alloc(&p->pbuf, pneed));
+        B2G_HIP(plan_publish(p));
         p->p_bytes = pneed;
         p->scratch_gen++;
     }
@@ -1733,6 +1752,7 @@ extern "C" int b2g_hpsi(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
     B2G_REQUIRE(precision != B2G_PREC_F32 || p->l32 != nullptr, B2G_ERR_STATE,
                 "plan was uploaded without FP32 shadows (flags bit 0 or 1)");
     B2G_HIP(hipSetDevice(ctx->device));
+    B2G_HIP(plan_launched_by(p, ctx));
     {
         const int r = plan_reserve(p, n_rhs, precision);
         if (r != B2G_OK)

@@ -71,6 +71,58 @@ def test_two_threads(gpu_ctx):
     assert not bad, bad
 
 
+@pytest.mark.parametrize("entry", ["f64", "f32", "bf16x3", "grad"])
+def test_plan_launched_by_another_context(gpu_ctx, entry):
+    # products (gradients) of one context's plan queued on another's stream;
+    # the plan and its operators are destroyed while they run, and the first
+    # context makes and solves other sites on the blocks they had
+    print("entry", entry, flush=True)
+    a, b = Context(0), Context(0)
+    n_orb, m, dim, seed = SITES[2]
+    pb = synth.middle_site(n_orb=n_orb, m=m, max_dim=dim, seed=seed)
+    g = torch.Generator(device="cuda:0").manual_seed(1)
+    x = torch.randn((8, pb.ket_len), generator=g, dtype=torch.float64,
+                    device="cuda:0")
+
+    def run(ctx, h, out):
+        if entry == "grad":
+            L.check(ctx.lib.b2g_grad_ops(
+                ctx.h, h.plan, x.data_ptr(), x.data_ptr(), len(x),
+                out[0].data_ptr(), out[1].data_ptr(), 0))
+        else:
+            L.check(ctx.lib.b2g_hpsi(
+                ctx.h, h.plan, x.data_ptr(), out[0].data_ptr(), len(x), 1.0,
+                0, L.PREC[entry]))
+
+    def outputs():
+        if entry == "grad":
+            return [torch.empty(n, dtype=torch.float64, device="cuda:0")
+                    for n in pb.data_len.values()]
+        return [torch.empty_like(x)]
+
+    def make():
+        return EffectiveHamiltonian(pb, a, fp32=entry == "f32")
+
+    h = make()
+    want, got = outputs(), [outputs() for _ in range(8)]
+    torch.cuda.synchronize()
+    run(a, h, want)
+    a.synchronize()
+    h.deallocate()
+    for _ in range(3):
+        h = make()
+        for o in got:
+            run(b, h, o)
+        h.deallocate()
+        for s in SITES:
+            site(a, s)
+    b.synchronize()
+    for o in got:
+        assert same(o, want)
+    a.close()
+    b.close()
+
+
 def test_trim_gives_back(gpu_ctx):
     ctx = Context(0)
     torch.cuda.synchronize()
