@@ -153,14 +153,15 @@ class SetupTimer {
 // the work between them.  A block is put back only once the work on it is
 // done or is ordered before any later work on the context's stream.  Kept:
 // at most kPoolCap bytes, oldest given back first; all of it when less than a
-// quarter of the device is free, when an allocation fails, and by trim().
+// quarter of the device is free, when an allocation of any context on the
+// device fails, and by trim().
 // Safe to call from several threads.  A fresh n=28 M=1000 site (setup and
 // FP64 Davidson) takes 5.2 ms, 15 to 36 ms with hipMalloc and hipFree (box to
 // box); the n=40 M=3000 truncation 11.0 against 14.1 ms.
 class BlockPool {
   public:
-    explicit BlockPool(bool pinned) : pinned_(pinned) {}
-    ~BlockPool() { trim(); }
+    BlockPool(bool pinned, int device);
+    ~BlockPool();
     hipError_t get(size_t bytes, void **out);
     void put(void *p); // nullptr: nothing
     void trim();
@@ -169,6 +170,7 @@ class BlockPool {
     hipError_t make(size_t bytes, void **out);
     void drop(void *p);
     const bool pinned_;
+    const int device_;
     std::mutex m_;
     std::vector<std::pair<size_t, void *>> free_; // oldest first
     std::unordered_map<void *, size_t> size_;     // of every block handed out
@@ -178,7 +180,7 @@ class BlockPool {
 } // namespace b2g
 
 struct b2g_ctx_s {
-    int device = 0;
+    const int device;
     int num_cu = 0;
     hipStream_t stream = nullptr;
     // auxiliary streams (default priority) for the independent launches of
@@ -194,7 +196,9 @@ struct b2g_ctx_s {
     // upload waits for its copy before returning)
     char *stage = nullptr;
     size_t stage_len = 0;
-    b2g::BlockPool pool{false}, pinned{true};
+    b2g::BlockPool pool, pinned;
+    explicit b2g_ctx_s(int dev)
+        : device(dev), pool(false, dev), pinned(true, dev) {}
     template <typename T> hipError_t alloc(T **out, size_t bytes) {
         return pool.get(bytes, (void **)out);
     }

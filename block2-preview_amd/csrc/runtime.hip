@@ -69,6 +69,24 @@ static int scratch_setup(int device) {
 // ------------------------------------------------------------- block pool
 constexpr size_t kPoolCap = (size_t)16 << 30;
 
+// every pool of the process (never destroyed: a context may outlive the
+// program's static objects); the lock is taken before a pool's
+static std::mutex g_pools_mu;
+static std::vector<BlockPool *> &g_pools = *new std::vector<BlockPool *>();
+
+BlockPool::BlockPool(bool pinned, int device)
+    : pinned_(pinned), device_(device) {
+    std::lock_guard<std::mutex> all(g_pools_mu);
+    g_pools.push_back(this);
+}
+BlockPool::~BlockPool() {
+    {
+        std::lock_guard<std::mutex> all(g_pools_mu);
+        g_pools.erase(std::find(g_pools.begin(), g_pools.end(), this));
+    }
+    trim();
+}
+
 hipError_t BlockPool::make(size_t bytes, void **out) {
     return pinned_ ? hipHostMalloc(out, bytes) : hipMalloc(out, bytes);
 }
@@ -84,7 +102,7 @@ hipError_t BlockPool::get(size_t bytes, void **out) {
     // whole 4 KiB or 2 MiB, so that nearly equal requests share blocks
     const size_t unit = bytes <= ((size_t)1 << 20) ? 4096 : (size_t)2 << 20;
     const size_t n = (std::max<size_t>(bytes, 1) + unit - 1) / unit * unit;
-    std::lock_guard<std::mutex> lock(m_);
+    std::unique_lock<std::mutex> lock(m_);
     size_t best = free_.size();
     for (size_t i = 0; i < free_.size(); i++)
         if (free_[i].first >= n && free_[i].first <= n + n / 4 + unit &&
@@ -98,15 +116,23 @@ hipError_t BlockPool::get(size_t bytes, void **out) {
         free_.erase(free_.begin() + best);
     } else {
         hipError_t e = make(n, out);
-        if (e != hipSuccess && !free_.empty()) {
+        if (e != hipSuccess) {
+            // what any context keeps on this device (one pool's lock at a
+            // time: two pools may be here at once)
             (void)hipGetLastError();
-            for (auto &b : free_)
-                drop(b.second);
-            free_.clear();
-            kept_ = 0;
+            lock.unlock();
+            {
+                std::lock_guard<std::mutex> all(g_pools_mu);
+                for (BlockPool *q : g_pools)
+                    if (q->pinned_ == pinned_ && q->device_ == device_)
+                        q->trim();
+            }
+            lock.lock();
             e = make(n, out);
         }
         if (e != hipSuccess) {
+            // (reported here: not again after the next launch)
+            (void)hipGetLastError();
             *out = nullptr;
             return e;
         }
@@ -186,8 +212,7 @@ extern "C" int b2g_ctx_create(int device, unsigned flags, b2g_ctx *out) {
         if (r != B2G_OK)
             return r;
     }
-    b2g_ctx c = new b2g_ctx_s();
-    c->device = device;
+    b2g_ctx c = new b2g_ctx_s(device);
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) != hipSuccess) {
         delete c;

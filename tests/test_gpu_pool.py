@@ -2,6 +2,7 @@
 truncations on reused (dirty) blocks equal those on fresh ones bit for bit,
 two threads with a context each do not disturb one another, and trim() gives
 the kept memory back."""
+import ctypes as C
 import threading
 
 import pytest
@@ -135,3 +136,24 @@ def test_trim_gives_back(gpu_ctx):
     # W alone is 56 MB here; the runtime keeps a little of its own
     assert before - after < 32 << 20, (before, after)
     ctx.close()
+
+
+def test_failed_allocation_trims_every_context(gpu_ctx):
+    # a 2^50-byte request fails; what another context on the device kept
+    # was given back before the second try
+    a, b = Context(0), Context(0)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    before = torch.cuda.mem_get_info(0)[0]
+    h = C.c_void_p()
+    L.check(a.lib.b2g_buf_create(a.h, 1 << 28, L.B2G_F64, C.byref(h)))
+    a.lib.b2g_buf_destroy(h)
+    assert before - torch.cuda.mem_get_info(0)[0] > 1 << 30  # kept
+    with pytest.raises(L.B2GError):
+        L.check(b.lib.b2g_buf_create(b.h, 1 << 47, L.B2G_F64, C.byref(h)))
+    assert before - torch.cuda.mem_get_info(0)[0] < 32 << 20
+    # both contexts work on
+    want = site(gpu_ctx, SITES[0])
+    assert same(site(a, SITES[0]), want) and same(site(b, SITES[0]), want)
+    a.close()
+    b.close()
