@@ -463,8 +463,10 @@ extern "C" int b2g_effham_create(b2g_ctx ctx, const b2g_problem *pb,
 extern "C" int b2g_effham_destroy(b2g_effham h) {
     if (h == nullptr)
         return B2G_OK;
-    if (h->ctx)
+    if (h->ctx) {
+        hipSetDevice(h->ctx->device);
         hipStreamSynchronize(h->ctx->stream);
+    }
     h->dav.release();
     b2g_plan_destroy(h->plan);
     b2g_buf_destroy(h->lbuf);

@@ -87,7 +87,25 @@ BlockPool::~BlockPool() {
     trim();
 }
 
+// `device` current in a scope, whichever was (a block of another device must
+// not get into the pool, nor that device's free memory decide)
+struct OnDevice {
+    int was;
+    explicit OnDevice(int device) : was(device) {
+        if (hipGetDevice(&was) == hipSuccess && was != device)
+            (void)hipSetDevice(device);
+        else
+            was = -1;
+    }
+    OnDevice(const OnDevice &) = delete;
+    ~OnDevice() {
+        if (was >= 0)
+            (void)hipSetDevice(was);
+    }
+};
+
 hipError_t BlockPool::make(size_t bytes, void **out) {
+    const OnDevice on(device_);
     return pinned_ ? hipHostMalloc(out, bytes) : hipMalloc(out, bytes);
 }
 void BlockPool::drop(void *p) {
@@ -154,6 +172,7 @@ void BlockPool::put(void *p) {
     kept_ += n;
     size_t cap = kPoolCap;
     if (!pinned_ && n >= ((size_t)64 << 20)) {
+        const OnDevice on(device_);
         size_t avail = 0, total = 0;
         if (hipMemGetInfo(&avail, &total) == hipSuccess && avail < total / 4)
             cap = 0;
