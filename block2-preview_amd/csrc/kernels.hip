@@ -503,10 +503,10 @@ int tile_m(int cfg) { return 32 << (cfg / 3); }
 int tile_n(int cfg) { return 32 << (cfg % 3); }
 
 // persistent grid: min(grid, ntasks) workgroups per right-hand side, a
-// multiple of 8
+// multiple of 8; a launch has fewer than 2^32 threads
 unsigned task_grid(int grid, int ntasks, int n_rhs) {
     const int64_t g = (int64_t)(grid < ntasks ? grid : ntasks) * n_rhs;
-    return (unsigned)((g < (1 << 30) ? g : (1 << 30)) + 7) & ~7u;
+    return (unsigned)((g < (1 << 20) ? g : (1 << 20)) + 7) & ~7u;
 }
 
 template <typename TA, typename TB, typename TD, typename TC, int PHASE>

@@ -145,3 +145,22 @@ def test_chunk_edges(gpu_ctx, small_blocks, precision, tile):
         assert rel(y[r], ys[r]) < tol, r
         one = run(gpu_ctx, pb, xs[r:r + 1], env, precision=precision)
         assert np.array_equal(one[0], y[r]), r
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32", "bf16x3"])
+def test_many_right_hand_sides(gpu_ctx, precision):
+    # 20000 vectors on some 900 tasks: more (task, vector) items than a launch
+    # may have workgroups.  A vector's result does not depend on the others,
+    # tolerances as above
+    pb = synth.middle_site(n_orb=6, m=16, max_dim=4, seed=5)
+    n = 20000
+    xs = np.random.default_rng(3).standard_normal((n, pb.ket_len))
+    print(precision, flush=True)
+    y = run(gpu_ctx, pb, xs, {"B2G_KSPLIT": "100000"}, precision=precision)
+    orc = O.Oracle(pb)
+    tol = {"f64": 1e-12, "f32": 2e-6, "bf16x3": 1e-4}[precision]
+    for r in (0, 1, 4097, n - 1):
+        assert rel(y[r], orc.hpsi(xs[r], nthreads=8)) < tol, r
+    part = run(gpu_ctx, pb, xs[n - 500:], {"B2G_KSPLIT": "100000"},
+               precision=precision)
+    assert np.array_equal(part, y[n - 500:])
