@@ -431,7 +431,7 @@ hipError_t launch_seg_gemm_pk(int cfg, const __bf16 *A, const __bf16 *B,
                               XcdSplit xs) {
     if (ntasks <= 0)
         return hipSuccess;
-    const dim3 g(task_grid(grid, ntasks, n_rhs));
+    const dim3 g = task_grid(grid, ntasks, n_rhs);
 #define B2G_LAUNCH(TM_, TN_)                                                   \
     hipLaunchKernelGGL((seg_gemm_pk_kernel<TM_, TN_, OUT>), g, dim3(256), 0,   \
                        st, A, B, D0, D1, tasks, ntasks, segs, a_rs,            \

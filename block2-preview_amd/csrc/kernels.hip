@@ -502,11 +502,13 @@ template hipError_t launch_splitk_reduce<double>(double *, const double *,
 int tile_m(int cfg) { return 32 << (cfg / 3); }
 int tile_n(int cfg) { return 32 << (cfg % 3); }
 
-// persistent grid: min(grid, ntasks) workgroups per right-hand side, a
-// multiple of 8; a launch has fewer than 2^32 threads
-unsigned task_grid(int grid, int ntasks, int n_rhs) {
-    const int64_t g = (int64_t)(grid < ntasks ? grid : ntasks) * n_rhs;
-    return (unsigned)((g < (1 << 20) ? g : (1 << 20)) + 7) & ~7u;
+// persistent grid: min(grid, ntasks) workgroups per right-hand side, rounded
+// up to eights
+dim3 task_grid(int grid, int ntasks, int n_rhs) {
+    const int ng = (n_rhs + kRhsGroup - 1) / kRhsGroup;
+    const int gs = (n_rhs + ng - 1) / ng;
+    const int g = grid < ntasks ? grid : ntasks;
+    return dim3(8u * gs, (unsigned)(g + 7) / 8, (unsigned)ng);
 }
 
 template <typename TA, typename TB, typename TD, typename TC, int PHASE>
@@ -517,7 +519,7 @@ hipError_t launch_seg_gemm(int cfg, const TA *A, const TB *B, TD *D, TD *P,
                            int grid, hipStream_t st, XcdSplit xs) {
     if (ntasks <= 0)
         return hipSuccess;
-    const dim3 g(task_grid(grid, ntasks, n_rhs));
+    const dim3 g = task_grid(grid, ntasks, n_rhs);
 #define B2G_LAUNCH(TM_, TN_, TK_)                                              \
     hipLaunchKernelGGL((seg_gemm_kernel<TA, TB, TD, TC, TM_, TN_, TK_, PHASE>), \
                        g,                                                      \

@@ -79,37 +79,50 @@ __host__ __device__ inline int task_cfg(const Task &t) {
     return (int)((t.beta >> 4) & 15u);
 }
 
-// Per-XCD task ranges of one launch: when off[8] != 0, workgroup b (dealt
-// to XCD b % 8 by the dispatcher) walks tasks [off[b % 8], off[b % 8 + 1])
-// with stride grid / 8; otherwise all workgroups stride the whole list.
+// Per-XCD task ranges of one launch: when off[8] != 0, the workgroups of XCD
+// x walk tasks [off[x], off[x + 1]); otherwise tasks are dealt in turn
+// (TaskRange).
 struct XcdSplit {
     uint32_t off[9];
 };
 
-// The (task, right-hand side) items of one launch, walked by a workgroup.
-// The right-hand sides of a task run next to one another on one XCD
-// (workgroup b runs on XCD b % 8), where the operator panels they share stay
-// in its L2.  The grid is a multiple of 8 workgroups (task_grid).
+// The tasks of one launch that a workgroup walks, for one right-hand side.
+// Grid (task_grid): x = 8 XCDs by up to kRhsGroup right-hand sides, y strides
+// the tasks by eights (split: an XCD's own list), z = groups of right-hand
+// sides.  Workgroups are dealt to the XCDs in turn, x % 8, so the right-hand
+// sides of a group run a task next to one another on one XCD, where the
+// operator panels they share stay in its L2; with z the tasks move on by one
+// XCD, since the first XCDs get the costlier task of each eight.  Without a
+// division per item: a small site's tasks take a few microseconds, and task
+// and right-hand side out of one index made its products slower than one
+// grid per right-hand side from 64 on (FP32 product at n=8 M=50: 64 of them
+// 356 us with a grid each, 403 us with the division, 368 us so; FP64 at n=26
+// M=1000: four 2617, 1310 and 1299 us, 128 of them 42.4, 43.8 and 42.0 ms).
+// Groups of 4 instead of 8 gain 2 % on one split-BF16 product (n=16 M=500)
+// and lose as much on another (n=30 M=1500, six right-hand sides).
+constexpr int kRhsGroup = 8;
 struct TaskRange {
-    int i, end, step, nrhs, x; // item of the XCD's own sequence
-    bool split;
-    __device__ __forceinline__ TaskRange(int ntasks, int nrhs_,
-                                         const XcdSplit &xs)
-        : nrhs(nrhs_), x(blockIdx.x & 7), split(xs.off[8] != 0) {
-        const int t0 = split ? (int)xs.off[x] : 0;
-        const int t1 = split ? (int)xs.off[x + 1] : (ntasks - x + 7) / 8;
-        i = t0 * nrhs + (int)(blockIdx.x >> 3);
-        end = t1 * nrhs;
-        step = (int)(gridDim.x >> 3);
+    int t, end, step, r;
+    __device__ __forceinline__ TaskRange(int ntasks, int nrhs,
+                                         const XcdSplit &xs) {
+        const int x = blockIdx.x & 7;
+        r = (int)(blockIdx.z * (gridDim.x >> 3) + (blockIdx.x >> 3));
+        if (xs.off[8] != 0) {
+            t = (int)(xs.off[x] + blockIdx.y);
+            end = (int)xs.off[x + 1];
+            step = (int)gridDim.y;
+        } else {
+            t = 8 * (int)blockIdx.y + ((x + (int)blockIdx.z) & 7);
+            end = ntasks;
+            step = 8 * (int)gridDim.y;
+        }
+        if (r >= nrhs) // the last group is short
+            end = t;
     }
-    __device__ __forceinline__ bool more() const { return i < end; }
-    __device__ __forceinline__ void next() { i += step; }
-    // task index and right-hand side of the current item
-    __device__ __forceinline__ int task() const {
-        const int t = i / nrhs;
-        return split ? t : 8 * t + x;
-    }
-    __device__ __forceinline__ int rhs() const { return i % nrhs; }
+    __device__ __forceinline__ bool more() const { return t < end; }
+    __device__ __forceinline__ void next() { t += step; }
+    __device__ __forceinline__ int task() const { return t; }
+    __device__ __forceinline__ int rhs() const { return r; }
 };
 
 // Deterministic split-K reduction of one output tile:

@@ -16,8 +16,8 @@ constexpr int kSmallCfg = 4;
 // tile area in units of 32 x 32
 inline int tile_area(int cfg) { return (1 << (cfg / 3)) << (cfg % 3); }
 
-// persistent grid size of a grouped-GEMM launch (a multiple of 8)
-unsigned task_grid(int grid, int ntasks, int n_rhs);
+// persistent grid of a grouped-GEMM launch (TaskRange)
+dim3 task_grid(int grid, int ntasks, int n_rhs);
 
 // PHASE (1: work = C op(B), 2: V += alpha op(A) work, 3 / 4: the two stages
 // of the operator gradients) only tags the kernel name, so that profiles tell

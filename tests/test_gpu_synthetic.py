@@ -164,3 +164,19 @@ def test_many_right_hand_sides(gpu_ctx, precision):
     part = run(gpu_ctx, pb, xs[n - 500:], {"B2G_KSPLIT": "100000"},
                precision=precision)
     assert np.array_equal(part, y[n - 500:])
+
+
+@pytest.mark.parametrize("xcd", ["0", "1"])
+@pytest.mark.parametrize("precision", ["f64", "f32", "bf16x3"])
+def test_right_hand_side_groups(gpu_ctx, small_blocks, precision, xcd):
+    # counts around a group of eight, whole and short groups, tasks dealt in
+    # turn and by XCD list: every vector as alone
+    pb, xs, ys = small_blocks
+    x = np.random.default_rng(6).standard_normal((25, pb.ket_len))
+    env = {"B2G_XCD": xcd}
+    print(precision, "xcd", xcd, flush=True)
+    want = np.stack([run(gpu_ctx, pb, v[None], env, precision=precision)[0]
+                     for v in x])
+    for n in (2, 7, 8, 9, 16, 17, 25):
+        y = run(gpu_ctx, pb, x[:n], env, precision=precision)
+        assert np.array_equal(y, want[:n]), n
