@@ -378,8 +378,8 @@ __device__ __forceinline__ void seg_gemm_task(
             }
 }
 
-// tiles with a side of 128: one launch per shape (two workgroups per compute
-// unit: 240 VGPRs for 128 x 128 in FP64)
+// tiles with a side of 128, and lists of 32 x 32 tiles only: one launch per
+// shape (two workgroups per compute unit: 240 VGPRs for 128 x 128 in FP64)
 template <typename TA, typename TB, typename TD, typename TC, int TM, int TN,
           int TK, int PHASE>
 __global__ __launch_bounds__(256, 2) void seg_gemm_kernel(
@@ -408,7 +408,10 @@ __global__ __launch_bounds__(256, 2) void seg_gemm_kernel(
 // Product at that site, one right-hand side: 1279 -> 391 us (FP64), three at
 // n=16 M=500: 1930 -> 412 us, FP32, two: 1588 -> 401 us, n=8 M=50: 127 -> 47
 // us (with the split along K of tile_env_refresh); one launch per shape for
-// the same tiles: 444, 498 and 460 us for the first three.
+// the same tiles: 444, 498 and 460 us for the first three.  A launch of
+// 32 x 32 tiles only (launch_tiny) takes their own kernel, which fits more
+// workgroups on a compute unit: FP32 product at n=8 M=50, 128 right-hand
+// sides 691 -> 625 us, one 47.4 -> 46.7 us.
 template <typename TA, typename TB, typename TD, typename TC, int PHASE>
 __global__ __launch_bounds__(256, 4) void seg_gemm_small_kernel(
     const TA *__restrict__ A, const TB *__restrict__ B, TD *__restrict__ D,
@@ -526,6 +529,7 @@ hipError_t launch_seg_gemm(int cfg, const TA *A, const TB *B, TD *D, TD *P,
                        dim3(256), 0, st, A, B, D, P, tasks, ntasks, segs,      \
                        a_rs, b_rs, d_rs, p_rs, scale, beta0, n_rhs, xs)
     switch (cfg) {
+    case 0: B2G_LAUNCH(32, 32, 32); break;
     case 2: B2G_LAUNCH(32, 128, 16); break;
     case 5: B2G_LAUNCH(64, 128, 16); break;
     case 6: B2G_LAUNCH(128, 32, 16); break;

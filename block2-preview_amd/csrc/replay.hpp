@@ -109,6 +109,7 @@ int cfg_of(const Tile &t);
 // launch (task bucket) of a tile of the FP64 / FP32 (table 0) or split-BF16
 // (1) kernels
 int launch_of(const Tile &t, int table);
+void launch_tiny(std::vector<Task> *tasks);
 // one task per tile of the block, all over segments [sb, se)
 void add_tiles(std::vector<Task> *tasks, uint64_t d_off, uint32_t M,
                uint32_t N, uint64_t K, uint32_t sb, uint32_t se,

@@ -661,6 +661,16 @@ int launch_of(const Tile &t, int table) {
     return kSmallCfg;
 }
 
+// A list whose small tiles are all 32 x 32 takes their own kernel
+// (seg_gemm_small_kernel says why).
+void launch_tiny(std::vector<Task> *tasks) {
+    std::vector<Task> &small = tasks[kSmallCfg];
+    if (tasks[0].empty() &&
+        std::all_of(small.begin(), small.end(),
+                    [](const Task &t) { return task_cfg(t) == 0; }))
+        tasks[0].swap(small);
+}
+
 // one task per tile (phase 1 and unsplit phase-2 blocks)
 void add_tiles(std::vector<Task> *tasks, uint64_t d_off, uint32_t M,
                       uint32_t N, uint64_t K, uint32_t sb, uint32_t se,
@@ -1322,6 +1332,8 @@ static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
             for (const BlockJob &job : ch.jobs2)
                 add_split_tiles(ch.s2, job, 0, ch.t2, ch.red, ch.p_len);
             tm.mark("chunk tasks");
+            launch_tiny(ch.t1);
+            launch_tiny(ch.t2);
             for (int c = 0; c < kTileConfigs; c++) {
                 ch.x1[c] = xcd_order(ch.t1[c], ch.s1, xcd_enabled());
                 ch.x2[c] = xcd_order(ch.t2[c], ch.s2, xcd_enabled());
