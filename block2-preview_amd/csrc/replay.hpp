@@ -56,6 +56,13 @@ struct b2g_plan_s {
     uint64_t p_max = 0;   // partial elements per RHS (max over chunks)
     uint64_t p_ref = 0;   // the same for the plain split (2048 deep, tiles to
                           // 128): what the allocation-free entry admits by
+    // the lists of products with many right-hand sides (FP64 / FP32, built by
+    // the first of them): tiles and split as of a plan of any size.  The
+    // segments are those of `chunks`.
+    std::vector<b2g::Chunk> many;
+    void *many_dev = nullptr;
+    uint64_t many_p = 0;     // their partial elements per RHS
+    bool plain = false;      // `chunks` are such lists already
     void *pbuf = nullptr; // split-K partial tiles (FP64)
     size_t p_bytes = 0;
     unsigned flags = 0;

@@ -519,6 +519,7 @@ struct TileEnv {
     uint32_t fm = 0, fn = 0; // forced tile shape (0: measured rates)
     uint64_t ksplit = 2048;  // split-K depth threshold of phase 2
     uint32_t cap = 128;      // largest tile side
+    bool cap_set = false;    // by B2G_TILE_CAP
 };
 // of the plan being built, and the settings it would have without regard to
 // its size
@@ -561,7 +562,7 @@ void tile_env_refresh(uint64_t macs, uint64_t macs2, int num_cu, int table) {
         v.cap = 64;
     if (const char *e = getenv("B2G_TILE_CAP"))
         if (atoi(e) == 64 || atoi(e) == 128)
-            v.cap = (uint32_t)atoi(e);
+            v.cap = (uint32_t)atoi(e), v.cap_set = true;
     // (split-BF16: k-steps of 32 and half the time per step: no shallower
     // than 256, and large plans as deep as they were: M=200 depths 64 / 256 /
     // 2048 take 71 / 64 / 133 us, M=2000 512 / 1024 / 2048 966 / 897 / 887)
@@ -1050,9 +1051,9 @@ int ctx_stage(b2g_ctx ctx, size_t bytes, char **out) {
 }
 
 // upload all chunks' task / segment / reduction arrays in one allocation
-static int upload_chunks(b2g_plan p) {
+static int upload_chunks(b2g_plan p, std::vector<Chunk> &chunks, void **dev) {
     size_t bytes = 0;
-    for (auto &ch : p->chunks) {
+    for (auto &ch : chunks) {
         for (int c = 0; c < kTileConfigs; c++)
             bytes += (ch.t1[c].size() + ch.t2[c].size()) * sizeof(Task);
         bytes += (ch.s1.size() + ch.s2.size()) * sizeof(Seg);
@@ -1062,7 +1063,7 @@ static int upload_chunks(b2g_plan p) {
     const int rs = ctx_stage(p->ctx, bytes + 16, &host);
     if (rs != B2G_OK)
         return rs;
-    B2G_HIP(p->ctx->alloc(&p->dev, bytes + 16));
+    B2G_HIP(p->ctx->alloc(dev, bytes + 16));
     size_t off = 0;
     auto put = [&](const void *src, size_t nb) -> size_t {
         size_t o = off;
@@ -1075,7 +1076,7 @@ static int upload_chunks(b2g_plan p) {
         size_t t1[kTileConfigs], t2[kTileConfigs], s1, s2, red;
     };
     std::vector<Offs> offs;
-    for (auto &ch : p->chunks) {
+    for (auto &ch : chunks) {
         Offs o;
         for (int c = 0; c < kTileConfigs; c++) {
             o.t1[c] = put(ch.t1[c].data(), ch.t1[c].size() * sizeof(Task));
@@ -1086,12 +1087,12 @@ static int upload_chunks(b2g_plan p) {
         o.red = put(ch.red.data(), ch.red.size() * sizeof(RedTask));
         offs.push_back(o);
     }
-    B2G_HIP(hipMemcpyAsync(p->dev, host, bytes, hipMemcpyHostToDevice,
+    B2G_HIP(hipMemcpyAsync(*dev, host, bytes, hipMemcpyHostToDevice,
                            p->ctx->stream));
     B2G_HIP(hipStreamSynchronize(p->ctx->stream));
-    char *base = (char *)p->dev;
-    for (size_t i = 0; i < p->chunks.size(); i++) {
-        Chunk &ch = p->chunks[i];
+    char *base = (char *)*dev;
+    for (size_t i = 0; i < chunks.size(); i++) {
+        Chunk &ch = chunks[i];
         for (int c = 0; c < kTileConfigs; c++) {
             ch.d_t1[c] = (Task *)(base + offs[i].t1[c]);
             ch.d_t2[c] = (Task *)(base + offs[i].t2[c]);
@@ -1100,6 +1101,85 @@ static int upload_chunks(b2g_plan p) {
         ch.d_s2 = (Seg *)(base + offs[i].s2);
         ch.d_red = (RedTask *)(base + offs[i].red);
     }
+    return B2G_OK;
+}
+
+// launches, order and operation counts of a chunk's task lists
+static void order_chunk(Chunk &ch, const std::vector<Seg> &s1,
+                        const std::vector<Seg> &s2) {
+    launch_tiny(ch.t1);
+    launch_tiny(ch.t2);
+    for (int c = 0; c < kTileConfigs; c++) {
+        ch.x1[c] = xcd_order(ch.t1[c], s1, xcd_enabled());
+        ch.x2[c] = xcd_order(ch.t2[c], s2, xcd_enabled());
+        ch.f1[c] = task_flops(ch.t1[c], s1);
+        ch.f2[c] = task_flops(ch.t2[c], s2);
+    }
+    ch.slices = red_slices(ch.red);
+}
+
+// The number of right-hand sides from which a product takes the lists of
+// `many`.  They fill the chip by themselves then, so tiles up to 128 with
+// their reuse, and no partials but of deep blocks.  FP32 product with the
+// plan's own lists / these / (own lists before tiles and split went by the
+// plan's size): n=12 M=200, 64 right-hand sides 1124 / 974 / 1195 us, 128
+// 2193 / 1817 / 1982 us; n=26 M=1000 16 3192 / 3386 / 4003 us, 32 6382 / 6057
+// / 6695 us, 128 25.6 / 22.7 / 24.2 ms; n=30 M=1500 6 2489 / 2712 / 3269 us,
+// 16 6617 / 6118 / 6978 us, 64 26.6 / 23.3 / 25.1 ms; n=16 M=500, in FP64, 32
+// 3542 / 3892 / 4566 us, 64 7094 / 7039 / 7749 us.  Never below the number
+// that the allocation-free entry takes at most: it runs the plan's own lists
+// and gives the same bits.
+static int many_from(const b2g_plan_s *p) {
+    const int none = 1 << 30;
+    if (p->plain || p->macs == 0)
+        return none;
+    const uint64_t n =
+        std::min<uint64_t>(64, std::max<uint64_t>(16, 150000000000ull / p->macs));
+    return (int)std::max<uint64_t>(
+        n, kNoAllocScratchBytes / (4 * std::max<uint64_t>(p->w_max, 1)) + 1);
+}
+
+static int build_many(b2g_plan p) {
+    SetupTimer tm("lists for many right-hand sides");
+    tile_env_refresh(p->macs, p->macs2, p->ctx->num_cu);
+    t_env.ksplit = t_plain.ksplit;
+    if (!t_env.cap_set)
+        t_env.cap = t_plain.cap;
+    std::vector<Chunk> many;
+    uint64_t p_len = 0;
+    for (const Chunk &ch : p->chunks) {
+        Chunk m;
+        // one W block per phase-1 segment, as its tiles have it
+        std::vector<const Task *> block(ch.s1.size(), nullptr);
+        for (const auto &list : ch.t1)
+            for (const Task &t : list)
+                block[t.seg_begin] = &t;
+        for (const Task *t : block)
+            if (t != nullptr)
+                add_tiles(m.t1, t->d_off, t->M, t->N, 1, t->seg_begin,
+                          t->seg_end, 0);
+        for (const BlockJob &job : ch.jobs2)
+            add_split_tiles(ch.s2, job, 0, m.t2, m.red, m.p_len);
+        order_chunk(m, ch.s1, ch.s2);
+        p_len = std::max(p_len, m.p_len);
+        many.push_back(std::move(m));
+    }
+    tm.mark("lists");
+    void *dev = nullptr;
+    const int r = upload_chunks(p, many, &dev);
+    if (r != B2G_OK) {
+        p->ctx->pool.put(dev);
+        return r;
+    }
+    p->many_dev = dev;
+    for (size_t i = 0; i < many.size(); i++) {
+        many[i].d_s1 = p->chunks[i].d_s1;
+        many[i].d_s2 = p->chunks[i].d_s2;
+        many[i].w_len = p->chunks[i].w_len;
+    }
+    p->many_p = p_len;
+    p->many.swap(many);
+    tm.mark("upload");
     return B2G_OK;
 }
 
@@ -1332,18 +1412,12 @@ static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
             for (const BlockJob &job : ch.jobs2)
                 add_split_tiles(ch.s2, job, 0, ch.t2, ch.red, ch.p_len);
             tm.mark("chunk tasks");
-            launch_tiny(ch.t1);
-            launch_tiny(ch.t2);
+            order_chunk(ch, ch.s1, ch.s2);
             for (int c = 0; c < kTileConfigs; c++) {
-                ch.x1[c] = xcd_order(ch.t1[c], ch.s1, xcd_enabled());
-                ch.x2[c] = xcd_order(ch.t2[c], ch.s2, xcd_enabled());
-                ch.f1[c] = task_flops(ch.t1[c], ch.s1);
-                ch.f2[c] = task_flops(ch.t2[c], ch.s2);
                 p->kflops[B2G_K_PHASE1 + c] += ch.f1[c];
                 p->kflops[B2G_K_PHASE2 + c] += ch.f2[c];
             }
             tm.mark("chunk order and flops");
-            ch.slices = red_slices(ch.red);
             p->w_max = std::max(p->w_max, ch.w_len);
             p->p_max = std::max(p->p_max, ch.p_len);
             p->chunks.push_back(std::move(ch));
@@ -1353,7 +1427,8 @@ static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
     };
     build(whole, false);
     build(windows, true);
-    const int r = upload_chunks(p);
+    p->plain = t_env.cap == t_plain.cap && t_env.ksplit == t_plain.ksplit;
+    const int r = upload_chunks(p, p->chunks, &p->dev);
     tm.mark("upload");
     return r;
 }
@@ -1428,7 +1503,8 @@ extern "C" int b2g_plan_destroy(b2g_plan p) {
         hipEventDestroy(st.start);
         hipEventDestroy(st.stop);
     }
-    for (void *q : {p->dev, (void *)p->l32, (void *)p->r32, p->w, p->pbuf})
+    for (void *q : {p->dev, p->many_dev, (void *)p->l32, (void *)p->r32, p->w,
+                    p->pbuf})
         p->ctx->pool.put(q);
     grad_plan_destroy(p->ctx, p->grad);
     pk_destroy(p->ctx, p->pk);
@@ -1595,9 +1671,19 @@ int plan_reserve(b2g_plan p, int n_rhs, int precision) {
         p->w_bytes = need;
         p->scratch_gen++;
     }
-    const uint64_t pmax =
-        std::max<uint64_t>(p->p_max, p->pk != nullptr ? p->pk->p_max : 0);
-    const size_t pneed = std::max<uint64_t>(pmax, 1) * n_rhs * 8;
+    // partials of this and of any smaller number of right-hand sides
+    const int from = many_from(p);
+    if (precision != B2G_PREC_BF16X3 && n_rhs >= from && p->many.empty()) {
+        const int r = build_many(p);
+        if (r != B2G_OK)
+            return r;
+    }
+    uint64_t plen = std::max<uint64_t>(
+        1, p->p_max * std::min<int>(n_rhs, from - 1));
+    plen = std::max(plen, p->many_p * n_rhs);
+    if (p->pk != nullptr)
+        plen = std::max(plen, p->pk->p_max * n_rhs);
+    const size_t pneed = plen * 8;
     if (pneed > p->p_bytes) {
         if (p->pbuf) {
             B2G_HIP(plan_wait(p));
@@ -1627,12 +1713,14 @@ extern "C" int b2g_plan_reserve(b2g_plan p, int n_rhs, int precision) {
 
 namespace b2g {
 
-// One H*psi with the FP64 / FP32 W scratch at `W` and the split-K partials
+// One H*psi by the lists `chunks` with p_max partial elements per right-hand
+// side, the FP64 / FP32 W scratch at `W` and the split-K partials
 // at `P` (for split-BF16 the packed operands of the plan); allocates nothing
 // itself.
-static int hpsi_run(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
-                    int n_rhs, double scale, int accumulate, int precision,
-                    void *W, double *P) {
+static int hpsi_run(b2g_ctx ctx, b2g_plan p, const std::vector<Chunk> &chunks,
+                    uint64_t p_max, const double *x, double *y, int n_rhs,
+                    double scale, int accumulate, int precision, void *W,
+                    double *P) {
     const int grid = ctx->num_cu * 8;
     // brackets one launch on stream `st` with timing events when enabled
     auto timed = [&](int kernel, hipStream_t st,
@@ -1727,8 +1815,8 @@ static int hpsi_run(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
                                     p->x_len,
                                     pk->x_len, n_rhs, grid, st);
         }));
-    for (size_t ic = 0; ic < p->chunks.size(); ic++) {
-        const Chunk &ch = p->chunks[ic];
+    for (size_t ic = 0; ic < chunks.size(); ic++) {
+        const Chunk &ch = chunks[ic];
         // chunk 0 overwrites unless accumulating; later chunks' tasks add
         const int beta0 = ic == 0 ? (accumulate ? 1 : 0) : 1;
         if (pk != nullptr) {
@@ -1778,17 +1866,17 @@ static int hpsi_run(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
                 return launch_seg_gemm<double, double, double, double, 2>(
                     c, (const double *)p->lbuf->ptr, (const double *)W, y,
                     P, ch.d_t2[c], nt, ch.d_s2, 0, p->w_max, p->y_len,
-                    p->p_max, scale, beta0, n_rhs, grid, st, ch.x2[c]);
+                    p_max, scale, beta0, n_rhs, grid, st, ch.x2[c]);
             return launch_seg_gemm<float, float, double, float, 2>(
                 c, p->l32, (const float *)W, y, P, ch.d_t2[c], nt,
-                ch.d_s2, 0, p->w_max, p->y_len, p->p_max, scale, beta0, n_rhs,
+                ch.d_s2, 0, p->w_max, p->y_len, p_max, scale, beta0, n_rhs,
                 grid, st, ch.x2[c]);
         }));
         const int nr = (int)ch.red.size();
         if (nr > 0)
             B2G_HIP(timed(B2G_K_SPLITK_REDUCE, ctx->stream, [&](hipStream_t st) {
                 return launch_splitk_reduce<double>(
-                    y, P, ch.d_red, nr, ch.slices, p->y_len, p->p_max, beta0,
+                    y, P, ch.d_red, nr, ch.slices, p->y_len, p_max, beta0,
                     n_rhs, grid, st);
             }));
     }
@@ -1814,8 +1902,10 @@ extern "C" int b2g_hpsi(b2g_ctx ctx, b2g_plan p, const double *x, double *y,
         if (r != B2G_OK)
             return r;
     }
-    return hpsi_run(ctx, p, x, y, n_rhs, scale, accumulate, precision, p->w,
-                    (double *)p->pbuf);
+    const bool many = precision != B2G_PREC_BF16X3 && n_rhs >= many_from(p);
+    return hpsi_run(ctx, p, many ? p->many : p->chunks,
+                    many ? p->many_p : p->p_max, x, y, n_rhs, scale,
+                    accumulate, precision, p->w, (double *)p->pbuf);
 }
 
 extern "C" int b2g_hpsi_noalloc(b2g_ctx ctx, b2g_plan p, const double *x,
@@ -1861,7 +1951,8 @@ extern "C" int b2g_hpsi_noalloc(b2g_ctx ctx, b2g_plan p, const double *x,
     // W element phase 2 reads, and each split-K partial is written before
     // the reduction reads it
     for (int r = 0; r < n_rhs; r += step) {
-        const int rc = hpsi_run(ctx, p, x + (size_t)r * p->x_len,
+        const int rc = hpsi_run(ctx, p, p->chunks, p->p_max,
+                                x + (size_t)r * p->x_len,
                                 y + (size_t)r * p->y_len,
                                 std::min(step, n_rhs - r), scale, accumulate,
                                 precision, base, (double *)(base + w_bytes));

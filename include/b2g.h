@@ -215,6 +215,9 @@ int b2g_plan_stats(b2g_plan plan, uint64_t *n_tasks1, uint64_t *n_tasks2,
                    uint64_t *scratch_elems);
 
 /* y[r] = (accumulate ? y[r] : 0) + scale * H * x[r]  for r < n_rhs.
+ * (FP64 and FP32: from 16 to 64 right-hand sides on, by the plan's size, the
+ * product is cut into larger tiles and sums in another order; the first such
+ * product, or b2g_plan_reserve, makes those lists.)
  * x and y are device arrays of n_rhs stacked vectors (x_len, y_len each),
  * FP64.  precision: B2G_PREC_*.  Enqueued on the context stream (with one
  * right-hand side the independent launches of a phase overlap on the

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+from b2g import _lib as L
 from b2g import synth
 from b2g.effham import EffectiveHamiltonian
 import b2g_oracle as O
@@ -180,3 +181,28 @@ def test_right_hand_side_groups(gpu_ctx, small_blocks, precision, xcd):
     for n in (2, 7, 8, 9, 16, 17, 25):
         y = run(gpu_ctx, pb, x[:n], env, precision=precision)
         assert np.array_equal(y, want[:n]), n
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_lists_for_many_right_hand_sides(gpu_ctx, problem, precision):
+    # from 64 right-hand sides on, this plan runs tiles up to 128; fewer after
+    # that run its own lists again, on the scratch that is there
+    pb, xs, ys = problem
+    tol = 1e-12 if precision == "f64" else 2e-6
+    h = EffectiveHamiltonian(pb, gpu_ctx, fp32=precision == "f32")
+    x = torch.tensor(np.tile(xs, (17, 1)), device="cuda:0")
+    own = None
+    for n in (3, 63, 64, 65, 68, 3, 63):
+        print(precision, n, flush=True)
+        h.set_timing(True)
+        y = h.multiply(x[:n], precision=precision).cpu().numpy()
+        ms, cnt = h.timing()
+        h.set_timing(False)
+        for k in (L.K_PHASE1, L.K_PHASE2):
+            assert (cnt[k + 8] > 0) == (n >= 64), (n, k)
+        for r in range(n):
+            assert rel(y[r], ys[r % 4]) < tol, (n, r)
+        if n < 64:
+            own = y[:3] if own is None else own
+            assert np.array_equal(y[:3], own), n
+    h.deallocate()
