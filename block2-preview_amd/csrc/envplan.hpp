@@ -81,7 +81,7 @@ struct WinGroup {
     uint64_t c_off;
     uint32_t ldc, rows, cols;
     uint32_t rec_begin, rec_end;
-    uint32_t pad;
+    uint32_t chunk0; // first of the window's chunks (winplan_finish)
 };
 
 // allocator whose resize leaves trivially constructible elements
