@@ -33,20 +33,33 @@ def problem():
     return pb, xs, ys
 
 
+def cfg(tile):
+    """Tile configuration of "T" or "TMxTN"."""
+    t = [int(v) for v in tile.split("x")]
+    return 3 * (t[0] // 64) + t[-1] // 64
+
+
 def run(gpu_ctx, pb, xs, env, precision="f64"):
+    # the product as well: the packed split-BF16 plan and the lists for many
+    # right-hand sides are tiled by the first of them
     old = {k: os.environ.get(k) for k in env}
     os.environ.update(env)
     try:
-        h = EffectiveHamiltonian(pb, gpu_ctx)
+        h = EffectiveHamiltonian(pb, gpu_ctx, fp32=precision == "f32")
+        x = torch.tensor(xs, dtype=torch.float64, device="cuda:0")
+        y = h.multiply(x, precision=precision).cpu().numpy()
+        fl = np.array(h.kernel_flops(precision))
     finally:
         for k, v in old.items():
             if v is None:
                 os.environ.pop(k, None)
             else:
                 os.environ[k] = v
-    x = torch.tensor(xs, dtype=torch.float64, device="cuda:0")
-    y = h.multiply(x, precision=precision).cpu().numpy()
     h.deallocate()
+    for k in (L.K_PHASE1, L.K_PHASE2):  # what was forced is what ran
+        used = set(np.flatnonzero(fl[k:k + 9]))
+        if "B2G_TILE" in env:
+            assert used == {cfg(env["B2G_TILE"])}, (env, used)
     return y
 
 
