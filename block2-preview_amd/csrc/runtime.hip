@@ -1394,7 +1394,9 @@ static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
                 }
             }
             // phase-2 tiles; a plan that the allocation-free entry may run
-            // keeps its partials below the room that entry has for them
+            // keeps its partials below the room that entry has for them (a
+            // B2G_TILE_CAP stays as it is: larger tiles are no fewer partial
+            // elements)
             const bool small = ch.w_len * 4 <= kNoAllocScratchBytes;
             if (small)
                 p->p_ref = std::max(p->p_ref,
@@ -1402,7 +1404,7 @@ static int compile_plan(b2g_plan p, const b2g_pair *pairs, size_t n_pairs,
             else
                 p->p_ref = ~(uint64_t)0 >> 8; // W alone is past its limit
             while (small && (t_env.ksplit < t_plain.ksplit ||
-                             t_env.cap < t_plain.cap) &&
+                             (t_env.cap < t_plain.cap && !t_env.cap_set)) &&
                    partial_len(ch.s2, ch.jobs2, t_env) > kPartialLimit) {
                 if (t_env.ksplit < t_plain.ksplit)
                     t_env.ksplit = std::min(2 * t_env.ksplit, t_plain.ksplit);

@@ -60,6 +60,10 @@ def run(gpu_ctx, pb, xs, env, precision="f64"):
         used = set(np.flatnonzero(fl[k:k + 9]))
         if "B2G_TILE" in env:
             assert used == {cfg(env["B2G_TILE"])}, (env, used)
+        if env.get("B2G_TILE_CAP") == "64":
+            assert used <= {0, 4}, (env, used)
+        elif "B2G_TILE_CAP" in env:
+            assert 8 in used, (env, used)
     return y
 
 
