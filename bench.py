@@ -558,7 +558,7 @@ def main():
     # dominant kernel is the one with the largest summed time, and its
     # algorithmic FLOPs per launch are the plan's per-kernel count (tiles of
     # that launch, all right-hand sides) divided by its launches per step
-    def kernel_table(ph, kfl):
+    def kernel_table(ph, kfl, prec):
         kms, kn = ph
         table = {}
         for k in range(L.NKERNELS):
@@ -567,18 +567,18 @@ def main():
             per_step = kn[k] // args.steps
             avg = kms[k] / kn[k]
             fl = kfl[k] * R / max(per_step, 1)
-            table[L.kernel_name(k)] = dict(
+            table[L.kernel_name(k, prec)] = dict(
                 launches_per_step=per_step, avg_launch_ms=round(avg, 4),
                 tflops=round(fl / (avg * 1e-3) / 1e12, 3) if fl > 0 else None)
         dk = max((k for k in range(L.NKERNELS) if kn[k] and kfl[k] > 0),
                  key=lambda k: kms[k])
         d_avg = kms[dk] / kn[dk]
         d_ach = kfl[dk] * R / max(kn[dk] // args.steps, 1) / (d_avg * 1e-3) / 1e12
-        return (table, L.kernel_name(dk), d_avg, kn[dk] // args.steps, d_ach,
+        return (table, L.kernel_name(dk, prec), d_avg, kn[dk] // args.steps, d_ach,
                 sum(kms[k] for k in range(L.NKERNELS)) / args.steps)
 
     kernels, dom, dur, per_step, achieved, t_gemm = kernel_table(
-        ph, h.kernel_flops("f64"))
+        ph, h.kernel_flops("f64"), "f64")
     log("FP64: %.3f ms/step, %.2f TFLOP/s; launches serialised for the "
         "per-kernel events: %.3f ms/step (%.3f ms in kernels)" % (
             ms64, tflops, ms64_serial, t_gemm))
@@ -593,7 +593,7 @@ def main():
     tflopsb = 2.0 * h.macs * R / (msb * 1e-3) / 1e12
     _, phb = run("bf16x3", args.steps, True)
     kernels_b, dom_b, dur_b, _, ach_b, _ = kernel_table(
-        phb, h.kernel_flops("bf16x3"))
+        phb, h.kernel_flops("bf16x3"), "bf16x3")
     log("split-BF16 x3: %.3f ms/step, %.2f TFLOP/s (FP64-equivalent work); "
         "dominant %s %.3f ms/launch, %.1f TFLOP/s" % (
             msb, tflopsb, dom_b, dur_b, ach_b))

@@ -157,14 +157,18 @@ KERNEL_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_double, MATVEC_FN,
 K_PHASE1, K_PHASE2, K_SPLITK_REDUCE, K_PACK, NKERNELS = 0, 9, 18, 19, 20
 
 
-def kernel_name(k):
+def kernel_name(k, precision=None):
+    """Name of kernel id k (b2g.h); with `precision` "f64" or "f32", whose
+    tiles of up to 64 x 64 share a launch, that launch is named so."""
     if k == K_SPLITK_REDUCE:
         return "splitk_reduce"
     if k == K_PACK:
         return "pack_bf16"
     c = k % 9
-    return "phase%d_%dx%d" % (1 if k < K_PHASE2 else 2, 32 << (c // 3),
-                              32 << (c % 3))
+    phase = 1 if k < K_PHASE2 else 2
+    if c == 4 and precision in ("f64", "f32"):
+        return "phase%d_to_64x64" % phase
+    return "phase%d_%dx%d" % (phase, 32 << (c // 3), 32 << (c % 3))
 
 _SIGS = {
     "b2g_last_error": (C.c_char_p, []),

@@ -174,7 +174,10 @@ int b2g_plan_macs(b2g_plan plan, uint64_t *out);
  * phase 1 (work = C op(B)) in tile configuration c is B2G_K_PHASE1 + c,
  * phase 2 (V += alpha op(A) work) is B2G_K_PHASE2 + c (c = 3*i + j,
  * TM = 32 << i, TN = 32 << j), the split-K reduction B2G_K_SPLITK_REDUCE,
- * and the split-BF16 packing of the wavefunction B2G_K_PACK.              */
+ * and the split-BF16 packing of the wavefunction B2G_K_PACK.  In FP64 and
+ * FP32 c = 4 is one launch of all tiles up to 64 x 64, whatever their shape;
+ * c = 0 a launch with tiles of 32 x 32 only; c = 1 and 3 occur only where
+ * B2G_TILE forces them.                                                   */
 #define B2G_K_PHASE1 0
 #define B2G_K_PHASE2 9
 #define B2G_K_SPLITK_REDUCE 18
@@ -192,7 +195,8 @@ int b2g_plan_timing(b2g_plan plan, double *ms, uint64_t *n_launch);
 /* Algorithmic FLOPs of one H*psi per right-hand side, per kernel id: 2 x the
  * multiply-adds of the kernel's tiles (phase 2 sums to exactly the
  * reference's second-GEMM count; phase 1 computes each distinct work matrix
- * once).  flops[B2G_NKERNELS].                                            */
+ * once), in the lists of few right-hand sides (b2g_hpsi).
+ * flops[B2G_NKERNELS].                                                    */
 int b2g_plan_kernel_flops(b2g_plan plan, double *flops);
 /* The same for the launches of one precision: B2G_PREC_BF16X3 counts the
  * tiles of the packed split-BF16 plan (built here if it is not yet), whose
