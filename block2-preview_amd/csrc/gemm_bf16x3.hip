@@ -18,7 +18,8 @@
 // arithmetic.  (As two planes, a k-step read half of two lines, twice the
 // requests between a compute unit's L1 and L2, whose number in flight bounds
 // these kernels: H*psi at M=3000 with four right-hand sides 14.4 against
-// 11.9 ms, matrix cores busy 33 against 46 % of phase 2.)  The constant
+// 11.9 ms, L1 read requests of phase 2 8.8e8 against 3.4e8, matrix cores busy
+// 33 against 49 % of it.)  The constant
 // operators are packed once per plan (in the orientation each pair reads
 // them), the wavefunction once per H*psi, and phase 1 writes its product W
 // directly as packed W^T for phase 2.

@@ -403,12 +403,13 @@ __global__ __launch_bounds__(256, 2) void seg_gemm_kernel(
 // shape drained the chip at the end of each.  Four rather than nine shapes
 // cover a block of up to 64 x 64, so nothing is rounded up past 32.  Bound
 // by the FP64 matrix cores and what keeps them waiting: at the n=26 M=1000
-// middle site they are busy 63 % of the time a compute unit has work, and
-// its blocks of 1..300 rows leave a quarter of the MFMA work in padding.
-// Product at that site, one right-hand side: 1279 -> 391 us (FP64), three at
+// middle site they are busy 61 (phase 1) and 69 % of the time a compute unit
+// has work, and its blocks of 1..300 rows leave a quarter of the MFMA work in
+// padding.  Product at that site, one right-hand side: 1279 -> 391 us (FP64), three at
 // n=16 M=500: 1930 -> 412 us, FP32, two: 1588 -> 401 us, n=8 M=50: 127 -> 47
-// us (with the split along K of tile_env_refresh); one launch per shape for
-// the same tiles: 444, 498 and 460 us for the first three.  A launch of
+// us (with the split along K of tile_env_refresh; 375, 386, 388 and 48 us as
+// loop and walk are now); one launch per shape for the same tiles: 444, 498
+// and 460 us for the first three.  A launch of
 // 32 x 32 tiles only (launch_tiny) takes their own kernel, which fits more
 // workgroups on a compute unit: FP32 product at n=8 M=50, 128 right-hand
 // sides 691 -> 625 us, one 47.4 -> 46.7 us.

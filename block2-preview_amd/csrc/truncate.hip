@@ -23,7 +23,7 @@
 //     giving an orthogonal Q, and the whole matrix is updated as
 //     A <- J^T A J, V <- V J with J the block-diagonal of the round's Qs:
 //     every 32 x 32 region (pair P rows, pair R columns) becomes
-//     Q_P^T A_PR Q_R.  Matrices are padded to a multiple of 16 with zero rows
+//     Q_P^T A_PR Q_R.  Matrices are padded to a multiple of 32 with zero rows
 //     and columns, which no rotation touches (a zero off-diagonal entry is
 //     never rotated), so positions >= n stay out of the spectrum.  A global
 //     sweep is max(nb) - 1 rounds (smaller matrices cycle through their own
@@ -65,11 +65,13 @@ static_assert((uint64_t)kMaxSyevOrder * kMaxSyevOrder < ((uint64_t)1 << 28) &&
                   kMaxSyevOrder % (2 * kJB) == 0,
               "kMaxSyevOrder");
 constexpr int kJLD = kJS + 1;
-constexpr int kMaxQrBlocks = 72; // orders above 1152: no QR step
+// orders above 1152 have no QR step (its panel in registers); a graded matrix
+// of order 1500 takes 32 sweeps, 74 ms, one of order 1100 with it 9 and 18 ms
+constexpr int kMaxQrBlocks = 72;
 
-// one matrix of a batch: A and V are N x N (N = 32 nb) from a_off; the
-// round's Qs are nb / 2 matrices of 64 x 64 from q_off, their flags from
-// f_off
+// one matrix of a batch: A and V are N x N (N = kJB nb, nb even) from a_off;
+// the round's Qs are nb / 2 matrices of kJS x kJS from q_off, their flags
+// from f_off
 struct JacBlock {
     uint64_t a_off, q_off;
     uint32_t nb, n, f_off;

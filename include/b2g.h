@@ -80,8 +80,9 @@ int b2g_ctx_create(int device, unsigned flags, b2g_ctx *out);
 int b2g_ctx_destroy(b2g_ctx ctx);
 int b2g_ctx_synchronize(b2g_ctx ctx);
 /* gives the device memory that the context keeps of released objects back
- * (at most 16 GiB; it does so by itself when an allocation fails or when
- * less than a quarter of the device is free as memory is released)        */
+ * (at most 16 GiB; it does so by itself when an allocation of any context on
+ * the device fails or when less than a quarter of the device is free as
+ * memory is released)                                                     */
 int b2g_ctx_trim(b2g_ctx ctx);
 /* the context's hipStream_t (for callers that order their own work or
  * record events against it)                                              */
@@ -504,8 +505,10 @@ int b2g_effham_eigs_ex(b2g_effham h, double *x, int k,
  * not modified).  Its eigenvalues go to w (device, compact: matrix i from
  * sum_{j<i} n[j]) in ascending order, its eigenvectors to v + off[i] as
  * rows (row j belongs to eigenvalue j), each signed so that its
- * largest-magnitude component is positive.  FP64 block Jacobi on the
- * device; sweeps (may be NULL) receives the number of Jacobi sweeps.     */
+ * largest-magnitude component is positive.  A matrix with an element that is
+ * not finite has values that are not finite and unit vectors.  FP64 block
+ * Jacobi on the device; sweeps (may be NULL) receives the number of Jacobi
+ * sweeps.                                                                 */
 int b2g_syev_batched(b2g_ctx ctx, int n_mats, const uint32_t *n,
                      const uint64_t *off, const double *a, double *w,
                      double *v, int *sweeps);

@@ -1,6 +1,7 @@
 """Device blocks kept by a context between objects: products, solves and
 truncations on reused (dirty) blocks equal those on fresh ones bit for bit,
-two threads with a context each do not disturb one another, and trim() gives
+two threads with a context each do not disturb one another, blocks of a plan
+that another context runs wait for it, and trim() and a failed allocation give
 the kept memory back."""
 import ctypes as C
 import threading

@@ -1,9 +1,9 @@
 """GPU H*psi on seeded synthetic middle-site problems against the oracle:
 every tile configuration of the grouped GEMM (32x32, 64x64, 128x128 forced
 through B2G_TILE, and the automatic choice), the scratch split into several
-chunks, split-K partial tiles (B2G_KSPLIT), 4 right-hand sides, FP32 and
-split-BF16 three-term (every tile shape).  Blocks range from 1x1 up to 200x200, so
-edge tiles, K remainders and single-element blocks all occur.
+chunks, split-K partial tiles (B2G_KSPLIT), 4 and many right-hand sides, FP32
+and split-BF16 three-term (every tile shape).  Blocks range from 1x1 up to
+200x200, so edge tiles, K remainders and single-element blocks all occur.
 Tolerances: FP64 1e-12 relative (2-norm), FP32 2e-6, split-BF16 1e-4."""
 import os
 

@@ -6,7 +6,8 @@ edges (1 .. 333), indefinite, positive semi-definite of low rank (the shape
 of a density matrix) and with a repeated eigenvalue; eigenvalues against
 numpy.linalg.eigh to 1e-12 * ||A||_2, residual ||A v - w v|| and
 orthonormality to 1e-11 * ||A||_2; eigenvectors of simple eigenvalues equal
-to the oracle's signed ones to 1e-9.
+to the oracle's signed ones to 1e-9.  Orders around the QR step's limits (to
+1153), powers of two in front, elements that are not finite.
 
 Split: on every golden fixture and truncation case (three without noise,
 two with block2's wavefunction / density-matrix noise drawn from its
