@@ -37,10 +37,20 @@ def _products(ctx, pb, nrhs, precision, accumulate, seed):
     L.check(lib.b2g_hpsi_noalloc(ctx.h, plan, x.data_ptr(), y_new.data_ptr(),
                                  nrhs, 0.75, accumulate, prec))
     ctx.synchronize()
+    # launches of either, counted on calls of their own
+    n, tmp = [], y0.clone()
+    torch.cuda.synchronize()
+    h.set_timing(True)
+    for f in (lib.b2g_hpsi, lib.b2g_hpsi_noalloc):
+        L.check(f(ctx.h, plan, x.data_ptr(), tmp.data_ptr(), nrhs, 0.75, 0,
+                  prec))
+        ctx.synchronize()
+        n.append(sum(h.timing()[1]))
+    batches = n[1] / n[0]
     w, t1, t2 = C.c_uint64(), C.c_uint64(), C.c_uint64()
     L.check(lib.b2g_plan_stats(plan, C.byref(t1), C.byref(t2), C.byref(w)))
     h.deallocate()
-    return y_ref.cpu().numpy(), y_new.cpu().numpy(), int(w.value)
+    return y_ref.cpu().numpy(), y_new.cpu().numpy(), int(w.value), batches
 
 
 @pytest.mark.parametrize("nrhs,precision,accumulate",
@@ -53,8 +63,9 @@ def test_noalloc_matches_hpsi_on_two_calls(gpu_ctx, nrhs, precision,
     for n_orb, m, dim, seed in [(12, 200, 80, 5), (8, 60, 30, 6)]:
         pb = synth.middle_site(n_orb=n_orb, m=m, max_dim=dim, seed=seed)
         print("noalloc", n_orb, m, nrhs, precision, accumulate, flush=True)
-        ref, new, w = _products(gpu_ctx, pb, nrhs, precision, accumulate,
-                                seed)
+        ref, new, w, batches = _products(gpu_ctx, pb, nrhs, precision,
+                                         accumulate, seed)
+        assert batches == (2 if nrhs == 7 and m == 200 else 1), batches
         assert w * nrhs * 8 < SCRATCH_BYTES, w
         assert np.isfinite(ref).all()
         assert np.array_equal(ref, new), np.abs(ref - new).max()
