@@ -66,6 +66,12 @@ static int scratch_setup(int device) {
     return B2G_OK;
 }
 
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &s) == hipSuccess &&
+           s != hipStreamCaptureStatusNone;
+}
+
 // ------------------------------------------------------------- block pool
 constexpr size_t kPoolCap = (size_t)16 << 30;
 
@@ -437,7 +443,9 @@ extern "C" int b2g_upload_blocks(b2g_ctx ctx, const void *host, size_t n,
 
 extern "C" void *b2g_buf_device_ptr(b2g_buf buf) {
     // its block may have work of its last user under way on the stream
-    if (buf && !buf->shown.exchange(true))
+    // (waiting would end a capture; what was queued before it is not waited
+    // for, as ever)
+    if (buf && !buf->shown.exchange(true) && !capturing(buf->ctx->stream))
         (void)hipStreamSynchronize(buf->ctx->stream);
     return buf ? buf->ptr : nullptr;
 }
@@ -1644,8 +1652,9 @@ hipError_t plan_launched_by(b2g_plan p, b2g_ctx ctx) {
     for (b2g_buf b : {p->lbuf, p->rbuf})
         if (b->ctx != ctx)
             b->shown = true;
-    return p->ctx != ctx && !p->elsewhere.exchange(true) ? plan_publish(p)
-                                                         : hipSuccess;
+    if (p->ctx == ctx || p->elsewhere.exchange(true))
+        return hipSuccess;
+    return capturing(ctx->stream) ? hipSuccess : plan_publish(p);
 }
 
 // scratch (W, split-K partials) for n_rhs right-hand sides at `precision`;
@@ -1771,11 +1780,7 @@ static int hpsi_run(b2g_ctx ctx, b2g_plan p, const std::vector<Chunk> &chunks,
         // 0.27 GB of device memory after its destruction (measured on the
         // n=26 M=1000 synthetic site, every effective Hamiltonian of a sweep
         // instantiating one).
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess)
-            cap = hipStreamCaptureStatusNone;
-        const int naux = (p->timing || n_rhs > 1 ||
-                          cap != hipStreamCaptureStatusNone)
+        const int naux = (p->timing || n_rhs > 1 || capturing(ctx->stream))
                              ? 0
                              : std::min<int>((int)ctx->aux.size(), n - 1);
         hipError_t e = hipSuccess;

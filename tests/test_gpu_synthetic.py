@@ -5,6 +5,7 @@ chunks, split-K partial tiles (B2G_KSPLIT), 4 and many right-hand sides, FP32
 and split-BF16 three-term (every tile shape).  Blocks range from 1x1 up to
 200x200, so edge tiles, K remainders and single-element blocks all occur.
 Tolerances: FP64 1e-12 relative (2-norm), FP32 2e-6, split-BF16 1e-4."""
+import ctypes as C
 import os
 
 import numpy as np
@@ -222,4 +223,48 @@ def test_lists_for_many_right_hand_sides(gpu_ctx, problem, precision):
         if n < 64:
             own = y[:3] if own is None else own
             assert np.array_equal(y[:3], own), n
+    h.deallocate()
+
+
+def test_many_right_hand_sides_in_chunks(gpu_ctx, problem):
+    # the W scratch split into chunks that accumulate: lists for many of each
+    pb, xs, ys = problem
+    y = run(gpu_ctx, pb, np.tile(xs, (24, 1)), {"B2G_W_CAP": "200000"})
+    for r in range(96):
+        assert rel(y[r], ys[r % 4]) < 1e-12, r
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32", "bf16x3"])
+@pytest.mark.parametrize("n", [1, 4, 70])
+def test_captured_product(gpu_ctx, problem, precision, n):
+    # a product on reserved scratch captured into a graph on the context's
+    # stream (its output's address first asked for in the capture): every
+    # replay as the eager product on the same vectors
+    pb, xs, _ = problem
+    lib, prec = gpu_ctx.lib, L.PREC[precision]
+    h = EffectiveHamiltonian(pb, gpu_ctx, fp32=precision == "f32")
+    L.check(lib.b2g_plan_reserve(h.plan, n, prec))
+    buf = C.c_void_p()
+    L.check(lib.b2g_buf_create(gpu_ctx.h, n * pb.bra_len, L.B2G_F64,
+                               C.byref(buf)))
+    x = torch.empty((n, pb.ket_len), dtype=torch.float64, device="cuda:0")
+    st = torch.cuda.ExternalStream(lib.b2g_ctx_stream(gpu_ctx.h))
+    graph = torch.cuda.CUDAGraph()
+    print(precision, n, flush=True)
+    with torch.cuda.graph(graph, stream=st):
+        y = lib.b2g_buf_device_ptr(buf)
+        L.check(lib.b2g_hpsi(gpu_ctx.h, h.plan, x.data_ptr(), y, n, 1.0, 0,
+                             prec))
+    got = np.empty((n, pb.bra_len))
+    for k in range(3):
+        x.copy_(torch.tensor(np.resize(xs[k:], (n, pb.ket_len))))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            graph.replay()
+        L.check(lib.b2g_buf_read(buf, got.ctypes.data, 0, got.size))
+        # (one right-hand side: eager launches overlap, with the same sums)
+        want = h.multiply(x, precision=precision).cpu().numpy()
+        assert np.array_equal(got, want), k
+    del graph
+    lib.b2g_buf_destroy(buf)
     h.deallocate()
