@@ -77,10 +77,7 @@ struct JacBlock {
     uint32_t nb, n, f_off;
     uint32_t qr;      // takes part in the QR step (jacobi_floor_kernel)
     double floor_abs; // off-diagonal entries below this are not rotated
-    // largest |a_ij| of the matrix, as bits (of NaN: above those of Inf)
-    unsigned long long amax;
 };
-static_assert(sizeof(unsigned long long) == sizeof(double), "bits of amax");
 // pair task (kind 0): x = pair index; region task (kind 1): x = row pair,
 // y = column pair; V task (kind 2): x = pair, y = slice of kJS rows
 struct JacTask {
@@ -108,16 +105,27 @@ __device__ __forceinline__ int pair_index(int bi, int bj, int l) {
     return l < kJB ? bi * kJB + l : bj * kJB + (l - kJB);
 }
 
-// A: padded copy of the compact symmetric matrices, V = I, amax (0 before)
+// largest of a value over the lanes of a wave
+__device__ __forceinline__ uint64_t wave_max(uint64_t v) {
+    for (int w = 32; w > 0; w >>= 1)
+        v = max(v, (uint64_t)__shfl_xor((unsigned long long)v, w));
+    return v;
+}
+
+// A: padded copy of the compact symmetric matrices, V = I; amax: the largest
+// |a_ij| that each workgroup met, gridDim.x of them per matrix, as bits (those
+// of NaN lie above those of Inf)
 __global__ __launch_bounds__(256) void jacobi_init_kernel(
-    JacBlock *__restrict__ blocks, int nblocks,
+    const JacBlock *__restrict__ blocks, int nblocks,
     const uint64_t *__restrict__ src_off, const double *__restrict__ src,
-    double *__restrict__ A, double *__restrict__ V) {
+    double *__restrict__ A, double *__restrict__ V,
+    uint64_t *__restrict__ amax) {
+    __shared__ uint64_t wtop[4];
     for (int b = blockIdx.y; b < nblocks; b += gridDim.y) {
         const JacBlock bl = blocks[b];
         const uint32_t N = bl.nb * kJB;
         const uint64_t NN = (uint64_t)N * N;
-        unsigned long long top = 0;
+        uint64_t top = 0;
         for (uint64_t e = blockIdx.x * 256ull + threadIdx.x; e < NN;
              e += (uint64_t)gridDim.x * 256) {
             const uint32_t i = (uint32_t)(e / N), j = (uint32_t)(e % N);
@@ -126,12 +134,16 @@ __global__ __launch_bounds__(256) void jacobi_init_kernel(
                                        : 0.0;
             A[bl.a_off + e] = a;
             V[bl.a_off + e] = i == j ? 1.0 : 0.0;
-            top = max(top, __builtin_bit_cast(unsigned long long, fabs(a)));
+            top = max(top, __builtin_bit_cast(uint64_t, fabs(a)));
         }
-        for (int w = 32; w > 0; w >>= 1)
-            top = max(top, __shfl_xor(top, w));
-        if ((threadIdx.x & 63) == 0 && top != 0)
-            atomicMax(&blocks[b].amax, top);
+        top = wave_max(top);
+        if ((threadIdx.x & 63) == 0)
+            wtop[threadIdx.x >> 6] = top;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            amax[(uint64_t)b * gridDim.x + blockIdx.x] =
+                max(max(wtop[0], wtop[1]), max(wtop[2], wtop[3]));
+        __syncthreads(); // before the next matrix's wtop
     }
 }
 
@@ -140,17 +152,21 @@ __global__ __launch_bounds__(256) void jacobi_init_kernel(
 // take of its elements neither overflow nor vanish (unscaled, norms below
 // 1e-153 counted as zero and above 6e153 as infinite); the eigenvectors are
 // those of A and the eigenvalues are taken from A itself (rayleigh_kernel).
+// The largest element comes from the nmax <= 64 parts of jacobi_init_kernel.
 // Then floor_abs: 64 eps ||A_b||_F.  Stage 1: workgroup (chunk, b) scales and
 // sums the squares of rows chunk, chunk + gridDim.x, ... of matrix b into
 // part[b * gridDim.x + chunk]; stage 2 (jacobi_floor_kernel) adds the parts
 // of each matrix in order (deterministic).
 __global__ __launch_bounds__(256) void jacobi_norm_kernel(
-    const JacBlock *__restrict__ blocks, double *__restrict__ A,
-    double *__restrict__ part) {
+    const JacBlock *__restrict__ blocks, const uint64_t *__restrict__ parts,
+    int nmax, double *__restrict__ A, double *__restrict__ part) {
     __shared__ double sh[256];
     const JacBlock bl = blocks[blockIdx.y];
     const uint32_t N = bl.nb * kJB;
-    const double amax = __builtin_bit_cast(double, bl.amax);
+    const int lane = threadIdx.x & 63;
+    const double amax = __builtin_bit_cast(
+        double,
+        wave_max(lane < nmax ? parts[(uint64_t)blockIdx.y * nmax + lane] : 0));
     const int sc = amax > 0.0 && isfinite(amax) ? -ilogb(amax) : 0;
     double s = 0.0;
     for (uint32_t i = blockIdx.x; i < N; i += gridDim.x)
@@ -1126,7 +1142,6 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
         b.f_off = (uint32_t)s.f_len;
         b.qr = 0;
         b.floor_abs = 0.0;
-        b.amax = 0;
         s.a_len += N * N;
         s.q_len += (uint64_t)(b.nb / 2) * kJS * kJS;
         s.f_len += b.nb / 2;
@@ -1183,15 +1198,17 @@ static int syev_run(b2g_ctx ctx, const std::vector<uint32_t> &n,
         const uint64_t nn = (uint64_t)s.max_nb * kJB * s.max_nb * kJB;
         const unsigned gx = (unsigned)std::min<uint64_t>((nn + 255) / 256, 64);
         const unsigned gy = (unsigned)std::min<size_t>(nm, 4096);
-        hipLaunchKernelGGL(jacobi_init_kernel, dim3(gx, gy), dim3(256), 0, st,
-                           s.d_blk, (int)nm, s.d_src_off, src, s.A, s.V);
-        B2G_HIP(hipGetLastError());
         const unsigned nparts = 32;
-        double *part = nullptr;
-        B2G_HIP(ctx->alloc(&part, nm * nparts * sizeof(double)));
+        double *part = nullptr; // then the init kernel's parts
+        B2G_HIP(ctx->alloc(&part, nm * (nparts + gx) * sizeof(double)));
         PoolGuard part_guard(ctx, part);
+        uint64_t *amax = (uint64_t *)(part + nm * nparts);
+        hipLaunchKernelGGL(jacobi_init_kernel, dim3(gx, gy), dim3(256), 0, st,
+                           s.d_blk, (int)nm, s.d_src_off, src, s.A, s.V, amax);
+        B2G_HIP(hipGetLastError());
         hipLaunchKernelGGL(jacobi_norm_kernel, dim3(nparts, (unsigned)nm),
-                           dim3(256), 0, st, s.d_blk, s.A, part);
+                           dim3(256), 0, st, s.d_blk, amax, (int)gx, s.A,
+                           part);
         B2G_HIP(hipGetLastError());
         hipLaunchKernelGGL(jacobi_floor_kernel,
                            dim3((unsigned)((nm + 255) / 256)), dim3(256), 0,
@@ -1761,13 +1778,14 @@ static int split_impl(b2g_ctx ctx, int symmetry, const b2g_sparse_info *wfn,
     if (k != -1) {
         // NaN as +Inf (comparing it, std::sort may leave its range): states of
         // a block that is not finite are kept, so that they show in the result
-        auto rank = [&](const std::pair<int, int> &x) {
-            const double v = wrv(x);
-            return std::isnan(v) ? std::numeric_limits<double>::infinity() : v;
-        };
+        std::vector<double> key(wr);
+        for (double &v : key)
+            if (std::isnan(v))
+                v = std::numeric_limits<double>::infinity();
         std::sort(ss.begin(), ss.end(),
                   [&](const std::pair<int, int> &a, const std::pair<int, int> &b) {
-                      return rank(a) > rank(b);
+                      return key[woff[a.first] + a.second] >
+                             key[woff[b.first] + b.second];
                   });
         const unsigned keep = trunc_type / 16u;
         if (keep == 0) {
