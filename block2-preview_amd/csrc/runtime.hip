@@ -1141,10 +1141,10 @@ static int many_from(const b2g_plan_s *p) {
     const int none = 1 << 30;
     if (p->plain || p->macs == 0)
         return none;
-    const uint64_t n =
-        std::min<uint64_t>(64, std::max<uint64_t>(16, 150000000000ull / p->macs));
-    return (int)std::max<uint64_t>(
-        n, kNoAllocScratchBytes / (4 * std::max<uint64_t>(p->w_max, 1)) + 1);
+    const uint64_t by_size = 150000000000ull / p->macs;
+    const uint64_t n = std::min<uint64_t>(64, std::max<uint64_t>(16, by_size));
+    const uint64_t w_bytes = 4 * std::max<uint64_t>(p->w_max, 1); // FP32
+    return (int)std::max(n, kNoAllocScratchBytes / w_bytes + 1);
 }
 
 static int build_many(b2g_plan p) {
